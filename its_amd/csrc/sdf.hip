@@ -201,6 +201,18 @@ __device__ inline float4 tri_sphere(const double* T) {
     return make_float4((float)c[0], (float)c[1], (float)c[2], (float)(r * (1.0 + 1e-6) + 1e-6 * (cm + r)));
 }
 
+// unit normal of a triangle, binary64 rounded once; zero for a degenerate one
+__device__ inline float4 tri_unit_normal(const double* T) {
+    const double u[3] = {T[3] - T[0], T[4] - T[1], T[5] - T[2]}, v[3] = {T[6] - T[0], T[7] - T[1], T[8] - T[2]};
+    const double x = u[1] * v[2] - u[2] * v[1], y = u[2] * v[0] - u[0] * v[2], z = u[0] * v[1] - u[1] * v[0];
+    const double l2 = x * x + y * y + z * z;
+    // a sliver's normal is mostly rounding: no bound is taken from it
+    const double m = fmax(u[0] * u[0] + u[1] * u[1] + u[2] * u[2], v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+    if (!(l2 > 1e-12 * m * m)) return make_float4(0.f, 0.f, 0.f, 0.f);
+    const double l = sqrt(l2);
+    return make_float4((float)(x / l), (float)(y / l), (float)(z / l), 0.f);
+}
+
 // ---------------------------------------------------------------- tree ----
 struct Shape {
     int32_t T;                  // triangles
@@ -246,6 +258,7 @@ struct TreeView {
     Quant q;
     const double* tris;      // 9 per sorted triangle
     const float4* sph;       // bounding sphere per sorted triangle
+    const float4* nrm;       // unit normal per sorted triangle (zero: none)
     const int32_t* tid;      // original index per sorted triangle
     const uint32_t* code;    // centroid Morton code per sorted triangle (ascending)
     const float4* node;      // 2 per node: box lo.xyz + first fan edge (int bits in w),
@@ -296,7 +309,7 @@ __global__ void k_tri_keys(const double* V, const int32_t* F, int64_t nF, Quant 
 }
 
 __global__ void k_tri_gather(const uint32_t* idx, int64_t nF, const double* V, const int32_t* F, double* tris,
-                             float4* sph, int32_t* tid, int32_t* pos) {
+                             float4* sph, float4* nrm, int32_t* tid, int32_t* pos) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nF) return;
     const int64_t t = (int64_t)idx[i];
@@ -305,6 +318,7 @@ __global__ void k_tri_gather(const uint32_t* idx, int64_t nF, const double* V, c
         for (int a = 0; a < 3; ++a) T[3 * c + a] = V[3 * (int64_t)F[3 * t + c] + a];
     for (int j = 0; j < 9; ++j) tris[9 * i + j] = T[j];
     sph[i] = tri_sphere(T);
+    nrm[i] = tri_unit_normal(T);
     tid[i] = (int32_t)t;
     pos[t] = (int32_t)i;
 }
@@ -519,30 +533,30 @@ int bits_for(uint64_t maxval) {
 // ---------------------------------------------------------- radix sort ----
 // Stable LSD radix sort on the low `bits` bits of the keys, 8-bit digits,
 // three launches per digit:
-//   - k_rs_hist: the digit histogram of each tile of 2048 keys (LDS
+//   - k_rs_hist: the digit histogram of each tile of ROUNDS * 256 keys (LDS
 //     atomics), stored digit-major, hist[d * tiles + tile];
 //   - k_rs_offsets: one workgroup per digit scans that digit's row of tile
 //     counts (exclusive) and stores the row total;
 //   - k_rs_scatter: each tile starts every digit at the sum of the smaller
-//     digits' totals plus its row offset, then, in 8 rounds of 256 keys in
-//     input order, ranks every key among the keys of its digit before it (a
+//     digits' totals plus its row offset, then, in ROUNDS rounds of 256 keys
+//     in input order, ranks every key among the keys of its digit before it (a
 //     mask of the wavefront's lanes with the same digit from 8 ballots, and
 //     per-wave counts in LDS) and writes key and value there.
 // Keys with equal digits keep their input order within a tile, and tiles
 // follow one another in the offsets, so every pass is stable and equal keys
 // end in their input order, which the triangle order and the fan edge order
 // rely on.
-constexpr int kRsThreads = 256, kRsRounds = 8, kRsTile = kRsThreads * kRsRounds, kRsBins = 256;
+constexpr int kRsThreads = 256, kRsBins = 256;
 static_assert(kRsThreads == kRsBins, "one histogram bin per thread");
 
-template <class K>
+template <int ROUNDS, class K>
 __global__ __launch_bounds__(kRsThreads) void k_rs_hist(const K* keys, int64_t n, int shift, uint32_t* hist,
                                                        int64_t tiles) {
     __shared__ uint32_t h[kRsBins];
     h[threadIdx.x] = 0u;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * kRsTile;
-    for (int j = 0; j < kRsRounds; ++j) {
+    const int64_t base = (int64_t)blockIdx.x * (ROUNDS * kRsThreads);
+    for (int j = 0; j < ROUNDS; ++j) {
         const int64_t i = base + (int64_t)j * kRsThreads + threadIdx.x;
         if (i < n) atomicAdd(&h[(uint32_t)(keys[i] >> shift) & (kRsBins - 1)], 1u);
     }
@@ -581,7 +595,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_offsets(uint32_t* hist, int64
     if (threadIdx.x == 0) tot[blockIdx.x] = carry;
 }
 
-template <class K, class V>
+template <int ROUNDS, class K, class V>
 __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const K* kin, const V* vin, K* kout, V* vout, int64_t n,
                                                           int shift, const uint32_t* off, int64_t tiles,
                                                           const uint32_t* tot) {
@@ -594,8 +608,8 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const K* kin, const V
     // digit d starts after every smaller digit's keys and this digit's keys of earlier tiles
     const uint32_t digit_base = block_excl_scan256(tot[threadIdx.x], sh);
     next[threadIdx.x] = digit_base + off[(int64_t)threadIdx.x * tiles + blockIdx.x];
-    const int64_t base = (int64_t)blockIdx.x * kRsTile;
-    for (int j = 0; j < kRsRounds; ++j) {
+    const int64_t base = (int64_t)blockIdx.x * (ROUNDS * kRsThreads);
+    for (int j = 0; j < ROUNDS; ++j) {
         const int64_t i = base + (int64_t)j * kRsThreads + threadIdx.x;
         const bool valid = i < n;
         const K k = valid ? kin[i] : K(0);
@@ -630,27 +644,35 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const K* kin, const V
 }
 
 // sorts keys (and vals, when given) in place; n below 2^32
-template <class K, class V>
-void radix_sort(DBuf<K>& keys, DBuf<V>* vals, int64_t n, int bits, hipStream_t st) {
-    if (n <= 1 || bits <= 0) return;
-    ITS_REQUIRE(n < (int64_t(1) << 32), ITS_E_RANGE, "radix sort of 2^32 keys or more");
-    const int64_t tiles = (n + kRsTile - 1) / kRsTile;
+template <int ROUNDS, class K, class V>
+void radix_sort_tiles(DBuf<K>& keys, DBuf<V>* vals, int64_t n, int bits, hipStream_t st) {
+    const int64_t tiles = (n + ROUNDS * kRsThreads - 1) / (ROUNDS * kRsThreads);
     DBuf<K> k2(n);
     DBuf<V> v2(vals ? n : 0);
     DBuf<uint32_t> hist(kRsBins * tiles), tot(kRsBins);
     for (int shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(k_rs_hist<K>, dim3((unsigned)tiles), dim3(kRsThreads), 0, st, (const K*)keys.p, n, shift,
-                           hist.p, tiles);
+        hipLaunchKernelGGL((k_rs_hist<ROUNDS, K>), dim3((unsigned)tiles), dim3(kRsThreads), 0, st, (const K*)keys.p, n,
+                           shift, hist.p, tiles);
         ITS_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_rs_offsets, dim3(kRsBins), dim3(kRsThreads), 0, st, hist.p, tiles, tot.p);
         ITS_LAUNCH_CHECK();
-        hipLaunchKernelGGL((k_rs_scatter<K, V>), dim3((unsigned)tiles), dim3(kRsThreads), 0, st, (const K*)keys.p,
-                           vals ? (const V*)vals->p : (const V*)nullptr, k2.p, vals ? v2.p : (V*)nullptr, n, shift,
-                           (const uint32_t*)hist.p, tiles, (const uint32_t*)tot.p);
+        hipLaunchKernelGGL((k_rs_scatter<ROUNDS, K, V>), dim3((unsigned)tiles), dim3(kRsThreads), 0, st,
+                           (const K*)keys.p, vals ? (const V*)vals->p : (const V*)nullptr, k2.p,
+                           vals ? v2.p : (V*)nullptr, n, shift, (const uint32_t*)hist.p, tiles, (const uint32_t*)tot.p);
         ITS_LAUNCH_CHECK();
         std::swap(keys, k2);
         if (vals) std::swap(*vals, v2);
     }
+}
+// Tiles of 2048 keys, or of 512 below kRsSmall keys: a tile's rounds follow
+// one another, and 2048-key tiles would leave most CUs without one.
+constexpr int64_t kRsSmall = int64_t(1) << 20;
+template <class K, class V>
+void radix_sort(DBuf<K>& keys, DBuf<V>* vals, int64_t n, int bits, hipStream_t st) {
+    if (n <= 1 || bits <= 0) return;
+    ITS_REQUIRE(n < (int64_t(1) << 32), ITS_E_RANGE, "radix sort of 2^32 keys or more");
+    if (n < kRsSmall) radix_sort_tiles<2>(keys, vals, n, bits, st);
+    else radix_sort_tiles<8>(keys, vals, n, bits, st);
 }
 
 struct TriTree {
@@ -659,7 +681,7 @@ struct TriTree {
     int64_t nodes = 0, fans = 0;
     DBuf<double> tris;
     DBuf<float> fan;
-    DBuf<float4> sph, node;
+    DBuf<float4> sph, nrm, node;
     DBuf<int32_t> tid;
     DBuf<uint32_t> code, cell_lb;
     int cell_bits = 0;
@@ -672,7 +694,7 @@ struct TriTree {
     uint64_t none = 0;
     int vb = 0;
     TreeView view() const {
-        return TreeView{s, q, tris.p, sph.p, tid.p, code.p, node.p, fan.p, cell_lb.p, cell_bits};
+        return TreeView{s, q, tris.p, sph.p, nrm.p, tid.p, code.p, node.p, fan.p, cell_lb.p, cell_bits};
     }
 };
 
@@ -728,10 +750,11 @@ void tree_build(TriTree& tr, hipStream_t st, const double* d_V, int64_t nV, cons
     radix_sort(tr.code, &tidx, nF, 30, st);
     tr.tris.alloc(9 * (size_t)nF);
     tr.sph.alloc(nF);
+    tr.nrm.alloc(nF);
     tr.tid.alloc(nF);
     DBuf<int32_t> pos(nF);
     hipLaunchKernelGGL(k_tri_gather, dim3(blocks_for(nF, kT)), dim3(kT), 0, st, (const uint32_t*)tidx.p, nF, d_V, d_F,
-                       tr.tris.p, tr.sph.p, tr.tid.p, pos.p);
+                       tr.tris.p, tr.sph.p, tr.nrm.p, tr.tid.p, pos.p);
     ITS_LAUNCH_CHECK();
     // code-prefix table with about one prefix per triangle (3 to 21 bits)
     tr.cell_bits = 3;
@@ -830,7 +853,7 @@ void fans_build(TriTree& tr, hipStream_t st, const double* d_V) {
 }
 
 // -------------------------------------------------------------- query -----
-// Both walks run one wavefront per point: the walk is the same for all
+// The node-by-node and winding walks run one wavefront per point: the walk is the same for all
 // lanes, and nodes of level kLeafLevel and below (at most 64 triangles) are
 // leaves whose triangles the 64 lanes take one each.  Per-lane results are
 // combined by a fixed butterfly, so nothing depends on timing.
@@ -858,9 +881,8 @@ __device__ inline void wave_argmin(double& d2, int32_t& id) {
     }
 }
 
-// Values that are equal in every lane (the point of the wavefront, the best
-// distance after the butterfly) are moved to scalar registers, which the
-// compiler cannot infer from threadIdx.x >> 6 or from shuffles.
+// Values that are equal in every lane are moved to scalar registers, which
+// the compiler cannot infer from threadIdx.x >> 6 or from shuffles.
 __device__ inline int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ inline double wave_uniform(double v) {
     const uint64_t u = (uint64_t)__double_as_longlong(v);
@@ -869,14 +891,23 @@ __device__ inline double wave_uniform(double v) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
-// false when the bounding sphere of sorted triangle i is farther than the
-// best distance so far
+__device__ inline float wave_uniform_f(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+// false when the bounding sphere of sorted triangle i, or its plane, is
+// farther than the best distance so far.  Far from the surface the sphere's
+// radius is most of what separates the candidates; the plane's distance is
+// within the triangle's tilt of the true one.
 __device__ inline bool sphere_within(const TreeView& t, int64_t i, const double p[3], float pm, double best) {
     const float4 S = t.sph[i];
     const float dx = (float)p[0] - S.x, dy = (float)p[1] - S.y, dz = (float)p[2] - S.z;
     const float m = bound_margin(pm + fmaxf(fabsf(S.x), fmaxf(fabsf(S.y), fabsf(S.z))) + S.w);
     const float lb = sqrtf(dx * dx + dy * dy + dz * dz) - S.w - m;
-    return !(lb > 0.f && (double)lb * (double)lb > best);
+    if (lb > 0.f && (double)lb * (double)lb > best) return false;
+    const float4 n = t.nrm[i];
+    const float pb = fabsf(n.x * dx + n.y * dy + n.z * dz) - m;
+    return !(pb > 0.f && (double)pb * (double)pb > best);
 }
 // binary64 distance of sorted triangle i (when take), merged over the
 // wavefront into (best, bt)
@@ -947,36 +978,20 @@ __device__ inline int start_level(const Shape& s, int leaf, int most) {
     while (h > leaf && s.count[h - 1] <= most) --h;
     return h;
 }
-// the distance walk starts at up to 512 nodes (eight per lane); at most
-// kFront of them survive
-constexpr int kDistStartNodes = 512;
 
 __device__ inline bool box_outside(const double p[3], float4 lo, float4 hi) {
     return p[0] < (double)lo.x || p[0] > (double)hi.x || p[1] < (double)lo.y || p[1] > (double)hi.y ||
            p[2] < (double)lo.z || p[2] > (double)hi.z;
 }
 
-// Nearest triangle: binary64 distance (unsigned, into out) and the original
-// index of the nearest triangle.  The walk starts with the leaf at the
-// point's Morton position, which usually holds the nearest triangle.
-// Distance walk, level by level: the wavefront keeps the nodes of one level
-// that can still hold the nearest triangle (the frontier, in LDS) and tests
-// all their children at once, one child pair per lane, against the distance
-// from the seed leaf.  The surviving leaves are then searched one by one,
-// skipped when their box is beyond the best distance found so far.  A leaf
-// that can hold the nearest triangle has every ancestor box within the final
-// distance, which is no larger than the seed's, so it is never dropped: the
-// result is the exact (d², index) minimum.  A frontier that would overflow
-// LDS sends the point to the node-by-node walk.
-constexpr int kFront = 512;
-// candidate queue: below 64 entries between rounds, plus two leaves of 64
-constexpr int kCandQueue = 192;
-__device__ void dist_dfs(const TreeView& t, int leaf, int64_t seed, int lane, const double p[3], const float pf[3],
-                         float pm, double& best, int32_t& bt) {
+// The node-by-node walk: depth first, skipping a node whose box is farther
+// than the best distance so far.  For points whose frontier overflows.
+__device__ void dist_dfs(const TreeView& t, int leaf, int lane, const double p[3], const float pf[3], float pm,
+                         double& best, int32_t& bt) {
     int h = t.s.H, k = 0;
     while (true) {
         const NodeRec r = load_node(t, t.s.off[h] + k);
-        if (!(h == leaf && k == seed) && !box_beyond(pf, pm, r.lo, r.hi, best)) {
+        if (!box_beyond(pf, pm, r.lo, r.hi, best)) {
             if (h > leaf) {
                 --h;
                 k <<= 1;
@@ -988,154 +1003,461 @@ __device__ void dist_dfs(const TreeView& t, int leaf, int64_t seed, int lane, co
     }
 }
 
-__global__ __launch_bounds__(kT) void k_sdf_dist(TreeView t, const double* pts, int64_t N, double* out,
-                                                 int32_t* tri_out) {
-    __shared__ uint32_t fk[2][kWavesPerBlock][kFront];   // frontier node indices within their level
-    __shared__ float flb[kWavesPerBlock][kFront];        // box lower bounds of the leaf-level frontier
-    __shared__ uint32_t cq[kWavesPerBlock][kCandQueue];  // candidate triangles (sorted positions)
-    const int lane = threadIdx.x & 63, w = wave_uniform((int)(threadIdx.x >> 6));
+// ------------------------------------------------------------- packets ----
+// Many points near one another (the octree's vertices above all) need almost
+// the same nodes and triangles, which a wavefront per point would read and test
+// once per point.  The packet kernels give a wavefront kPk neighbouring points
+// and walk the tree once for all of them:
+//   - k_pt_seed gives every point the exact distance to one triangle near its
+//     Morton position and a sort key: the size of that distance (powers of
+//     two of the mesh box), then the Morton prefix.  Points of like distance
+//     and place end up side by side, so one far point does not widen the
+//     search of the near ones.
+//   - A packet keeps the frontier of one tree level in LDS, nodes that the
+//     box of its points can need, one node per lane and round, down to the
+//     buckets of 8 triangles.
+//   - Every (point, bucket) pair is tested, kPk points by 64 / kPk buckets a
+//     round; the pairs that pass go to an LDS queue.
+//   - 64 queued pairs at a time test their bucket's 8 bounding spheres, in
+//     binary32 with the margins of sphere_within; the (point, triangle) pairs
+//     that pass go to a second queue and take the exact binary64 test 64 at a
+//     time, whatever their points.
+// Every triangle that the exact minimum (or crossing count) needs passes
+// these tests, and the exact tests are those of the node-by-node walks, so the
+// results are theirs bit for bit.  Bound by vector instructions (about 3,800
+// per packet of 16 points, 65 % of the issue slots; a wavefront per point took
+// over 1,200 per point): 200,000 triangles and 554,122 octree vertices,
+// distances 2,736 -> 370 us and 350 us for the 2 % of points on the second
+// pass, crossings 1,692 -> 270 us, seeds 58 us and their sort 75 us.
+//
+// P points per packet: 16 on the first pass, over all points.  Packets whose
+// frontier would overflow put their points on a list, which the second pass
+// walks one point at a time (P = 1, 64 buckets a round).  There a frontier
+// that would overflow stays at its level, and all buckets below its nodes are
+// tested.
+constexpr int kPk = 16;
+constexpr int kFrontPacket = 384, kFrontPoint = 512;   // nodes per frontier of the two passes
+constexpr int kPairQueue = 128;  // (point, bucket): below 64 before a round, up to 64 a round
+constexpr int kTriQueue = 576;   // (point, triangle): below 64 before a round, up to 512 a round
+constexpr int kSeedWindow = 16;  // sorted triangles looked at around the Morton position
+
+// The points of a pass: n, in the given order, or those of a list whose length
+// is in device memory; both null: points 0 .. n - 1.
+struct Work {
+    int64_t n;
+    const uint32_t* list;
+    const unsigned* list_n;
+    __device__ int64_t size() const { return list_n ? (int64_t)*list_n : n; }
+    __device__ int64_t point(int64_t at) const { return list ? (int64_t)list[at] : at; }
+};
+
+// Margin for binary32 tests of a point (largest coordinate pm) against any
+// box or sphere of the tree
+__device__ inline float root_scale(const NodeRec& root) {
+    float sc = 0.f;
+    const float l[3] = {root.lo.x, root.lo.y, root.lo.z}, u[3] = {root.hi.x, root.hi.y, root.hi.z};
+    for (int a = 0; a < 3; ++a) sc = fmaxf(sc, fmaxf(fabsf(l[a]), fabsf(u[a])));
+    return sc;
+}
+
+__device__ inline float wave_min_f(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+    return wave_uniform_f(v);
+}
+__device__ inline float wave_max_f(float v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    return wave_uniform_f(v);
+}
+
+constexpr int kSeedKeyBits = 24;
+// d2_out, at_out: exact squared distance and sorted position of the triangle near p
+__global__ void k_pt_seed(TreeView t, const double* pts, int64_t N, uint32_t* key, uint32_t* idx, double* d2_out,
+                          int32_t* at_out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N) return;
+    const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
+    const uint32_t c = quant_code(t.q, p);
+    const uint32_t C = c >> (30 - t.cell_bits);
+    int64_t a = t.cell_lb[C], b = t.cell_lb[C + 1];
+    while (a < b) {
+        const int64_t m = (a + b) >> 1;
+        if (t.code[m] < c) a = m + 1; else b = m;
+    }
+    const int64_t lo = max((int64_t)0, min(a, (int64_t)t.s.T) - kSeedWindow / 2);
+    const int64_t hi = min((int64_t)t.s.T, lo + kSeedWindow);
+    const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
+    float near2 = INFINITY;
+    int64_t j = min(a, (int64_t)t.s.T - 1);
+    for (int64_t k = lo; k < hi; ++k) {
+        const float4 S = t.sph[k];
+        const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z;
+        const float d2 = dx * dx + dy * dy + dz * dz;
+        if (d2 < near2) {
+            near2 = d2;
+            j = k;
+        }
+    }
+    const NodeRec root = load_node(t, t.s.off[t.s.H]);
+    const float ext = fmaxf(root.hi.x - root.lo.x, fmaxf(root.hi.y - root.lo.y, root.hi.z - root.lo.z));
+    // Away from the surface the Morton position says little (a tenth of the
+    // seeds are over twice as far as the nearest triangle), and the reach of
+    // a packet grows with it: such a point also descends the tree, to the
+    // child whose box is nearer by its nearest and farthest corner together,
+    // and looks at that bucket.
+    if (near2 > ext * ext * (1.f / (128.f * 128.f))) {
+        int k = 0;
+        for (int h = t.s.H; h > 0; --h) {
+            float m[2] = {INFINITY, INFINITY};
+            for (int c = 0; c < 2; ++c) {
+                if (2 * k + c >= t.s.count[h - 1]) break;
+                const NodeRec r = load_node(t, t.s.off[h - 1] + 2 * k + c);
+                const float l[3] = {r.lo.x, r.lo.y, r.lo.z}, u[3] = {r.hi.x, r.hi.y, r.hi.z};
+                m[c] = 0.f;
+                for (int x = 0; x < 3; ++x) {
+                    const float e = fmaxf(fmaxf(l[x] - pf[x], pf[x] - u[x]), 0.f);
+                    const float f = fmaxf(fabsf(pf[x] - l[x]), fabsf(pf[x] - u[x]));
+                    m[c] += e * e + f * f;
+                }
+            }
+            k = 2 * k + (m[1] < m[0] ? 1 : 0);
+        }
+        for (int q = k * kBucket; q < min((k + 1) * kBucket, t.s.T); ++q) {
+            const float4 S = t.sph[q];
+            const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z;
+            const float d2 = dx * dx + dy * dy + dz * dz;
+            if (d2 < near2) {
+                near2 = d2;
+                j = q;
+            }
+        }
+    }
+    const double* T = t.tris + 9 * j;
+    double best = point_tri_dist2(p, T, T + 3, T + 6);
+    if (!(best <= INFINITY)) best = INFINITY;   // a degenerate triangle never wins
+    // distance classes: below 1/128 of the box, then one per power of two
+    const float rel = sqrtf((float)best) * 128.f;
+    uint32_t cls = 0;
+    for (float lim = ext; cls < 7 && !(rel < lim); lim *= 2.f) ++cls;
+    key[i] = (cls << 21) | (c >> 9);   // kSeedKeyBits bits
+    idx[i] = (uint32_t)i;
+    d2_out[i] = best;
+    at_out[i] = (int32_t)j;
+}
+
+// bucket j of the frontier: its nodes are of `level`, each standing for the
+// 2^level buckets below it
+__device__ inline int front_bucket(const uint32_t* list, int level, uint32_t j) {
+    return (int)((list[j >> level] << level) | (j & ((1u << level) - 1u)));
+}
+
+// appends v of the lanes with take to a queue of n entries
+__device__ inline void queue_push(uint32_t* queue, int& n, bool take, uint32_t v, uint64_t below) {
+    const uint64_t m = __ballot(take);
+    if (take) queue[n + __popcll(m & below)] = v;
+    n += __popcll(m);
+}
+
+// The walk starts at the lowest level of at most this many nodes, all loaded
+// at once.  Packets go down to the buckets.  A single point stops at nodes
+// of 64 triangles, whose buckets are then tested 64 a round: three rounds of
+// the frontier that would each wait for a load are left out.
+constexpr int start_nodes(int P) { return P > 1 ? 256 : 512; }
+constexpr int stop_level(int P) { return P > 1 ? 0 : 3; }
+static_assert(start_nodes(1) <= kFrontPoint, "the start level always fits");
+
+// 64 boxes, loaded one per lane and read by the lanes of any point
+struct BoxStage {
+    float4 lo[64], hi[64];
+    __device__ void fill(const TreeView& t, int node, int lane) {
+        const float4 l = t.node[2 * node], h = t.node[2 * node + 1];
+        lds_fence();
+        lo[lane] = l;
+        hi[lane] = h;
+        lds_fence();
+    }
+};
+
+// Frontier of a packet: nodes of one level that some point needs, from the
+// start level down, one node (pair) per lane and round.  keep(lo, hi) is the
+// test with the box of all points; lists longer than kPkRefine are cut down
+// to the nodes that need(lo, hi) holds for with one of the points (P points
+// by 64 / P nodes a round).  Both must hold for a node whenever they hold
+// for one of its children.  Returns the count (list in fk[cur], nodes of
+// `level`).  A list that would overflow ends the walk: -1 with several
+// points, the list of the level above with one.
+constexpr int kPkRefine = 40;
+template <int P, int FRONT, class Keep, class Need>
+__device__ inline int packet_frontier(const TreeView& t, int start, int lane, uint32_t (*fk)[FRONT], BoxStage& box,
+                                      int& cur, int& level, Keep&& keep, Need&& need) {
+    constexpr int SUB = 64 / P, kQ = start_nodes(P) / 64, stop = stop_level(P);
     const uint64_t below = (1ull << lane) - 1ull;
-    const int64_t nw = (int64_t)gridDim.x * kWavesPerBlock;
-    const int leaf = std::min(kLeafLevel, (int)t.s.H);
-    const int start = start_level(t.s, leaf, kDistStartNodes), start_count = t.s.count[start];
-    for (int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + w; i < N; i += nw) {
-        const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
-        const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
-        const float pm = fmaxf(fabsf(pf[0]), fmaxf(fabsf(pf[1]), fabsf(pf[2])));
-        double best = INFINITY;
-        int32_t bt = 0x7fffffff;
-        // the lower bound of c among the sorted codes lies within its prefix's range
-        const uint32_t c = quant_code(t.q, p);
-        const uint32_t C = c >> (30 - t.cell_bits);
-        int64_t a = t.cell_lb[C], b = t.cell_lb[C + 1];
-        while (a < b) {
-            const int64_t m = (a + b) >> 1;
-            if (t.code[m] < c) a = m + 1; else b = m;
-        }
-        const int64_t seed = std::min<int64_t>(a, t.s.T - 1) >> (__builtin_ctz(kBucket) + leaf);
-        leaf_nearest(t, leaf, seed, lane, p, pm, best, bt);
-        // frontier: the nodes of the start level whose boxes are within the
-        // seed's distance
-        int n = 0, cur = 0;
-        {
-            constexpr int kQ = kDistStartNodes / 64;
-            static_assert(kDistStartNodes <= kFront && kDistStartNodes % 64 == 0, "start nodes: kQ per lane");
-            float lb[kQ];
-            bool keep[kQ];
+    const int slot = lane / P;
+    const int count = t.s.count[start];
+    int n = 0;
+    cur = 0;
+    bool kp[kQ];
 #pragma unroll
-            for (int q = 0; q < kQ; ++q) {
-                lb[q] = 0.f;
-                keep[q] = false;
-                if (lane + 64 * q < start_count) {
-                    const NodeRec r = load_node(t, t.s.off[start] + lane + 64 * q);
-                    lb[q] = box_lb(pf, pm, r.lo, r.hi);
-                    keep[q] = !lb_beyond(lb[q], best);
-                }
-            }
-            lds_fence();
-#pragma unroll
-            for (int q = 0; q < kQ; ++q) {
-                const uint64_t m = __ballot(keep[q]);
-                if (keep[q]) {
-                    const int pos = n + __popcll(m & below);
-                    fk[0][w][pos] = (uint32_t)(lane + 64 * q);
-                    flb[w][pos] = lb[q];
-                }
-                n += __popcll(m);
-            }
-            lds_fence();
+    for (int q = 0; q < kQ; ++q) {
+        kp[q] = false;
+        if (lane + 64 * q < count) {
+            const NodeRec r = load_node(t, t.s.off[start] + lane + 64 * q);
+            kp[q] = keep(r.lo, r.hi);
         }
-        bool overflow = false;
-        for (int h = start; h > leaf && n > 0; --h) {
-            const int64_t coff = t.s.off[h - 1];
-            const int ccount = t.s.count[h - 1];
-            const bool to_leaf = (h - 1 == leaf);
-            int m = 0;   // next frontier size (uniform)
+    }
+    lds_fence();   // the lists of the packet before
+    level = start;
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+        if (P > 1 && n + __popcll(__ballot(kp[q])) > FRONT) return -1;
+        queue_push(fk[0], n, kp[q], (uint32_t)(lane + 64 * q), below);
+    }
+    lds_fence();
+    for (int h = start; h > stop && n > 0; --h) {
+        if (P > 1 && n > kPkRefine) {
+            int m = 0;
             for (int j0 = 0; j0 < n; j0 += 64) {
-                const int j = j0 + lane;
-                bool keep0 = false, keep1 = false;
-                uint32_t c0 = 0;
-                float lb0 = 0.f, lb1 = 0.f;
-                if (j < n) {
-                    c0 = 2u * fk[cur][w][j];
-                    const NodeRec r0 = load_node(t, (int)(coff + c0));
-                    lb0 = box_lb(pf, pm, r0.lo, r0.hi);
-                    keep0 = !lb_beyond(lb0, best);
-                    if ((int)c0 + 1 < ccount) {
-                        const NodeRec r1 = load_node(t, (int)(coff + c0 + 1));
-                        lb1 = box_lb(pf, pm, r1.lo, r1.hi);
-                        keep1 = !lb_beyond(lb1, best);
-                    }
+                const uint32_t k = j0 + lane < n ? fk[cur][j0 + lane] : 0u;
+                box.fill(t, t.s.off[h] + (int)k, lane);
+                uint64_t used = 0;   // nodes of this round that some point needs
+                const int rounds = (min(64, n - j0) + SUB - 1) / SUB;
+                for (int r = 0; r < rounds; ++r) {
+                    const int b = r * SUB + slot;
+                    const uint64_t votes = __ballot(need(box.lo[b], box.hi[b]));
+#pragma unroll
+                    for (int q = 0; q < SUB; ++q)
+                        if ((votes >> (q * P)) & ((1ull << P) - 1ull)) used |= 1ull << (r * SUB + q);
                 }
-                const uint64_t m0 = __ballot(keep0), m1 = __ballot(keep1);
-                const int tot = __popcll(m0) + __popcll(m1);
-                if (m + tot > kFront) {
-                    overflow = true;
-                    break;
-                }
-                const int pos = m + __popcll(m0 & below) + __popcll(m1 & below);
-                if (keep0) {
-                    fk[cur ^ 1][w][pos] = c0;
-                    if (to_leaf) flb[w][pos] = lb0;
-                }
-                if (keep1) {
-                    fk[cur ^ 1][w][pos + (keep0 ? 1 : 0)] = c0 + 1u;
-                    if (to_leaf) flb[w][pos + (keep0 ? 1 : 0)] = lb1;
-                }
-                m += tot;
+                queue_push(fk[cur ^ 1], m, j0 + lane < n && ((used >> lane) & 1ull), k, below);
             }
             lds_fence();
-            if (overflow) break;
             cur ^= 1;
             n = m;
         }
-        if (overflow) {
-            dist_dfs(t, leaf, seed, lane, p, pf, pm, best, bt);
-        } else {
-            // Candidates: the triangles of the surviving leaves that pass
-            // the sphere test are queued and their binary64 distances taken
-            // 64 at a time, so the wavefront runs the exact distance once per
-            // 64 candidates rather than once per leaf.  A test against an
-            // older, larger best only queues more, so the minimum is that of
-            // the full search.
-            // Two leaves per round, so each lane has two sphere reads in
-            // flight; both are culled against the best of the round's start.
-            int qn = 0;   // queued candidates, below 64 between rounds
-            for (int j = 0; j < n; j += 2) {
-                const int64_t k0 = fk[cur][w][j];
-                const int64_t k1 = (j + 1 < n) ? (int64_t)fk[cur][w][j + 1] : -1;
-                const bool use0 = !(k0 == seed || lb_beyond(flb[w][j], best));
-                const bool use1 = k1 >= 0 && !(k1 == seed || lb_beyond(flb[w][j + 1], best));
-                const int64_t t0 = use0 ? node_first(leaf, k0) + lane : 0;
-                const int64_t t1 = use1 ? node_first(leaf, k1) + lane : 0;
-                const bool pass0 = use0 && t0 < node_last(t.s, leaf, k0) && sphere_within(t, t0, p, pm, best);
-                const bool pass1 = use1 && t1 < node_last(t.s, leaf, k1) && sphere_within(t, t1, p, pm, best);
-                const uint64_t m0 = __ballot(pass0), m1 = __ballot(pass1);
-                if (pass0) cq[w][qn + __popcll(m0 & below)] = (uint32_t)t0;
-                qn += __popcll(m0);
-                if (pass1) cq[w][qn + __popcll(m1 & below)] = (uint32_t)t1;
-                qn += __popcll(m1);
-                while (qn >= 64) {
-                    lds_fence();
-                    tri_nearest(t, cq[w][lane], true, p, best, bt);
-                    qn -= 64;
-                    const uint32_t rest0 = lane < qn ? cq[w][64 + lane] : 0u;
-                    const uint32_t rest1 = lane + 64 < qn ? cq[w][128 + lane] : 0u;
-                    lds_fence();
-                    if (lane < qn) cq[w][lane] = rest0;
-                    if (lane + 64 < qn) cq[w][64 + lane] = rest1;
-                }
+        const int64_t coff = t.s.off[h - 1];
+        const int ccount = t.s.count[h - 1];
+        int m = 0;
+        for (int j0 = 0; j0 < n; j0 += 64) {
+            const int j = j0 + lane;
+            bool keep0 = false, keep1 = false;
+            uint32_t c0 = 0;
+            if (j < n) {
+                c0 = 2u * fk[cur][j];
+                const NodeRec r0 = load_node(t, (int)(coff + c0));
+                const bool two = (int)c0 + 1 < ccount;
+                const NodeRec r1 = load_node(t, (int)(coff + c0 + (two ? 1u : 0u)));
+                keep0 = keep(r0.lo, r0.hi);
+                keep1 = two && keep(r1.lo, r1.hi);
             }
-            if (qn > 0) {
+            const uint64_t m0 = __ballot(keep0), m1 = __ballot(keep1);
+            const int tot = __popcll(m0) + __popcll(m1);
+            if (m + tot > FRONT) return P > 1 ? -1 : n;
+            const int pos = m + __popcll(m0 & below) + __popcll(m1 & below);
+            if (keep0) fk[cur ^ 1][pos] = c0;
+            if (keep1) fk[cur ^ 1][pos + (keep0 ? 1 : 0)] = c0 + 1u;
+            m += tot;
+        }
+        lds_fence();
+        cur ^= 1;
+        n = m;
+        level = h - 1;
+    }
+    return n;
+}
+
+// points of a packet that goes to the second pass
+__device__ inline void packet_pass_on(bool valid, int64_t i, int lane, uint32_t* rest, unsigned* rest_n) {
+    const uint64_t m = __ballot(valid);
+    unsigned base = 0;
+    if (lane == 0) base = atomicAdd(rest_n, (unsigned)__popcll(m));
+    base = (unsigned)wave_uniform((int)base);
+    if (valid) rest[base + __popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)i;
+}
+
+// Point sets below this take the second pass alone: 2,000 packets or fewer
+// leave most of the chip's 1,024 SIMDs with one wavefront or none, and 16
+// times as many wavefronts hide more (20,000 uniform points around a
+// 10,000-triangle torus: 0.61 ms in packets, 0.47 one by one; 100,000: 0.74
+// in packets).
+constexpr int64_t kPacketPoints = 32768;
+
+// out holds the seeds' squared distances on entry
+template <int P, int FRONT>
+__global__ __launch_bounds__(64, 5) void k_dist_packet(TreeView t, const double* pts, Work work, const int32_t* seed_at,
+                                                    double* out, int32_t* tri_out, uint32_t* rest, unsigned* rest_n) {
+    constexpr int SUB = 64 / P;   // buckets tested at once
+    __shared__ uint32_t fk[2][FRONT];
+    __shared__ BoxStage box;
+    __shared__ uint32_t pairs[kPairQueue];   // frontier slot * P + point
+    __shared__ uint32_t cand[kTriQueue];     // (frontier slot * 8 + triangle) * P + point
+    __shared__ double sp[3][P];
+    __shared__ float sub[P];               // upper bounds with margin
+    __shared__ float4 sseed[P];            // bounding spheres of the points' seed triangles
+    __shared__ unsigned long long sbest[P];   // bits of the best squared distance (order of non-negative doubles)
+    __shared__ int32_t sid[P];
+    const int lane = threadIdx.x, pt = lane & (P - 1), slot = lane / P;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int64_t N = work.size(), groups = (N + P - 1) / P;
+    const NodeRec root = load_node(t, t.s.off[t.s.H]);
+    const float rs = root_scale(root);
+    const int start = start_level(t.s, std::min(stop_level(P), (int)t.s.H), start_nodes(P));
+    for (int64_t g = blockIdx.x; g < groups; g += gridDim.x) {
+    // the far points' packets, the longest, are last in the order and taken first
+    const int64_t at = (groups - 1 - g) * P + pt;
+    const bool valid = at < N;
+    const int64_t i = work.point(valid ? at : N - 1);
+    const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
+    const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
+    // a coordinate beyond binary32 (or NaN) is for the node-by-node walk
+    const bool wild = __ballot(!(isfinite(pf[0]) && isfinite(pf[1]) && isfinite(pf[2]))) != 0ull;
+    const float pm = fmaxf(fabsf(pf[0]), fmaxf(fabsf(pf[1]), fabsf(pf[2])));
+    const float M = bound_margin(pm + 4.f * rs);   // covers any centre and radius of the tree
+    auto upper = [M](double d2) { return sqrtf((float)d2) * 1.000001f + M; };
+    const double seed_d2 = out[i];
+    float ubm = upper(seed_d2);   // upper bound of the distance, with the margin
+    lds_fence();   // the packet before has been read
+    if (slot == 0) {
+        const int32_t j = seed_at[i];
+        for (int a = 0; a < 3; ++a) sp[a][pt] = p[a];
+        sseed[pt] = t.sph[j];
+        sbest[pt] = (unsigned long long)__double_as_longlong(seed_d2);
+        sid[pt] = seed_d2 < INFINITY ? t.tid[j] : 0x7fffffff;
+    }
+    lds_fence();
+    // A point's Morton position can miss a triangle that a neighbour's found:
+    // the centres of all the packet's seeds bound its distance too.
+    for (int q = slot; q < P; q += SUB) {
+        const float4 S = sseed[q];
+        const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z;
+        ubm = fminf(ubm, sqrtf(dx * dx + dy * dy + dz * dz) + M);
+    }
+#pragma unroll
+    for (int o = P; o < 64; o <<= 1) ubm = fminf(ubm, __shfl_xor(ubm, o, 64));
+    if (slot == 0) sub[pt] = ubm;
+    // the packet's box, grown by the largest upper bound
+    float blo[3], bhi[3];
+    for (int a = 0; a < 3; ++a) {
+        blo[a] = wave_min_f(pf[a]);
+        bhi[a] = wave_max_f(pf[a]);
+    }
+    const float reach = wave_max_f(ubm), reach2 = reach * reach;
+    // can the box hold a triangle nearer than this lane's point has found?
+    auto needs = [&](float4 lo, float4 hi) {
+        const float ex = fmaxf(fmaxf(lo.x - pf[0], pf[0] - hi.x), 0.f);
+        const float ey = fmaxf(fmaxf(lo.y - pf[1], pf[1] - hi.y), 0.f);
+        const float ez = fmaxf(fmaxf(lo.z - pf[2], pf[2] - hi.z), 0.f);
+        return valid && !(ex * ex + ey * ey + ez * ez > ubm * ubm);
+    };
+    int cur = 0;
+    int level = 0;
+    const int n = wild ? -1 : packet_frontier<P, FRONT>(t, start, lane, fk, box, cur, level, [&](float4 lo, float4 hi) {
+        const float ex = fmaxf(fmaxf(lo.x - bhi[0], blo[0] - hi.x), 0.f);
+        const float ey = fmaxf(fmaxf(lo.y - bhi[1], blo[1] - hi.y), 0.f);
+        const float ez = fmaxf(fmaxf(lo.z - bhi[2], blo[2] - hi.z), 0.f);
+        return !(ex * ex + ey * ey + ez * ez > reach2);
+    }, needs);
+    if (n < 0) {
+        if (P > 1) {
+            packet_pass_on(valid && slot == 0, i, lane, rest, rest_n);
+        } else {   // the node-by-node walk of the one point
+            double best = seed_d2;
+            int32_t bt = sid[0];
+            dist_dfs(t, std::min(kLeafLevel, (int)t.s.H), lane, p, pf, pm, best, bt);
+            if (lane == 0) {
+                out[i] = sqrt(best);
+                if (tri_out) tri_out[i] = bt;
+            }
+        }
+        continue;
+    }
+    // points much farther than a triangle's size also test the planes
+    const bool planes = reach > 4.f * sseed[0].w;
+    int qp = 0, qt = 0;
+    const int nb = n << level;   // buckets of the frontier
+    uint64_t have = 0;           // which of the 64 staged buckets exist
+    for (int j0 = 0;; j0 += SUB) {
+        const bool more = j0 < nb;
+        if (more) {
+            const int j = j0 + slot;
+            bool pass = false;
+            if ((j0 & 63) == 0) {   // the next 64 buckets
+                const int b = j0 + lane < nb ? front_bucket(fk[cur], level, (uint32_t)(j0 + lane)) : 0;
+                have = __ballot(j0 + lane < nb && b < t.s.count[0]);
+                box.fill(t, t.s.off[0] + min(b, t.s.count[0] - 1), lane);
+            }
+            if ((have >> (j & 63)) & 1ull) pass = needs(box.lo[j & 63], box.hi[j & 63]);
+            queue_push(pairs, qp, pass, (uint32_t)(j * P + pt), below);
+        }
+        if (qp >= 64 || (!more && qp > 0)) {
+            lds_fence();
+            const int cnt = min(qp, 64);
+            qp -= cnt;
+            const bool take = lane < cnt;
+            const uint32_t e = pairs[qp + (take ? lane : 0)];
+            const int o = (int)(e & (P - 1));
+            const uint32_t js = e / P;
+            const float ox = (float)sp[0][o], oy = (float)sp[1][o], oz = (float)sp[2][o], ou = sub[o];
+            const int first = front_bucket(fk[cur], level, js) * kBucket;
+#pragma unroll
+            for (int q = 0; q < kBucket; ++q) {
+                const int k = first + q;
+                const float4 S = t.sph[min(k, t.s.T - 1)];
+                const float dx = ox - S.x, dy = oy - S.y, dz = oz - S.z, lim = ou + S.w;
+                bool pass = take && k < t.s.T && !(dx * dx + dy * dy + dz * dz > lim * lim);
+                if (planes && pass) {
+                    const float4 nr = t.nrm[k];
+                    pass = !(fabsf(nr.x * dx + nr.y * dy + nr.z * dz) > ou);
+                }
+                queue_push(cand, qt, pass, (js * kBucket + q) * P + o, below);
+            }
+        }
+        while (qt >= 64 || (!more && qp == 0 && qt > 0)) {
+            lds_fence();
+            const int cnt = min(qt, 64);
+            qt -= cnt;
+            const bool take = lane < cnt;
+            const uint32_t e = cand[qt + (take ? lane : 0)];
+            const int o = (int)(e & (P - 1));
+            const uint32_t jq = e / P;
+            const int64_t k = (int64_t)front_bucket(fk[cur], level, jq / kBucket) * kBucket + jq % kBucket;
+            const double q[3] = {sp[0][o], sp[1][o], sp[2][o]};
+            const double* T = t.tris + 9 * k;
+            double d2 = point_tri_dist2(q, T, T + 3, T + 6);
+            int32_t id = t.tid[k];
+            if (!take || !(d2 <= INFINITY)) {   // a degenerate triangle never wins
+                d2 = INFINITY;
+                id = 0x7fffffff;
+            }
+            const unsigned long long bits = (unsigned long long)__double_as_longlong(d2), pre = sbest[o];
+            lds_fence();
+            if (P == 1) {   // one point: a butterfly instead of 64 atomics on one word
+                wave_argmin(d2, id);
+                if (lane == 0) {
+                    const unsigned long long now = (unsigned long long)__double_as_longlong(d2);
+                    if (now < pre || (now == pre && id < sid[0])) sid[0] = id;
+                    sbest[0] = now < pre ? now : pre;
+                }
+            } else {
+                if (take) atomicMin(&sbest[o], bits);
                 lds_fence();
-                tri_nearest(t, lane < qn ? cq[w][lane] : 0u, lane < qn, p, best, bt);
+                const unsigned long long now = sbest[o];
+                const bool win = take && bits == now;
+                if (win && now < pre) sid[o] = 0x7fffffff;   // a smaller distance: the old index does not count
+                lds_fence();
+                if (win) atomicMin(&sid[o], id);
             }
             lds_fence();
+            ubm = fminf(ubm, upper(__longlong_as_double((long long)sbest[pt])));
+            sub[pt] = ubm;   // the same value from every lane of the point
+            lds_fence();
         }
-        if (lane == 0) {
-            out[i] = sqrt(best);
-            if (tri_out) tri_out[i] = bt;
-        }
+        if (!more && qp == 0 && qt == 0) break;
+    }
+    if (valid && slot == 0) {
+        out[i] = sqrt(__longlong_as_double((long long)sbest[pt]));
+        if (tri_out) tri_out[i] = sid[pt];
+    }
     }
 }
 
@@ -1261,21 +1583,6 @@ __device__ inline Ray choose_ray(const double p[3], float4 lo, float4 hi) {
     return R;
 }
 
-// false when the ray surely misses sorted triangle j: its bounding sphere,
-// which holds the triangle with a margin for the binary32 rounding here,
-// lies wholly beside the ray or wholly behind p.  Such a triangle is
-// rejected without reading its binary64 vertices; that p lies outside its
-// projection is then certain, so the crossing count is unchanged.
-__device__ inline bool sphere_on_ray(const TreeView& t, int64_t j, const double p[3], float pm, const Ray& R) {
-    const float4 S = t.sph[j];
-    const float du = (float)sel3(p, R.u) - sel3(S, R.u), dv = (float)sel3(p, R.v) - sel3(S, R.v);
-    const float dw = (float)sel3(p, R.w) - sel3(S, R.w);
-    const float m = bound_margin(pm + fmaxf(fabsf(S.x), fmaxf(fabsf(S.y), fabsf(S.z))) + S.w);
-    const float beside = sqrtf(du * du + dv * dv) - S.w - m;
-    const float behind = (R.sg > 0 ? dw : -dw) - S.w - m;
-    return !(beside > 0.f) && !(behind > 0.f);
-}
-
 // Signed crossing of the ray from p with one triangle: +1 / -1 (the sign of
 // n . d, its normal against the ray direction) when the ray crosses it ahead
 // of p, else 0; unsure is set when an orientation that decides this is not
@@ -1316,146 +1623,148 @@ __device__ inline int tri_ray(const double* T, const double p[3], const Ray& R, 
     return s4 == dir ? dir : 0;
 }
 
-// Winding numbers of a closed mesh by an axis ray (see the file comment):
-// the wavefront walks the tree level by level, keeping the nodes whose
-// boxes meet the ray, then tests the triangles of the leaves it reaches,
-// one per lane.  decided[i] = 1 and the sign is applied when every
-// orientation was certain and the lists fitted; otherwise decided[i] = 0
-// and the fan walk takes the point.
-constexpr int kRayFront = 256, kRayLeaves = 64;
-// the ray walk starts at up to 256 nodes (four per lane), one round lower
-constexpr int kRayStartNodes = 256;
-__device__ inline bool box_on_ray(const double p[3], float4 lo, float4 hi, const Ray& R) {
-    const double pu = sel3(p, R.u), pv = sel3(p, R.v), pw = sel3(p, R.w);
-    return pu >= (double)sel3(lo, R.u) && pu <= (double)sel3(hi, R.u) && pv >= (double)sel3(lo, R.v) &&
-           pv <= (double)sel3(hi, R.v) && (R.sg > 0 ? pw <= (double)sel3(hi, R.w) : pw >= (double)sel3(lo, R.w));
-}
-__global__ __launch_bounds__(kT) void k_sdf_ray(TreeView t, const double* pts, int64_t N, double* out,
-                                               uint8_t* decided, unsigned* undecided) {
-    __shared__ uint32_t fk[2][kWavesPerBlock][kRayFront];
-    __shared__ uint32_t leaves[kWavesPerBlock][kRayLeaves];
-    __shared__ uint32_t cq[kWavesPerBlock][kCandQueue];   // candidate triangles (sorted positions)
-    const int lane = threadIdx.x & 63, w = wave_uniform((int)(threadIdx.x >> 6));
+// Crossings of a packet: all its rays take the axis direction that leaves the
+// mesh's box soonest from the middle of the packet (any ray gives the winding
+// number), so one walk serves them all.
+// decided[i] = 1 and the sign is applied when every orientation was certain
+// and the lists fitted; otherwise decided[i] = 0 and the fan walk takes the
+// point.
+template <int P, int FRONT>
+__global__ __launch_bounds__(64, 5) void k_ray_packet(TreeView t, const double* pts, Work work, double* out,
+                                                   uint8_t* decided, unsigned* undecided, uint32_t* rest,
+                                                   unsigned* rest_n) {
+    constexpr int SUB = 64 / P;   // buckets tested at once
+    __shared__ uint32_t fk[2][FRONT];
+    __shared__ BoxStage box;
+    __shared__ uint32_t pairs[kPairQueue];   // frontier slot * P + point
+    __shared__ uint32_t cand[kTriQueue];     // (frontier slot * 8 + triangle) * P + point
+    __shared__ double sp[3][P];
+    __shared__ float sf[4][P];             // u, v, place along the ray, margin
+    __shared__ int scross[P], sunsure[P];
+    const int lane = threadIdx.x, pt = lane & (P - 1), slot = lane / P;
     const uint64_t below = (1ull << lane) - 1ull;
-    const int64_t nw = (int64_t)gridDim.x * kWavesPerBlock;
-    const int leaf = std::min(kLeafLevel, (int)t.s.H);
-    const int start = start_level(t.s, leaf, kRayStartNodes), start_count = t.s.count[start];
+    const int64_t N = work.size(), groups = (N + P - 1) / P;
     const NodeRec root = load_node(t, t.s.off[t.s.H]);
-    for (int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + w; i < N; i += nw) {
-        const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
-        bool unsure = !(isfinite(p[0]) && isfinite(p[1]) && isfinite(p[2]));
-        const Ray R = choose_ray(p, root.lo, root.hi);
-        int n = 0, cur = 0, nl = 0;
-        {   // the nodes of the start level whose boxes meet the ray
-            constexpr int kQ = kRayStartNodes / 64;
-            static_assert(kRayStartNodes <= kRayFront && kRayStartNodes % 64 == 0, "start nodes: kQ per lane");
-            bool keep[kQ];
+    const float rs = root_scale(root);
+    const int start = start_level(t.s, std::min(stop_level(P), (int)t.s.H), start_nodes(P));
+    for (int64_t g = blockIdx.x; g < groups; g += gridDim.x) {
+    const int64_t at = (groups - 1 - g) * P + pt;
+    const bool valid = at < N;
+    const int64_t i = work.point(valid ? at : N - 1);
+    const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
+    const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
+    const bool wild = __ballot(!(isfinite(pf[0]) && isfinite(pf[1]) && isfinite(pf[2]))) != 0ull;
+    double mid[3];
+    for (int a = 0; a < 3; ++a) mid[a] = 0.5 * ((double)wave_min_f(pf[a]) + (double)wave_max_f(pf[a]));
+    Ray R = choose_ray(mid, root.lo, root.hi);
+    R.w = wave_uniform(R.w);
+    R.sg = wave_uniform(R.sg);
+    R.u = R.w == 2 ? 0 : R.w + 1;
+    R.v = R.u == 2 ? 0 : R.u + 1;
+    const bool fwd = R.sg > 0;
+    const float pm = fmaxf(fabsf(pf[0]), fmaxf(fabsf(pf[1]), fabsf(pf[2])));
+    const float M = bound_margin(pm + 4.f * rs);
+    auto at3 = [](float x, float y, float z, int a) { return a == 0 ? x : (a == 1 ? y : z); };
+    const float pu = at3(pf[0], pf[1], pf[2], R.u), pv = at3(pf[0], pf[1], pf[2], R.v);
+    const float pw = at3(pf[0], pf[1], pf[2], R.w) * (fwd ? 1.f : -1.f);   // place along the ray
+    lds_fence();   // the packet before has been read
+    if (slot == 0) {
+        for (int a = 0; a < 3; ++a) sp[a][pt] = p[a];
+        sf[0][pt] = pu;
+        sf[1][pt] = pv;
+        sf[2][pt] = pw;
+        sf[3][pt] = M;
+        scross[pt] = 0;
+        sunsure[pt] = 0;
+    }
+    const float ulo = wave_min_f(pu - M), uhi = wave_max_f(pu + M);
+    const float vlo = wave_min_f(pv - M), vhi = wave_max_f(pv + M);
+    const float wlo = wave_min_f(pw - M);
+    // last place of a box along the ray
+    auto box_far = [&](float4 lo, float4 hi) { return fwd ? sel3(hi, R.w) : -sel3(lo, R.w); };
+    // does the ray of this lane's point meet the box?
+    auto needs = [&](float4 lo, float4 hi) {
+        return valid && !(sel3(hi, R.u) < pu - M || sel3(lo, R.u) > pu + M || sel3(hi, R.v) < pv - M ||
+                          sel3(lo, R.v) > pv + M || box_far(lo, hi) < pw - M);
+    };
+    int cur = 0;
+    int level = 0;
+    const int n = wild ? -1 : packet_frontier<P, FRONT>(t, start, lane, fk, box, cur, level, [&](float4 lo, float4 hi) {
+        return !(sel3(hi, R.u) < ulo || sel3(lo, R.u) > uhi || sel3(hi, R.v) < vlo || sel3(lo, R.v) > vhi ||
+                 box_far(lo, hi) < wlo);
+    }, needs);
+    if (n < 0) {
+        if (P > 1) {
+            packet_pass_on(valid && slot == 0, i, lane, rest, rest_n);
+        } else if (lane == 0) {
+            decided[i] = 0;
+            atomicAdd(undecided, 1u);
+        }
+        continue;
+    }
+    int qp = 0, qt = 0;
+    const int nb = n << level;   // buckets of the frontier
+    uint64_t have = 0;           // which of the 64 staged buckets exist
+    for (int j0 = 0;; j0 += SUB) {
+        const bool more = j0 < nb;
+        if (more) {
+            const int j = j0 + slot;
+            bool pass = false;
+            if ((j0 & 63) == 0) {   // the next 64 buckets
+                const int b = j0 + lane < nb ? front_bucket(fk[cur], level, (uint32_t)(j0 + lane)) : 0;
+                have = __ballot(j0 + lane < nb && b < t.s.count[0]);
+                box.fill(t, t.s.off[0] + min(b, t.s.count[0] - 1), lane);
+            }
+            if ((have >> (j & 63)) & 1ull) pass = needs(box.lo[j & 63], box.hi[j & 63]);
+            queue_push(pairs, qp, pass, (uint32_t)(j * P + pt), below);
+        }
+        if (qp >= 64 || (!more && qp > 0)) {
+            lds_fence();
+            const int cnt = min(qp, 64);
+            qp -= cnt;
+            const bool take = lane < cnt;
+            const uint32_t e = pairs[qp + (take ? lane : 0)];
+            const int o = (int)(e & (P - 1));
+            const uint32_t js = e / P;
+            const float ou = sf[0][o], ov = sf[1][o], ow = sf[2][o], om = sf[3][o];
+            const int first = front_bucket(fk[cur], level, js) * kBucket;
 #pragma unroll
-            for (int q = 0; q < kQ; ++q) {
-                keep[q] = false;
-                if (!unsure && lane + 64 * q < start_count) {
-                    const NodeRec r = load_node(t, t.s.off[start] + lane + 64 * q);
-                    keep[q] = box_on_ray(p, r.lo, r.hi, R);
-                }
+            for (int q = 0; q < kBucket; ++q) {
+                const int k = first + q;
+                const float4 S = t.sph[min(k, t.s.T - 1)];
+                // wholly beside the ray or behind its start: no crossing
+                const float du = ou - sel3(S, R.u), dv = ov - sel3(S, R.v), lim = S.w + om;
+                const float behind = ow - sel3(S, R.w) * (fwd ? 1.f : -1.f);
+                const bool pass = take && k < t.s.T && !(du * du + dv * dv > lim * lim) && !(behind > lim);
+                queue_push(cand, qt, pass, (js * kBucket + q) * P + o, below);
             }
-            lds_fence();
-#pragma unroll
-            for (int q = 0; q < kQ; ++q) {
-                const uint64_t m = __ballot(keep[q]);
-                if (keep[q]) fk[0][w][n + __popcll(m & below)] = (uint32_t)(lane + 64 * q);
-                n += __popcll(m);
-            }
-            lds_fence();
         }
-        for (int h = start; n > 0; --h) {
-            if (h <= leaf) {   // every node of this level is a leaf
-                if (nl + n > kRayLeaves) {
-                    unsure = true;
-                    break;
-                }
-                for (int j = lane; j < n; j += 64) leaves[w][nl + j] = fk[cur][w][j];
-                nl += n;
-                lds_fence();
-                break;
-            }
-            const int64_t coff = t.s.off[h - 1];
-            const int cnext = t.s.count[h - 1];
-            int m = 0;
-            for (int j0 = 0; j0 < n; j0 += 64) {
-                const int j = j0 + lane;
-                bool keep0 = false, keep1 = false;
-                uint32_t c0 = 0;
-                if (j < n) {
-                    c0 = 2u * fk[cur][w][j];
-                    const NodeRec r0 = load_node(t, (int)(coff + c0));
-                    keep0 = box_on_ray(p, r0.lo, r0.hi, R);
-                    if ((int)c0 + 1 < cnext) {
-                        const NodeRec r1 = load_node(t, (int)(coff + c0 + 1));
-                        keep1 = box_on_ray(p, r1.lo, r1.hi, R);
-                    }
-                }
-                const uint64_t m0 = __ballot(keep0), m1 = __ballot(keep1);
-                const int tot = __popcll(m0) + __popcll(m1);
-                if (m + tot > kRayFront) {
-                    unsure = true;
-                    break;
-                }
-                const int pos = m + __popcll(m0 & below) + __popcll(m1 & below);
-                if (keep0) fk[cur ^ 1][w][pos] = c0;
-                if (keep1) fk[cur ^ 1][w][pos + (keep0 ? 1 : 0)] = c0 + 1u;
-                m += tot;
-            }
+        while (qt >= 64 || (!more && qp == 0 && qt > 0)) {
             lds_fence();
-            if (unsure) break;
-            cur ^= 1;
-            n = m;
-        }
-        // Candidates: the triangles of the reached leaves whose bounding
-        // spheres meet the ray are queued and tested 64 at a time, so the
-        // wavefront reads binary64 vertices and runs the crossing test once
-        // per 64 candidates rather than once per leaf.  The count is a sum of
-        // integers, so the order does not change it.
-        int cross = 0;
-        bool lane_unsure = false;
-        if (!unsure) {
-            const float pm = fmaxf(fabsf((float)p[0]), fmaxf(fabsf((float)p[1]), fabsf((float)p[2])));
-            int qn = 0;   // queued candidates, below 64 between rounds (two leaves a round)
-            for (int l = 0; l < nl; l += 2) {
-                const int64_t k0 = leaves[w][l];
-                const int64_t k1 = (l + 1 < nl) ? (int64_t)leaves[w][l + 1] : -1;
-                const int64_t j0 = node_first(leaf, k0) + lane;
-                const int64_t j1 = k1 >= 0 ? node_first(leaf, k1) + lane : 0;
-                const bool pass0 = j0 < node_last(t.s, leaf, k0) && sphere_on_ray(t, j0, p, pm, R);
-                const bool pass1 = k1 >= 0 && j1 < node_last(t.s, leaf, k1) && sphere_on_ray(t, j1, p, pm, R);
-                const uint64_t m0 = __ballot(pass0), m1 = __ballot(pass1);
-                if (pass0) cq[w][qn + __popcll(m0 & below)] = (uint32_t)j0;
-                qn += __popcll(m0);
-                if (pass1) cq[w][qn + __popcll(m1 & below)] = (uint32_t)j1;
-                qn += __popcll(m1);
-                while (qn >= 64) {
-                    lds_fence();
-                    cross += tri_ray(t.tris + 9 * (int64_t)cq[w][lane], p, R, lane_unsure);
-                    qn -= 64;
-                    const uint32_t rest0 = lane < qn ? cq[w][64 + lane] : 0u;
-                    const uint32_t rest1 = lane + 64 < qn ? cq[w][128 + lane] : 0u;
-                    lds_fence();
-                    if (lane < qn) cq[w][lane] = rest0;
-                    if (lane + 64 < qn) cq[w][64 + lane] = rest1;
-                }
-            }
-            if (qn > 0) {
-                lds_fence();
-                if (lane < qn) cross += tri_ray(t.tris + 9 * (int64_t)cq[w][lane], p, R, lane_unsure);
+            const int cnt = min(qt, 64);
+            qt -= cnt;
+            if (lane < cnt) {
+                const uint32_t e = cand[qt + lane];
+                const int o = (int)(e & (P - 1));
+                const uint32_t jq = e / P;
+                const int64_t k = (int64_t)front_bucket(fk[cur], level, jq / kBucket) * kBucket + jq % kBucket;
+                const double q[3] = {sp[0][o], sp[1][o], sp[2][o]};
+                bool unsure = false;
+                const int c = tri_ray(t.tris + 9 * k, q, R, unsure);
+                if (c) atomicAdd(&scross[o], c);
+                if (unsure) sunsure[o] = 1;
             }
             lds_fence();
         }
-        unsure = unsure || __ballot(lane_unsure) != 0ull;
-        const int wn = wave_sum(cross);
-        if (lane == 0) {
-            decided[i] = unsure ? 0 : 1;
-            if (unsure) atomicAdd(undecided, 1u);
-            if (!unsure && wn >= 1) out[i] = -out[i];   // winding number > 1/2
-        }
+        if (!more && qp == 0 && qt == 0) break;
+    }
+    const bool mine = valid && slot == 0, unsure = mine && sunsure[pt] != 0;
+    const uint64_t mu = __ballot(unsure);
+    if (mu != 0ull && lane == 0) atomicAdd(undecided, (unsigned)__popcll(mu));
+    if (mine) {
+        decided[i] = unsure ? 0 : 1;
+        if (!unsure && scross[pt] >= 1) out[i] = -out[i];   // winding number > 1/2
+    }
     }
 }
 
@@ -1546,22 +1855,42 @@ void signed_distance(hipStream_t st, const double* d_V, int64_t nV, const int32_
     if (N <= 0) return;
     TriTree tr;
     tree_build(tr, st, d_V, nV, d_F, nF);
-    // One wavefront per point, grid-strided over as many blocks as the CUs
-    // hold at once for that kernel: a block that waited for a free slot would
-    // start its whole share after the resident blocks ended theirs.
+    // grid-strided launches: as many blocks as the CUs hold at once
     int dev = 0, cus = 256;
     ITS_HIP(hipGetDevice(&dev));
     ITS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    auto grid_of = [&](const void* kernel) {
+    auto grid_of = [&](const void* kernel, int threads, int64_t most) {
         int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kT, 0) != hipSuccess || per_cu < 1) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess || per_cu < 1) {
             (void)hipGetLastError();
             per_cu = 1;
         }
-        return (unsigned)std::min<int64_t>((N + kWavesPerBlock - 1) / kWavesPerBlock, (int64_t)per_cu * cus);
+        return (unsigned)std::min<int64_t>(most, (int64_t)per_cu * cus);
     };
-    hipLaunchKernelGGL(k_sdf_dist, dim3(grid_of((const void*)k_sdf_dist)), dim3(kT), 0, st, tr.view(), d_pts, N, d_out,
-                       d_tri);
+    constexpr auto dist1 = k_dist_packet<kPk, kFrontPacket>, dist2 = k_dist_packet<1, kFrontPoint>;
+    constexpr auto ray1 = k_ray_packet<kPk, kFrontPacket>, ray2 = k_ray_packet<1, kFrontPoint>;
+    // every point's seed; with packets, also their order
+    const bool packets = N >= kPacketPoints && N < (int64_t(1) << 32);
+    DBuf<uint32_t> key(N), order(N), rest;
+    DBuf<int32_t> seed_at(N);
+    hipLaunchKernelGGL(k_pt_seed, dim3(blocks_for(N, kT)), dim3(kT), 0, st, tr.view(), d_pts, N, key.p, order.p, d_out,
+                       seed_at.p);
+    ITS_LAUNCH_CHECK();
+    DBuf<unsigned> counts(3);   // points passed on by the two packet kernels, undecided points
+    ITS_HIP(hipMemsetAsync(counts.p, 0, counts.bytes(), st));
+    const unsigned pgrid = (unsigned)((N + kPk - 1) / kPk);
+    Work all{N, nullptr, nullptr}, left = all;
+    if (packets) {
+        radix_sort(key, &order, N, kSeedKeyBits, st);
+        rest.alloc(N);
+        all.list = order.p;
+        left = Work{N, rest.p, counts.p};
+        hipLaunchKernelGGL(dist1, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, (const int32_t*)seed_at.p, d_out,
+                           d_tri, rest.p, counts.p);
+        ITS_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(dist2, dim3(grid_of((const void*)dist2, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left,
+                       (const int32_t*)seed_at.p, d_out, d_tri, (uint32_t*)nullptr, (unsigned*)nullptr);
     ITS_LAUNCH_CHECK();
     tr.closed = read1(tr.is_open.p, st) == 0;
     // closed mesh: signs by the ray where it decides them; the fans are built
@@ -1570,16 +1899,20 @@ void signed_distance(hipStream_t st, const double* d_V, int64_t nV, const int32_
     int64_t undecided = N;
     if (tr.closed && tune_get(ITS_TUNE_SDF_RAY)) {
         decided.alloc(N);
-        DBuf<unsigned> count(1);
-        ITS_HIP(hipMemsetAsync(count.p, 0, sizeof(unsigned), st));
-        hipLaunchKernelGGL(k_sdf_ray, dim3(grid_of((const void*)k_sdf_ray)), dim3(kT), 0, st, tr.view(), d_pts, N, d_out,
-                           decided.p, count.p);
+        if (packets) {
+            left.list_n = counts.p + 1;
+            hipLaunchKernelGGL(ray1, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, d_out, decided.p,
+                               counts.p + 2, rest.p, counts.p + 1);
+            ITS_LAUNCH_CHECK();
+        }
+        hipLaunchKernelGGL(ray2, dim3(grid_of((const void*)ray2, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left, d_out,
+                           decided.p, counts.p + 2, (uint32_t*)nullptr, (unsigned*)nullptr);
         ITS_LAUNCH_CHECK();
-        undecided = read1(count.p, st);
+        undecided = read1(counts.p + 2, st);
     }
     if (undecided > 0) {
         fans_build(tr, st, d_V);
-        hipLaunchKernelGGL(k_sdf_wind, dim3(grid_of((const void*)k_sdf_wind)), dim3(kT), 0, st, tr.view(), d_pts, N, d_out,
+        hipLaunchKernelGGL(k_sdf_wind, dim3(grid_of((const void*)k_sdf_wind, kT, (N + kWavesPerBlock - 1) / kWavesPerBlock)), dim3(kT), 0, st, tr.view(), d_pts, N, d_out,
                            (const uint8_t*)decided.p);
         ITS_LAUNCH_CHECK();
     }
