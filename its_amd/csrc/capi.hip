@@ -695,15 +695,11 @@ ShellInput shell_upload(const double* V, int64_t nV, const int32_t* F, int64_t n
     for (int64_t i = 0; i < 3 * nF; ++i)
         ITS_REQUIRE(F[i] >= 0 && F[i] < nV, ITS_E_INVALID, "face index out of range");
     ShellInput in;
-    std::vector<uint64_t> e = mesh_edges(F, nF);
-    std::vector<double> t(9 * (size_t)nF);
-    for (int64_t f = 0; f < nF; ++f)
-        for (int c = 0; c < 3; ++c)
-            for (int a = 0; a < 3; ++a) t[9 * f + 3 * c + a] = V[3 * (int64_t)F[3 * f + c] + a];
     in.V = upload(V, 3 * (size_t)nV, st);
-    in.tris = upload(t.data(), t.size(), st);
-    in.edges = upload(e.data(), e.size(), st);
-    in.ne = (int64_t)e.size();
+    DBuf<int32_t> d_F = upload(F, 3 * (size_t)nF, st);
+    in.tris.alloc(9 * (size_t)nF);
+    face_corners(in.V.p, d_F.p, nF, in.tris.p, st);
+    in.ne = mesh_edges(d_F.p, nF, nV, in.edges, st);
     return in;
 }
 }  // namespace
@@ -749,12 +745,17 @@ int its_shell_iso(its_ctx ctx, its_svo s, const double* V, int64_t nV, const int
     const double dummy[3] = {0, 0, 0};
     eval_points_aos64(s, in.V.p, nV, dummy, ITS_EVAL_RAW, 0.f, f.p, st);
     if (np > 0) eval_points_aos64(s, P.p, np, dummy, ITS_EVAL_RAW, 0.f, f.p + nV, st);
-    std::vector<float> h(nall);
-    ITS_HIP(hipMemcpyAsync(h.data(), f.p, nall * sizeof(float), hipMemcpyDeviceToHost, st));
-    ITS_HIP(hipStreamSynchronize(st));
-    const auto mm = std::minmax_element(h.begin(), h.end());
-    iso[0] = *mm.first;
-    iso[1] = *mm.second;
+    float range[2];
+    if (!value_range(f.p, nall, range, st)) {   // a NaN: whatever comparing in order leaves
+        std::vector<float> h(nall);
+        ITS_HIP(hipMemcpyAsync(h.data(), f.p, nall * sizeof(float), hipMemcpyDeviceToHost, st));
+        ITS_HIP(hipStreamSynchronize(st));
+        const auto mm = std::minmax_element(h.begin(), h.end());
+        range[0] = *mm.first;
+        range[1] = *mm.second;
+    }
+    iso[0] = range[0];
+    iso[1] = range[1];
     if (n_points) *n_points = np;
     ITS_API_END
 }

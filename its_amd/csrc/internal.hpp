@@ -133,6 +133,8 @@ void mc_lattice(its_svo s, const double origin[3], const double width[3], const 
 // sdf.hip
 void signed_distance(hipStream_t st, const double* d_V, int64_t nV, const int32_t* d_F, int64_t nF,
                      const double* d_pts, int64_t N, double* d_out, int32_t* d_tri);
+// stable radix sort of the low `bits` bits, in place
+void sort_u64(DBuf<uint64_t>& keys, int64_t n, int bits, hipStream_t st);
 void nearest_normals(hipStream_t st, const double* d_V, const int32_t* d_F, const int32_t* d_tri, int64_t N,
                      float4* d_nrm);
 void eval_batch(its_svo const* svos, int64_t count, const int64_t* off, const float* x, const float* y,
@@ -149,7 +151,9 @@ void eval_batch_noalloc(its_svo const* svos, int64_t count, const int64_t* off, 
 int64_t fine_edges(its_svo s, DBuf<double>& ends, DBuf<uint32_t>& owner, hipStream_t st);
 void shell_points(its_svo s, const double* d_V, const uint64_t* d_edges, int64_t ne, const double* d_tris, int64_t nT,
                   DBuf<double>& pts, int64_t* n_edge, int64_t* n_face, hipStream_t st);
-std::vector<uint64_t> mesh_edges(const int32_t* F, int64_t nF);
+int64_t mesh_edges(const int32_t* d_F, int64_t nF, int64_t nV, DBuf<uint64_t>& edges, hipStream_t st);
+void face_corners(const double* d_V, const int32_t* d_F, int64_t nF, double* d_tris, hipStream_t st);
+bool value_range(const float* d_f, int64_t n, float range[2], hipStream_t st);
 // batch.hip
 its_batch batch_new(its_ctx ctx);
 void batch_delete(its_batch b);

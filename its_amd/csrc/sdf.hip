@@ -1942,4 +1942,8 @@ void nearest_normals(hipStream_t st, const double* d_V, const int32_t* d_F, cons
     ITS_LAUNCH_CHECK();
 }
 
+void sort_u64(DBuf<uint64_t>& keys, int64_t n, int bits, hipStream_t st) {
+    radix_sort(keys, (DBuf<uint32_t>*)nullptr, n, bits, st);
+}
+
 }  // namespace its

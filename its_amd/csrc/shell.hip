@@ -5,7 +5,7 @@
 // and the min / max of cpLatentBSplineValue (655-755):
 //   - edge points: every mesh edge (the ordered set of vertex pairs of the
 //     faces) against the back (x), left (y) and bottom (z) face planes of the
-//     level-0 nodes in its voxel range widened by one voxel, with the
+//     level-0 nodes in its voxel range, with the
 //     reference's parameter and range tests in binary64;
 //   - face points: every level-0 node edge against every triangle it can
 //     cross: the plane parameter t in [0, 1] and the three edge-side tests of
@@ -13,7 +13,7 @@
 // The reference finds the candidate node edges by sweeps over edges sorted by
 // their end point; a node edge outside a triangle's bounding box cannot pass
 // the edge-side tests, so here every triangle enumerates the lattice edges of
-// its bounding box widened by one voxel instead, and keeps those that are
+// its bounding box instead, and keeps those that are
 // edges of a level-0 node (one of the 4 cells around the lattice edge is a
 // node; the end points come from the node of smallest index).  Point sets
 // are produced by count / scan / emit, so their order is deterministic.
@@ -56,13 +56,22 @@ __device__ inline void cross3(const double* a, const double* b, double* c) {
     c[2] = a[0] * b[1] - a[1] * b[0];
 }
 
+// Candidates reach kSlack voxels beyond the edge's or triangle's own extent.
+// The tests below place a point on the segment or inside the triangle up to
+// binary64 rounding, about 1e-13 voxels, and a triangle passes the plane test
+// only with a height far above that (|n . edge| >= 1e-9), so no candidate
+// farther out can pass.  (One voxel of slack on every side, as the reference
+// sweeps with, gave 46 candidates per mesh edge and 120 per triangle of the
+// knot at R = 256 instead of 4 and 4: 2 x 0.49 and 2 x 1.45 ms.)
+constexpr double kSlack = 1e-3;
+__device__ inline int clamp_cell(double u, int lo, int hi) { return (int)fmin(fmax(u, (double)lo), (double)hi); }
+
 // ---- mesh edges x node faces
 __device__ inline void edge_range(const Fine& S, const double* p1, const double* p2, int lo[3], int hi[3]) {
     for (int a = 0; a < 3; ++a) {
-        const int d1 = (int)((p1[a] - S.o[a]) / S.vw), d2 = (int)((p2[a] - S.o[a]) / S.vw);
-        const int l = min(d1, d2) - 1, h = max(d1, d2) + 1;
-        lo[a] = max(0, min(l, S.R - 1));
-        hi[a] = max(0, min(h, S.R - 1));
+        const double u1 = (p1[a] - S.o[a]) / S.vw, u2 = (p2[a] - S.o[a]) / S.vw;
+        lo[a] = clamp_cell(floor(fmin(u1, u2) - kSlack), 0, S.R - 1);
+        hi[a] = clamp_cell(floor(fmax(u1, u2) + kSlack), 0, S.R - 1);
     }
 }
 __global__ void k_edge_count(int64_t ne, const uint64_t* edges, const double* V, Fine S, uint64_t* cnt) {
@@ -120,30 +129,35 @@ __global__ void k_edge_points(int64_t ne, const uint64_t* edges, const double* V
 }
 
 // ---- node edges x mesh faces
-__device__ inline void tri_range(const Fine& S, const double* T, int lo[3], int hi[3]) {
+// Lattice points and lattice edges (from i to i + 1) that the triangle's box
+// reaches, per axis.
+struct TriRange {
+    int p0[3], np[3];   // points: first, count
+    int e0[3], ne[3];   // edges: first, count
+};
+__device__ inline TriRange tri_range(const Fine& S, const double* T) {
+    TriRange r;
     for (int a = 0; a < 3; ++a) {
         const double mn = fmin(T[a], fmin(T[3 + a], T[6 + a])), mx = fmax(T[a], fmax(T[3 + a], T[6 + a]));
-        lo[a] = max(0, (int)floor((mn - S.o[a]) / S.vw) - 1);
-        hi[a] = min(S.R, (int)floor((mx - S.o[a]) / S.vw) + 1);
-        if (hi[a] < lo[a]) hi[a] = lo[a] - 1;
+        const double lo = (mn - S.o[a]) / S.vw - kSlack, hi = (mx - S.o[a]) / S.vw + kSlack;
+        r.p0[a] = clamp_cell(ceil(lo), 0, S.R + 1);
+        r.np[a] = max(0, clamp_cell(floor(hi), -1, S.R) - r.p0[a] + 1);
+        r.e0[a] = clamp_cell(ceil(lo) - 1.0, 0, S.R);
+        r.ne[a] = max(0, clamp_cell(floor(hi), -1, S.R - 1) - r.e0[a] + 1);
     }
+    return r;
 }
-// lattice edges along axis a in the box: a-extent [lo, hi-1] (edge from i to i+1), others [lo, hi]
-__device__ inline uint64_t tri_cands(const int lo[3], const int hi[3], int a) {
+// lattice edges along axis a
+__device__ inline uint64_t tri_cands(const TriRange& r, int a) {
     uint64_t n = 1;
-    for (int b = 0; b < 3; ++b) {
-        const int64_t len = (b == a) ? (hi[b] - lo[b]) : (hi[b] - lo[b] + 1);
-        if (len <= 0) return 0;
-        n *= (uint64_t)len;
-    }
+    for (int b = 0; b < 3; ++b) n *= (uint64_t)(b == a ? r.ne[b] : r.np[b]);
     return n;
 }
 __global__ void k_face_count(int64_t nT, const double* tris, Fine S, uint64_t* cnt) {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nT) return;
-    int lo[3], hi[3];
-    tri_range(S, tris + 9 * t, lo, hi);
-    cnt[t] = tri_cands(lo, hi, 0) + tri_cands(lo, hi, 1) + tri_cands(lo, hi, 2);
+    const TriRange r = tri_range(S, tris + 9 * t);
+    cnt[t] = tri_cands(r, 0) + tri_cands(r, 1) + tri_cands(r, 2);
 }
 template <int PASS>
 __global__ void k_face_points(int64_t nT, const double* tris, Fine S, const uint64_t* coff, uint64_t total,
@@ -158,21 +172,22 @@ __global__ void k_face_points(int64_t nT, const double* tris, Fine S, const uint
     }
     const int64_t t = lo_t;
     const double* T = tris + 9 * t;
-    int lo[3], hi[3];
-    tri_range(S, T, lo, hi);
+    const TriRange r = tri_range(S, T);
     uint64_t k = c - coff[t];
     int a = 0;
-    for (; a < 3; ++a) {
-        const uint64_t n = tri_cands(lo, hi, a);
+    for (; a < 2; ++a) {
+        const uint64_t n = tri_cands(r, a);
         if (k < n) break;
         k -= n;
     }
-    int len[3];
-    for (int b = 0; b < 3; ++b) len[b] = (b == a) ? (hi[b] - lo[b]) : (hi[b] - lo[b] + 1);
-    int L[3];
-    L[0] = lo[0] + (int)(k % len[0]);
-    L[1] = lo[1] + (int)((k / len[0]) % len[1]);
-    L[2] = lo[2] + (int)(k / ((uint64_t)len[0] * len[1]));
+    int len[3], L[3];
+    for (int b = 0; b < 3; ++b) {
+        len[b] = b == a ? r.ne[b] : r.np[b];
+        L[b] = b == a ? r.e0[b] : r.p0[b];
+    }
+    L[0] += (int)(k % len[0]);
+    L[1] += (int)((k / len[0]) % len[1]);
+    L[2] += (int)(k / ((uint64_t)len[0] * len[1]));
     // the cells around the lattice edge: offsets 0 / -1 in the two other axes
     const int b1 = a == 0 ? 1 : 0, b2 = a == 2 ? 1 : 2;
     int64_t best = -1;
@@ -431,20 +446,110 @@ void shell_points(its_svo s, const double* d_V, const uint64_t* d_edges, int64_t
     *n_face = (int64_t)fcount;
 }
 
-// the ordered set of (min, max) vertex pairs of the faces (BaseModel.cpp:291-313)
-std::vector<uint64_t> mesh_edges(const int32_t* F, int64_t nF) {
-    std::vector<uint64_t> k(3 * (size_t)nF);
-    for (int64_t f = 0; f < nF; ++f) {
-        const int32_t i0 = F[3 * f], i1 = F[3 * f + 1], i2 = F[3 * f + 2];
-        const int32_t mx = std::max(i0, std::max(i1, i2)), mn = std::min(i0, std::min(i1, i2));
-        const int32_t md = i0 + i1 + i2 - mx - mn;
-        k[3 * f] = ((uint64_t)(uint32_t)mn << 32) | (uint32_t)md;
-        k[3 * f + 1] = ((uint64_t)(uint32_t)md << 32) | (uint32_t)mx;
-        k[3 * f + 2] = ((uint64_t)(uint32_t)mn << 32) | (uint32_t)mx;
+namespace {
+// the three vertex pairs of every face, smaller index first, as the sort key
+// smaller << vb | larger
+__global__ void k_face_edges(const int32_t* F, int64_t nF, int vb, uint64_t* keys) {
+    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= nF) return;
+    for (int e = 0; e < 3; ++e) {
+        const uint32_t a = (uint32_t)F[3 * f + e], b = (uint32_t)F[3 * f + (e + 1) % 3];
+        keys[3 * f + e] = ((uint64_t)min(a, b) << vb) | max(a, b);
     }
-    std::sort(k.begin(), k.end());
-    k.erase(std::unique(k.begin(), k.end()), k.end());
-    return k;
+}
+__global__ void k_edge_heads(const uint64_t* keys, int64_t n, uint32_t* head) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) head[i] = (i == 0 || keys[i] != keys[i - 1]) ? 1u : 0u;
+}
+__global__ void k_edge_pick(const uint64_t* keys, const uint32_t* rank, int64_t n, int vb, uint64_t* edges) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n || (i > 0 && keys[i] == keys[i - 1])) return;
+    edges[rank[i]] = ((keys[i] >> vb) << 32) | (keys[i] & ((1ull << vb) - 1ull));
+}
+__global__ void k_face_corners(const double* V, const int32_t* F, int64_t nF, double* tris) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;   // one thread per corner
+    if (i >= 3 * nF) return;
+    const double* v = V + 3 * (int64_t)F[i];
+    for (int a = 0; a < 3; ++a) tris[3 * i + a] = v[a];
+}
+// per block: smallest and largest value and how many are NaN
+__global__ __launch_bounds__(kT) void k_minmax(const float* f, int64_t n, float* part, unsigned* nans) {
+    __shared__ float lo[kT / 64], hi[kT / 64];
+    float a = INFINITY, b = -INFINITY;
+    int bad = 0;
+    for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT) {
+        const float v = f[i];
+        bad += v != v;
+        a = fminf(a, v);
+        b = fmaxf(b, v);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        a = fminf(a, __shfl_xor(a, o, 64));
+        b = fmaxf(b, __shfl_xor(b, o, 64));
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (__ballot(bad != 0) != 0ull && lane == 0) atomicAdd(nans, 1u);
+    if (lane == 0) {
+        lo[w] = a;
+        hi[w] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < kT / 64; ++q) {
+            lo[0] = fminf(lo[0], lo[q]);
+            hi[0] = fmaxf(hi[0], hi[q]);
+        }
+        part[2 * blockIdx.x] = lo[0];
+        part[2 * blockIdx.x + 1] = hi[0];
+    }
+}
+}  // namespace
+
+// The ordered set of (smaller, larger) vertex pairs of the faces
+// (BaseModel.cpp:291-313): keys sorted by the radix sort, one of each kept.
+// 600,000 pairs took 25 ms in a host sort.
+int64_t mesh_edges(const int32_t* d_F, int64_t nF, int64_t nV, DBuf<uint64_t>& edges, hipStream_t st) {
+    const int64_t n = 3 * nF;
+    int vb = 1;
+    while (vb < 32 && ((nV - 1) >> vb) != 0) ++vb;
+    DBuf<uint64_t> keys(n);
+    DBuf<uint32_t> rank(n);
+    hipLaunchKernelGGL(k_face_edges, dim3(blocks_for(nF, kT)), dim3(kT), 0, st, d_F, nF, vb, keys.p);
+    ITS_LAUNCH_CHECK();
+    sort_u64(keys, n, 2 * vb, st);
+    hipLaunchKernelGGL(k_edge_heads, dim3(blocks_for(n, kT)), dim3(kT), 0, st, (const uint64_t*)keys.p, n, rank.p);
+    ITS_LAUNCH_CHECK();
+    const int64_t ne = (int64_t)scan_exclusive_u32(rank.p, rank.p, n, st);
+    edges.alloc(ne);
+    hipLaunchKernelGGL(k_edge_pick, dim3(blocks_for(n, kT)), dim3(kT), 0, st, (const uint64_t*)keys.p,
+                       (const uint32_t*)rank.p, n, vb, edges.p);
+    ITS_LAUNCH_CHECK();
+    return ne;
+}
+void face_corners(const double* d_V, const int32_t* d_F, int64_t nF, double* d_tris, hipStream_t st) {
+    hipLaunchKernelGGL(k_face_corners, dim3(blocks_for(3 * nF, kT)), dim3(kT), 0, st, d_V, d_F, nF, d_tris);
+    ITS_LAUNCH_CHECK();
+}
+
+// smallest and largest of n > 0 values; false when one of them is NaN
+bool value_range(const float* d_f, int64_t n, float range[2], hipStream_t st) {
+    const int64_t nb = std::min<int64_t>(256, blocks_for(n, kT));
+    DBuf<float> part(2 * nb);
+    DBuf<unsigned> nans(1);
+    ITS_HIP(hipMemsetAsync(nans.p, 0, sizeof(unsigned), st));
+    hipLaunchKernelGGL(k_minmax, dim3((unsigned)nb), dim3(kT), 0, st, d_f, n, part.p, nans.p);
+    ITS_LAUNCH_CHECK();
+    std::vector<float> h(2 * nb);
+    ITS_HIP(hipMemcpyAsync(h.data(), part.p, 2 * nb * sizeof(float), hipMemcpyDeviceToHost, st));
+    if (read1(nans.p, st) != 0) return false;
+    range[0] = h[0];
+    range[1] = h[1];
+    for (int64_t b = 1; b < nb; ++b) {
+        range[0] = std::min(range[0], h[2 * b]);
+        range[1] = std::max(range[1], h[2 * b + 1]);
+    }
+    return true;
 }
 
 }  // namespace its

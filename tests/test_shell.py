@@ -119,3 +119,32 @@ def test_gpu_classes_match_oracle(ctx, name, R):
     assert not bad.any()
     assert (cls_r == 0).sum() > 100 and (cls_r == -1).sum() > 100 and (cls_r == 1).sum() > 100
     g.close()
+
+
+def _aligned(kind):
+    """Triangles where candidate ranges can go wrong: every vertex on a
+    lattice point, or thin triangles across many voxels."""
+    rng = np.random.default_rng(5)
+    if kind == "lattice":
+        V = rng.integers(0, 9, size=(60, 3)) / 8.0
+        F = np.array([f for f in rng.integers(0, 60, size=(80, 3)) if len(set(f)) == 3], np.int32)
+        return V, F, np.zeros(3), np.ones(3), 8
+    A, B = rng.uniform(0, 1, (40, 3)), rng.uniform(0, 1, (40, 3))
+    V = np.stack([A, B, (A + B) / 2 + 1e-4 * rng.standard_normal((40, 3))], 1).reshape(-1, 3)
+    return V, np.arange(120, dtype=np.int32).reshape(-1, 3), np.full(3, -0.1), np.full(3, 1.2), 32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["lattice", "thin"])
+def test_gpu_points_at_range_edges(ctx, kind):
+    from its_amd import _capi, meshes
+    V, F, origin, width, R = _aligned(kind)
+    tris = meshes.triangles(V, F)
+    print(f"[shell] {kind} R={R}", flush=True)
+    g = _capi.Octree(ctx, tris, origin, width, R)
+    P, ne = g.shell_points(V, F)
+    Q, qe = O.intersections(O.SVO(tris, origin, width, R), V, F)
+    assert np.array_equal(np.unique(P[:ne], axis=0), np.unique(Q[:qe], axis=0))
+    assert len(P) - ne == len(Q) - qe
+    assert np.abs(_sorted(P[ne:]) - _sorted(Q[qe:])).max() <= 1e-12
+    g.close()
