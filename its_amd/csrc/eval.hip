@@ -46,44 +46,114 @@ namespace its {
 namespace {
 constexpr int kT = 256;
 
-__global__ void k_mark_cells(int64_t nv, int64_t voff, const uint16_t* vx, const uint16_t* vy, const uint16_t* vz,
-                             int R, uint32_t* bits) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nv) return;
-    int64_t v = voff + i;
-    int X = vx[v], Y = vy[v], Z = vz[v];
+// ------------------------------------------------------ field structure ----
+// Levels of the field side by side, finest first.
+struct FieldLevels {
+    int n, lc;                           // levels; collapsed level
+    int R0;                              // cells per axis of the finest level
+    int64_t word[kMaxLevels + 1];        // first word of each level's cell bitset
+    int64_t first[kMaxLevels + 1];       // first cell of each level
+    const RankWord* lattice[kMaxLevels]; // the level's vertices
+    int64_t voff[kMaxLevels];            // first vertex of each level
+};
+__device__ inline int level_of(const int64_t* first, int n, int64_t i) {
+    int d = 0;
+    while (d + 1 < n && i >= first[d + 1]) ++d;
+    return d;
+}
+
+// Marks the 8 cells around every vertex, all levels in one launch.  The cells
+// fall into 2 or 3 words, since a word holds 4 x 4 x 2 cells: one atomic for
+// each word that does not hold them yet (a cell has up to 8 vertices).
+__global__ void k_mark_cells(int64_t nv, const uint16_t* vx, const uint16_t* vy, const uint16_t* vz,
+                             const uint8_t* vlevel, FieldLevels F, RankWord* cells) {
+    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= nv) return;
+    const int d = vlevel[v], R = max(1, F.R0 >> d);
+    RankWord* g = cells + F.word[d];
+    const int X = vx[v], Y = vy[v], Z = vz[v];
+    uint32_t word = 0, bits = 0;
+    auto flush = [&]() {
+        if (bits == 0) return;
+        const uint32_t have = __hip_atomic_load(&g[word].bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((have & bits) != bits) atomicOr(&g[word].bits, bits);
+    };
     for (int k = 0; k < 8; ++k) {
-        int cx = X - (k & 1), cy = Y - ((k >> 1) & 1), cz = Z - ((k >> 2) & 1);
+        const int cx = X - (k & 1), cy = Y - ((k >> 1) & 1), cz = Z - ((k >> 2) & 1);
         if (cx < 0 || cy < 0 || cz < 0 || cx >= R || cy >= R || cz >= R) continue;
-        uint32_t m = morton3(cx, cy, cz);
-        atomicOr(&bits[m >> 5], 1u << (m & 31));
+        const uint32_t m = morton3(cx, cy, cz);
+        if ((m >> 5) != word) {
+            flush();
+            word = m >> 5;
+            bits = 0;
+        }
+        bits |= 1u << (m & 31);
+    }
+    flush();
+}
+
+// first cell of each level, and the total, from the ranks at the level starts
+__global__ void k_level_first(const RankWord* cells, FieldLevels F, const uint32_t* total, uint32_t* first) {
+    const int d = threadIdx.x;
+    if (d < F.n) first[d] = cells[F.word[d]].rank;
+    if (d == F.n) first[d] = *total;
+}
+
+// code of every cell; *orphan = the finest level whose cell has no marked
+// parent (the walk goes down from marked cells only)
+__global__ void k_cell_codes(const RankWord* cells, FieldLevels F, int64_t nwords, uint32_t* code, int* orphan) {
+    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= nwords) return;
+    const RankWord rw = cells[w];
+    if (rw.bits == 0) return;
+    const int d = level_of(F.word, F.n, w);
+    uint32_t b = rw.bits, r = rw.rank;
+    while (b) {
+        const int i = __ffs(b) - 1;
+        b &= b - 1;
+        const uint32_t m = (uint32_t)((w - F.word[d]) * 32 + i);
+        code[r++] = m;
+        if (d + 1 < F.n && !bit_test(cells + F.word[d + 1], m >> 3)) atomicMin(orphan, d);
     }
 }
 
-__global__ void k_pack(const uint32_t* bits, int64_t nwords, RankWord* g) {
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w < nwords) g[w] = RankWord{bits[w], 0u};
+// Child link of the cell with Morton code m, from the bitset of the level
+// below: the children's bits are one byte of one word.  Corner k carries mask
+// bit k and bits 4k .. 4k + 3 of the first child's index in the 5 low bits of
+// its value, which is first rounded to the nearest multiple of 32 ulps
+// (halves away from zero).
+__device__ inline float with_link(float v, const RankWord* below, uint32_t m, int k) {
+    const RankWord w = below[m >> 2];
+    const int sh = 8 * (int)(m & 3u);
+    const uint32_t mask = (w.bits >> sh) & 255u;
+    const uint32_t base = w.rank + __popc(w.bits & ((1u << sh) - 1u));
+    return __uint_as_float(((__float_as_uint(v) + 16u) & ~31u) | ((mask >> k) & 1u) | (((base >> (4 * k)) & 15u) << 1));
 }
 
-__global__ void k_fill_blocks(int64_t nv, int64_t voff, const uint16_t* vx, const uint16_t* vy, const uint16_t* vz,
-                              int R, const RankWord* cells, const double* lambda, float* blocks) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nv) return;
-    int64_t v = voff + i;
-    int X = vx[v], Y = vy[v], Z = vz[v];
-    float lam = (float)lambda[v];
-    for (int k = 0; k < 8; ++k) {
-        int a = k & 1, b = (k >> 1) & 1, c = (k >> 2) & 1;
-        int cx = X - a, cy = Y - b, cz = Z - c;
-        if (cx < 0 || cy < 0 || cz < 0 || cx >= R || cy >= R || cz >= R) continue;
-        uint32_t idx = bit_rank(cells, morton3(cx, cy, cz));
-        blocks[8 * (int64_t)idx + k] = lam;   // vertex sits at corner (a,b,c) of the cell
-    }
+// Corner values of every cell, one thread per (cell, corner): the cell's
+// vertices are looked up in the level's lattice, so the blocks are written
+// once, whole lines at a time, links included.
+__global__ void k_fill_blocks(int64_t n, FieldLevels F, const RankWord* cells, const uint32_t* code,
+                              const double* lambda, float* blocks) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    const int64_t i = t >> 3;
+    const int k = (int)(t & 7);
+    const int d = level_of(F.first, F.n, i);
+    const uint32_t m = code[i];
+    uint32_t x, y, z;
+    demorton3(m, x, y, z);
+    const uint32_t D = (uint32_t)max(1, F.R0 >> d) + 1u;
+    const uint32_t key = ((x + (k & 1)) * D + (y + ((k >> 1) & 1))) * D + (z + ((k >> 2) & 1));
+    const uint32_t r = bit_find(F.lattice[d], key);
+    float v = r != ITS_NONE ? (float)lambda[F.voff[d] + r] : 0.f;
+    if (d > 0 && d < F.lc) v = with_link(v, cells + F.word[d - 1], m, k);
+    blocks[t] = v;
 }
 
 struct EvalParams {
     const RankWord* cells[kMaxLevels];
-    const float4* blocks[kMaxLevels];
+    const float4* blocks;              // of all levels: cell indices count over the levels
     const float4* G;                   // per level-lc cell: 8 corner values of levels >= lc
     int L;
     int R;
@@ -247,7 +317,7 @@ __device__ float eval_walk(const EvalParams& P, float ux, float uy, float uz, in
         if (!(w.bits & bit)) break;
         const uint32_t idx = w.rank + __popc(w.bits & (bit - 1u));
         const float s = pow2neg(d);
-        float4 b0 = P.blocks[d][2 * idx], b1 = P.blocks[d][2 * idx + 1];
+        float4 b0 = P.blocks[2 * idx], b1 = P.blocks[2 * idx + 1];
         if (d > 0 && d < P.lc) {   // linked level: drop the link payload
             b0 = link_clear(b0);
             b1 = link_clear(b1);
@@ -360,8 +430,8 @@ __global__ __launch_bounds__(kT) void k_eval(Loader load, int64_t N, EvalParams 
 #pragma unroll
             for (int j = 0; j < K; ++j) {
                 if (!act[j]) continue;
-                b0[j] = P.blocks[d][2 * (size_t)idx[j]];
-                b1[j] = P.blocks[d][2 * (size_t)idx[j] + 1];
+                b0[j] = P.blocks[2 * (size_t)idx[j]];
+                b1[j] = P.blocks[2 * (size_t)idx[j] + 1];
             }
             const float s = pow2neg(d);
             more = false;
@@ -410,8 +480,8 @@ __device__ inline float eval_query(const Loader& load, const EvalParams& P, int6
     if (!((mask >> key) & 1u)) return f;
     uint32_t idx = child_index(base, mask, key);
     for (int d = lc - 1; d >= 0; --d) {
-        b0 = P.blocks[d][2 * (size_t)idx];
-        b1 = P.blocks[d][2 * (size_t)idx + 1];
+        b0 = P.blocks[2 * (size_t)idx];
+        b1 = P.blocks[2 * (size_t)idx + 1];
         if (d == 0) return f + tri_level(b0, b1, ux, uy, uz, pow2neg(d));
         mask = link_decode(b0, b1, base);
         f += tri_level(b0, b1, ux, uy, uz, pow2neg(d));
@@ -487,8 +557,8 @@ __device__ inline float fine_walk(const EvalParams& P, float ux, float uy, float
     const uint32_t mask = link_unpack(lk, base);
     uint32_t idx = child_index(base, mask, child_key(cx, cy, cz, P.lc - 1));
     for (int d = P.lc - 1; d >= 0; --d) {
-        float4 b0 = P.blocks[d][2 * (size_t)idx];
-        float4 b1 = P.blocks[d][2 * (size_t)idx + 1];
+        float4 b0 = P.blocks[2 * (size_t)idx];
+        float4 b1 = P.blocks[2 * (size_t)idx + 1];
         if (d == 0) return f + tri_level(b0, b1, ux, uy, uz, pow2neg(d));
         uint32_t nbase;
         const uint32_t m = link_decode(b0, b1, nbase);
@@ -731,67 +801,19 @@ __global__ __launch_bounds__(kTopThreads) void k_dense_top(TopLevels T, const do
     }
 }
 
-// lattice values (x fastest, D = Rc + 1 per axis) -> one 64-byte block per
-// cell: 8 corner values (index x | y<<1 | z<<2), child base, child mask
-__global__ void k_cell_blocks(int Rc, const float* lat, float* blocks) {
-    const int64_t n = (int64_t)Rc * Rc * Rc;
+// lattice values (x fastest, D = Rc + 1 per axis) -> 8 corner values per cell
+// (index x | y<<1 | z<<2), one thread per (cell, corner); below != null:
+// with the child links into the level below
+__global__ void k_cell_blocks(int Rc, const float* lat, const RankWord* below, float* blocks) {
+    const int64_t n = 8 * (int64_t)Rc * Rc * Rc;
     const int64_t D = Rc + 1;
-    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += (int64_t)gridDim.x * blockDim.x) {
-        int64_t x = c % Rc, y = (c / Rc) % Rc, z = c / ((int64_t)Rc * Rc);
-        float* o = blocks + 8 * c;
-        for (int k = 0; k < 8; ++k)
-            o[k] = lat[((z + ((k >> 2) & 1)) * D + (y + ((k >> 1) & 1))) * D + (x + (k & 1))];
-    }
-}
-
-// every marked cell of the child level links into its parent's link word:
-// the smallest child index and the bit of its key (marked cells only have
-// marked parents, so the parent entry exists)
-__global__ void k_link(int64_t n, const uint32_t* codes, const RankWord* parent_cells, int parent_dense_R,
-                       uint2* parent_link, int* err) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t c = codes[i], p = c >> 3;
-    uint32_t slot;
-    if (parent_dense_R > 0) {
-        uint32_t x, y, z;
-        demorton3(p, x, y, z);
-        slot = (z * (uint32_t)parent_dense_R + y) * (uint32_t)parent_dense_R + x;
-    } else {
-        slot = bit_find(parent_cells, p);
-        if (slot == ITS_NONE) { atomicOr(err, 1); return; }
-    }
-    atomicMin(&parent_link[slot].x, (uint32_t)i);
-    atomicOr(&parent_link[slot].y, 1u << (c & 7));
-}
-
-// link words before linking: no child
-__global__ void k_link_clear(int64_t n, uint2* link) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        link[i] = make_uint2(ITS_NONE, 0u);
-}
-
-// link word of each cell into the 5 low bits of its 8 corner values (value
-// rounded to the nearest multiple of 32 ulps first, halves away from zero)
-__global__ void k_embed_link(int64_t n, const uint2* link, uint32_t* blocks) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint2 L = link[i];
-        for (int k = 0; k < 8; ++k) {
-            const uint32_t u = (blocks[8 * i + k] + 16u) & ~31u;
-            blocks[8 * i + k] = u | ((L.y >> k) & 1u) | (((L.x >> (4 * k)) & 15u) << 1);
-        }
-    }
-}
-
-__global__ void k_emit_codes(const RankWord* g, int64_t nwords, uint32_t* out) {
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nwords) return;
-    RankWord rw = g[w];
-    uint32_t b = rw.bits, r = rw.rank;
-    while (b) {
-        int i = __ffs(b) - 1;
-        out[r++] = (uint32_t)(w * 32 + i);
-        b &= b - 1;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t c = t >> 3;
+        const int k = (int)(t & 7);
+        const int64_t x = c % Rc, y = (c / Rc) % Rc, z = c / ((int64_t)Rc * Rc);
+        float v = lat[((z + ((k >> 2) & 1)) * D + (y + ((k >> 1) & 1))) * D + (x + (k & 1))];
+        if (below) v = with_link(v, below, morton3((uint32_t)x, (uint32_t)y, (uint32_t)z), k);
+        blocks[t] = v;
     }
 }
 
@@ -799,9 +821,9 @@ EvalParams make_params(its_svo s, const double box_end[3], int mode, float out_v
     ITS_REQUIRE(s->field_ready, ITS_E_STATE, "no coefficient field: run a fit or set lambda first");
     EvalParams P{};
     for (int d = 0; d < s->depth; ++d) {
-        P.cells[d] = s->lv[d].cells.p;
-        P.blocks[d] = s->lv[d].blocks.p;
+        P.cells[d] = s->cells.p + s->cell_word[d];
     }
+    P.blocks = s->blocks.p;
     P.G = s->dense_blocks.p;
     P.L = s->depth;
     P.R = s->R;
@@ -868,87 +890,94 @@ void launch_eval(Loader ld, its_svo s, int64_t N, const EvalParams& P, float* ou
 }
 }  // namespace
 
+namespace {
+FieldLevels field_levels(its_svo s, int lc) {
+    FieldLevels F{};
+    F.n = s->depth;
+    F.lc = lc;
+    F.R0 = s->R;
+    for (int d = 0; d < s->depth; ++d) {
+        F.lattice[d] = s->lv[d].lattice.p;
+        F.voff[d] = s->esum_verts[d];
+    }
+    for (int d = 0; d <= s->depth; ++d) {
+        F.word[d] = s->cell_word[d];
+        F.first[d] = s->cell_first[d];
+    }
+    return F;
+}
+
+// The marked cells of all levels, once per octree: one launch each for the
+// marks, the ranks' scan and the codes, one read-back.  (Level by level, with
+// an atomic per vertex and cell, a read-back per level and the child links
+// built by atomics, a field of the knot at R = 256 took 0.62 ms, on every
+// change of the coefficients.)
+void cells_build(its_svo s, hipStream_t st) {
+    int64_t words = 0;
+    for (int d = 0; d < s->depth; ++d) {
+        const int64_t R = s->lv[d].R;
+        s->cell_word[d] = words;
+        words += std::max<int64_t>(1, (R * R * R + 31) / 32);
+    }
+    s->cell_word[s->depth] = words;
+    s->cells.ensure(words);
+    ITS_HIP(hipMemsetAsync(s->cells.p, 0, words * sizeof(RankWord), st));
+    FieldLevels F = field_levels(s, 0);
+    hipLaunchKernelGGL(k_mark_cells, dim3(blocks_for(s->num_verts, kT)), dim3(kT), 0, st, s->num_verts, s->vx.p, s->vy.p,
+                       s->vz.p, s->vlevel.p, F, s->cells.p);
+    ITS_LAUNCH_CHECK();
+    DBuf<uint32_t> first(s->depth + 2);
+    uint32_t* total = first.p + s->depth + 1;
+    rank_build_async(s->cells.p, words, st, total);
+    hipLaunchKernelGGL(k_level_first, dim3(1), dim3(64), 0, st, s->cells.p, F, (const uint32_t*)total, first.p);
+    ITS_LAUNCH_CHECK();
+    std::vector<uint32_t> h;
+    to_host(h, first.p, s->depth + 1, st);
+    for (int d = 0; d <= s->depth; ++d) s->cell_first[d] = (int64_t)h[d];
+    const int64_t n = s->cell_first[s->depth];
+    s->cell_code.ensure(std::max<int64_t>(n, 1));
+    s->blocks.ensure(std::max<int64_t>(2 * n, 2));
+    DBuf<int> orphan(1);
+    ITS_HIP(hipMemsetAsync(orphan.p, 0x7f, sizeof(int), st));
+    F = field_levels(s, 0);
+    hipLaunchKernelGGL(k_cell_codes, dim3(blocks_for(words, kT)), dim3(kT), 0, st, (const RankWord*)s->cells.p, F, words,
+                       s->cell_code.p, orphan.p);
+    ITS_LAUNCH_CHECK();
+    s->orphan_level = read1(orphan.p, st);
+    s->cells_ready = true;
+}
+}  // namespace
+
 void field_build(its_svo s) {
     lambda_changing(s);
     ITS_REQUIRE(s->has_lambda, ITS_E_STATE, "no coefficients");
     ITS_REQUIRE(s->depth > 0, ITS_E_STATE, "empty octree");
     hipStream_t st = s->ctx->stream;
-    for (int d = 0; d < s->depth; ++d) {
-        Level& L = s->lv[d];
-        const int R = L.R;
-        const int64_t ncell = (int64_t)R * R * R;
-        const int64_t nwords = std::max<int64_t>(1, (ncell + 31) / 32);
-        DBuf<uint32_t> bits(nwords);
-        ITS_HIP(hipMemsetAsync(bits.p, 0, bits.bytes(), st));
-        hipLaunchKernelGGL(k_mark_cells, dim3(blocks_for(L.n_verts, kT)), dim3(kT), 0, st, L.n_verts, s->esum_verts[d],
-                           s->vx.p, s->vy.p, s->vz.p, R, bits.p);
-        ITS_LAUNCH_CHECK();
-        L.cells.ensure(nwords);
-        hipLaunchKernelGGL(k_pack, dim3(blocks_for(nwords, kT)), dim3(kT), 0, st, bits.p, nwords, L.cells.p);
-        ITS_LAUNCH_CHECK();
-        L.n_cells = (int64_t)rank_build(L.cells.p, nwords, st);
-        L.blocks.ensure(std::max<int64_t>(2 * L.n_cells, 2));
-        ITS_HIP(hipMemsetAsync(L.blocks.p, 0, 2 * L.n_cells * sizeof(float4), st));
-        hipLaunchKernelGGL(k_fill_blocks, dim3(blocks_for(L.n_verts, kT)), dim3(kT), 0, st, L.n_verts,
-                           s->esum_verts[d], s->vx.p, s->vy.p, s->vz.p, R, L.cells.p, s->lambda64.p,
-                           (float*)L.blocks.p);
-        ITS_LAUNCH_CHECK();
-    }
-    // dense cascade from the root level down to the collapsed level
+    if (!s->cells_ready) cells_build(s, st);
+    // the collapsed level: the finest with at most that many cells
     int lc = 0;
     const int64_t max_cells = tune_get(ITS_TUNE_DENSE_CELLS);
     while (lc < s->depth - 1 && (int64_t)s->lv[lc].R * s->lv[lc].R * s->lv[lc].R > max_cells) ++lc;
     s->dense_level = lc;
-    {
-        DBuf<float> lat;
-        dense_cascade(s, lc, lat);
-        const int Rc = s->lv[lc].R;
-        const int64_t nc = (int64_t)Rc * Rc * Rc;
-        s->dense_blocks.ensure(2 * nc);
-        hipLaunchKernelGGL(k_cell_blocks, dim3((unsigned)std::min<int64_t>(blocks_for(nc, kT), 65536)), dim3(kT), 0, st,
-                           Rc, lat.p, (float*)s->dense_blocks.p);
+    ITS_REQUIRE(s->orphan_level + 1 >= lc, ITS_E_STATE, "marked cell without a marked parent");
+    const int64_t n = 8 * s->cell_first[s->depth];
+    if (n > 0) {
+        hipLaunchKernelGGL(k_fill_blocks, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, field_levels(s, lc),
+                           (const RankWord*)s->cells.p, (const uint32_t*)s->cell_code.p, (const double*)s->lambda64.p,
+                           (float*)s->blocks.p);
         ITS_LAUNCH_CHECK();
     }
-    if (lc == 0) {   // no linked levels: the values stay exact
-        ITS_HIP(hipStreamSynchronize(st));
-        s->field_ready = true;
-        return;
-    }
-    // child links of every level above the finest, down to the collapsed one:
-    // a link word (first marked child, child mask) per cell, then folded into
-    // the cell's block
-    const int64_t nc_dense = (int64_t)s->lv[lc].R * s->lv[lc].R * s->lv[lc].R;
-    std::vector<DBuf<uint2>> links(lc + 1);
-    for (int d = 1; d <= lc; ++d) {
-        const int64_t m = d == lc ? nc_dense : std::max<int64_t>(s->lv[d].n_cells, 1);
-        links[d].alloc(m);
-        hipLaunchKernelGGL(k_link_clear, dim3((unsigned)std::min<int64_t>(blocks_for(m, kT), 65536)), dim3(kT), 0, st,
-                           m, links[d].p);
-        ITS_LAUNCH_CHECK();
-    }
-    DBuf<int> err(1);
-    ITS_HIP(hipMemsetAsync(err.p, 0, sizeof(int), st));
-    for (int d = 0; d < lc; ++d) {   // link the marked cells of level d into level d+1
-        Level& L = s->lv[d];
-        const int64_t nwords = std::max<int64_t>(1, ((int64_t)L.R * L.R * L.R + 31) / 32);
-        DBuf<uint32_t> codes(std::max<int64_t>(L.n_cells, 1));
-        hipLaunchKernelGGL(k_emit_codes, dim3(blocks_for(nwords, kT)), dim3(kT), 0, st, L.cells.p, nwords, codes.p);
-        ITS_LAUNCH_CHECK();
-        const bool dense_parent = (d + 1 == lc);
-        hipLaunchKernelGGL(k_link, dim3(blocks_for(L.n_cells, kT)), dim3(kT), 0, st, L.n_cells, codes.p,
-                           s->lv[d + 1].cells.p, dense_parent ? s->lv[lc].R : 0, links[d + 1].p, err.p);
-        ITS_LAUNCH_CHECK();
-        ITS_HIP(hipStreamSynchronize(st));
-    }
-    ITS_REQUIRE(read1(err.p, st) == 0, ITS_E_STATE, "marked cell without a marked parent");
-    for (int d = 1; d <= lc; ++d) {
-        const int64_t m = d == lc ? nc_dense : s->lv[d].n_cells;
-        if (m == 0) continue;
-        uint32_t* blocks = (uint32_t*)(d == lc ? s->dense_blocks.p : s->lv[d].blocks.p);
-        hipLaunchKernelGGL(k_embed_link, dim3((unsigned)std::min<int64_t>(blocks_for(m, kT), 65536)), dim3(kT), 0, st,
-                           m, (const uint2*)links[d].p, blocks);
-        ITS_LAUNCH_CHECK();
-    }
+    // dense cascade from the root level down to the collapsed level; at level
+    // 0 there is nothing to link and the values stay exact
+    DBuf<float> lat;
+    dense_cascade(s, lc, lat);
+    const int Rc = s->lv[lc].R;
+    const int64_t nc = (int64_t)Rc * Rc * Rc;
+    s->dense_blocks.ensure(2 * nc);
+    hipLaunchKernelGGL(k_cell_blocks, dim3((unsigned)std::min<int64_t>(blocks_for(8 * nc, kT), 65536)), dim3(kT), 0, st,
+                       Rc, (const float*)lat.p, lc > 0 ? (const RankWord*)s->cells.p + s->cell_word[lc - 1] : nullptr,
+                       (float*)s->dense_blocks.p);
+    ITS_LAUNCH_CHECK();
     ITS_HIP(hipStreamSynchronize(st));
     s->field_ready = true;
 }

@@ -19,11 +19,6 @@ struct Level {
     DBuf<uint32_t> occ;     // occupied cell codes, ascending
     DBuf<uint32_t> prank;   // rank of each occupied cell's parent among the parents
     DBuf<RankWord> lattice; // corner lattice (R+1)^3 bits, index (x*(R+1)+y)*(R+1)+z
-    // evaluation field: cells whose corners include a vertex
-    DBuf<RankWord> cells;   // R^3 bits by Morton code
-    DBuf<float4> blocks;    // 2 float4 (8 corner coefficients) per marked cell; on the
-                            // linked levels the 5 low bits of each carry the child link
-    int64_t n_cells = 0;
 };
 
 struct Fit;   // matrix-free collocation operator and solver state (lscg.hip)
@@ -76,6 +71,17 @@ struct its_svo_s {
     its::DBuf<double> lambda64;
     bool has_lambda = false;
     bool field_ready = false;
+    // evaluation field: the cells whose corners include a vertex, all levels
+    // in one array, finest first.  The cells depend on the vertices alone and
+    // stay; their blocks follow the coefficients.
+    bool cells_ready = false;
+    int64_t cell_word[its::kMaxLevels + 1] = {0};    // first bitset word of each level (R^3 bits by Morton code)
+    int64_t cell_first[its::kMaxLevels + 1] = {0};   // first cell of each level
+    int orphan_level = its::kMaxLevels;              // finest level with a marked cell under an unmarked one
+    its::DBuf<its::RankWord> cells;                    // bits and ranks, counted over all levels
+    its::DBuf<uint32_t> cell_code;                   // Morton code within its level
+    its::DBuf<float4> blocks;                        // 2 float4 (8 corner coefficients) per cell; on the linked
+                                                     // levels the 5 low bits of each carry the child link
     its::DBuf<float4> dense_blocks;   // per dense_level cell: corner values of levels >= dense_level,
                                       // child link in the 5 low bits of each
     int dense_level = 0;
