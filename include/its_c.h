@@ -287,8 +287,9 @@ int its_lscg_solve_mlp(its_ctx ctx, its_svo svo, its_mlp net, const double* b, d
 /* ---- many meshes per launch (no reference counterpart: the reference fits
  *      one model per process) ----
  * A batch holds octrees, each with its right-hand side
- * (its_sdf_at_vertices).  its_batch_fit solves the meshes with at most
- * ITS_TUNE_BATCH_MAX_VERTS unknowns in one persistent launch (one workgroup
+ * (its_sdf_at_vertices).  its_batch_fit solves small meshes (at most
+ * ITS_TUNE_BATCH_MAX_VERTS unknowns, and among those the ones that would not
+ * hold the others up) in one persistent launch (one workgroup
  * per mesh runs that mesh's whole mixed-precision LSCG, the algorithm and
  * stopping rule of its_lscg_solve), captured once as a hipGraph and replayed
  * on later calls; the larger meshes run at the same time through the
@@ -345,7 +346,7 @@ int its_batch_eval_device_noalloc(its_batch b, const float* d_x, const float* d_
  *   gathered per wavefront in LDS and walked 64 at a time; 0 = every thread
  *   walks its own query (default 1).
  * ITS_TUNE_BATCH_MAX_VERTS: meshes of a batch with at most this many
- *   unknowns share the one-launch fit (default 65536).
+ *   unknowns may share the one-launch fit (default 65536).
  * ITS_TUNE_SDF_RAY: 1 = for a closed, consistently oriented mesh the sign of
  *   the signed distance comes from the crossings of a ray where exact
  *   orientation tests decide it (the winding-number fan sum for the other
