@@ -386,7 +386,7 @@ int its_svo_export_voxels(its_svo s, uint32_t* morton) {
     DeviceGuard g(s->ctx->device);
     AllocStream as(s->ctx->stream);
     if (s->num_voxels && morton) {
-        ITS_HIP(hipMemcpyAsync(morton, s->lv[0].occ.p, s->num_voxels * sizeof(uint32_t), hipMemcpyDeviceToHost,
+        ITS_HIP(hipMemcpyAsync(morton, s->occ_codes.p, s->num_voxels * sizeof(uint32_t), hipMemcpyDeviceToHost,
                                s->ctx->stream));
         ITS_HIP(hipStreamSynchronize(s->ctx->stream));
     }

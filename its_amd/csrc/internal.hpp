@@ -12,13 +12,12 @@ constexpr int kMaxLevels = ITS_MAX_LEVELS;
 // One octree level (0 = finest voxels).
 struct Level {
     int64_t n_nodes = 0;    // nodes (octets of children of occupied parents)
-    int64_t n_occ = 0;      // occupied cells (sorted Morton codes)
+    int64_t n_occ = 0;      // occupied cells
     int64_t n_verts = 0;    // distinct node corners
     int R = 1;              // cells per axis at this level
     double width = 0;       // node width
-    DBuf<uint32_t> occ;     // occupied cell codes, ascending
-    DBuf<uint32_t> prank;   // rank of each occupied cell's parent among the parents
-    DBuf<RankWord> lattice; // corner lattice (R+1)^3 bits, index (x*(R+1)+y)*(R+1)+z
+    struct { RankWord* p = nullptr; } lattice;   // corner lattice (R+1)^3 bits, index (x*(R+1)+y)*(R+1)+z;
+                                                 // part of the octree's lattice array
 };
 
 struct Fit;   // matrix-free collocation operator and solver state (lscg.hip)
@@ -54,9 +53,11 @@ struct its_svo_s {
     its::Level lv[its::kMaxLevels];
 
     // nodes, global order finest -> root
-    its::DBuf<uint32_t> morton, parent, childbase, neighbors, node_corner;
+    its::DBuf<uint32_t> morton, parent, childbase, neighbors;
     its::DBuf<uint8_t> is_leaf;
     its::DBuf<double> node_origin, node_width;
+    its::DBuf<uint32_t> occ_codes;   // occupied cells of every level, ascending codes, finest level first
+    its::DBuf<its::RankWord> lattice;   // the levels' corner lattices, finest first
     // vertices, global order level by level, lexicographic within a level
     its::DBuf<double> vxyz;
     its::DBuf<uint32_t> vowner;

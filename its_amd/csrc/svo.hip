@@ -16,8 +16,6 @@
 #include <algorithm>
 #include <cmath>
 
-#include <mutex>
-
 #include "internal.hpp"
 
 namespace its {
@@ -44,7 +42,7 @@ __device__ inline void tri_box(const double* t, const Grid& g, int bo[3], int be
         double lo = dmin(v0, dmin(v1, v2)), hi = dmax(v0, dmax(v1, v2));
         int l = (int)(lo / g.unit[a]), h = (int)(hi / g.unit[a]);
         bo[a] = max(0, min(l, g.R - 1));
-        be[a] = max(0, min(h, g.R - 1));
+        be[a] = max(bo[a], min(h, g.R - 1));   // never empty: a triangle has a candidate
     }
 }
 
@@ -56,22 +54,46 @@ __global__ void k_tri_count(const double* tris, int64_t T, Grid g, uint64_t* cnt
     cnt[t] = (uint64_t)(be[0] - bo[0] + 1) * (uint64_t)(be[1] - bo[1] + 1) * (uint64_t)(be[2] - bo[2] + 1);
 }
 
-// one thread per (triangle, candidate voxel); the triangle set-up is
-// recomputed per candidate, in the reference's expression order
-__global__ void k_voxelize(const double* tris, int64_t T, const uint64_t* off, uint64_t total, Grid g,
-                           uint32_t* bits) {
-    for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < total;
-         c += (uint64_t)gridDim.x * blockDim.x) {
-        int64_t lo = 0, hi = T - 1;   // last t with off[t] <= c
-        while (lo < hi) {
-            int64_t mid = (lo + hi + 1) >> 1;
-            if (off[mid] <= c) lo = mid;
-            else hi = mid - 1;
+// One thread per (triangle, candidate voxel); the triangle set-up is
+// recomputed per candidate, in the reference's expression order.  A block's
+// 256 candidates belong to at most 256 consecutive triangles, since every
+// triangle has one: the block finds the range once and each thread searches
+// its part of the offsets in LDS (18 dependent global reads a thread before:
+// 108 us for 200,000 triangles at R = 256).
+__global__ __launch_bounds__(kT) void k_voxelize(const double* tris, int64_t T, const uint64_t* off, uint64_t total,
+                                                 Grid g, RankWord* occ) {
+    __shared__ uint64_t s_off[kT + 1];
+    __shared__ int64_t s_t[2];
+    for (uint64_t c0 = (uint64_t)blockIdx.x * kT; c0 < total; c0 += (uint64_t)gridDim.x * kT) {
+        __syncthreads();
+        if (threadIdx.x < 2) {   // last t with off[t] <= the block's first / last candidate
+            const uint64_t c = threadIdx.x == 0 ? c0 : min(c0 + kT, total) - 1;
+            int64_t lo = 0, hi = T - 1;
+            while (lo < hi) {
+                const int64_t mid = (lo + hi + 1) >> 1;
+                if (off[mid] <= c) lo = mid;
+                else hi = mid - 1;
+            }
+            s_t[threadIdx.x] = lo;
         }
+        __syncthreads();
+        const int64_t t0 = s_t[0];
+        const int nt = (int)(s_t[1] - t0) + 1;
+        for (int q = threadIdx.x; q < nt; q += kT) s_off[q] = off[t0 + q];
+        __syncthreads();
+        const uint64_t c = c0 + threadIdx.x;
+        if (c >= total) continue;
+        int lq = 0, hq = nt - 1;
+        while (lq < hq) {
+            const int mid = (lq + hq + 1) >> 1;
+            if (s_off[mid] <= c) lq = mid;
+            else hq = mid - 1;
+        }
+        const int64_t lo = t0 + lq;
         const double* tri = tris + 9 * lo;
         int bo[3], be[3];
         tri_box(tri, g, bo, be);
-        uint64_t local = c - off[lo];
+        uint64_t local = c - s_off[lq];
         uint64_t nx = be[0] - bo[0] + 1, ny = be[1] - bo[1] + 1;
         int x = bo[0] + (int)(local % nx);
         int y = bo[1] + (int)((local / nx) % ny);
@@ -136,47 +158,100 @@ __global__ void k_voxelize(const double* tris, int64_t T, const uint64_t* off, u
         }
         if (!ok) continue;
         uint32_t m = morton3((uint32_t)x, (uint32_t)y, (uint32_t)z);
-        atomicOr(&bits[m >> 5], 1u << (m & 31));
+        const uint32_t bit = 1u << (m & 31);
+        if (!(__hip_atomic_load(&occ[m >> 5].bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit))
+            atomicOr(&occ[m >> 5].bits, bit);
     }
 }
 
-// set bits of a RankWord bitset -> their indices, ascending
-__global__ void k_emit_bits(const RankWord* g, int64_t nwords, uint32_t* out) {
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nwords) return;
-    RankWord rw = g[w];
+// --------------------------------------------------------------- levels ----
+// All levels side by side, finest first: every kernel below takes the nodes,
+// cells or vertices of all levels in one launch, since most levels are far
+// too small to fill the chip or even a launch.
+//
+// The occupied cells are a pyramid of Morton bitsets.  A node is a child of
+// an occupied cell, and the children of the cell of rank r sit at 8r .. 8r+7
+// of their level, so a node's index, its parent, its children and its 27
+// neighbours are each one bit and rank of the level above or its own.
+struct Tree {
+    int top;                          // levels of the pyramid
+    int depth;                        // levels up to the root
+    int R0;
+    double go[3];
+    double width[kMaxLevels];
+    int64_t word[kMaxLevels + 1];     // first word of each level's occupancy
+    int64_t first[kMaxLevels + 1];    // first occupied cell of each level (ranks count over the levels)
+    int64_t node[kMaxLevels + 1];     // first node of each level
+    int64_t lat[kMaxLevels + 1];      // first word of each level's corner lattice
+    int64_t vert[kMaxLevels + 1];     // first vertex of each level
+};
+__device__ inline int level_of(const int64_t* first, int n, int64_t i) {
+    int d = 0;
+    while (d + 1 < n && i >= first[d + 1]) ++d;
+    return d;
+}
+
+// parents' bits from the children's: a parent is one byte of its level below
+__device__ inline uint32_t parent_bits(const RankWord* child, int64_t nchild, int64_t w) {
+    uint32_t bits = 0;
+    for (int q = 0; q < 8; ++q) {
+        const uint32_t b = 8 * w + q < nchild ? child[8 * w + q].bits : 0u;
+        for (int y = 0; y < 4; ++y)
+            if ((b >> (8 * y)) & 255u) bits |= 1u << (4 * q + y);
+    }
+    return bits;
+}
+__global__ void k_occ_up(const RankWord* child, int64_t nchild, RankWord* up, int64_t nup) {
+    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w < nup) up[w].bits = parent_bits(child, nchild, w);
+}
+// the upper levels in one workgroup
+constexpr int kOccTopThreads = 1024;
+__global__ __launch_bounds__(kOccTopThreads) void k_occ_top(Tree T, int from, RankWord* occ) {
+    for (int d = from; d + 1 < T.top; ++d) {
+        const int64_t nup = T.word[d + 2] - T.word[d + 1];
+        for (int64_t w = threadIdx.x; w < nup; w += kOccTopThreads)
+            occ[T.word[d + 1] + w].bits = parent_bits(occ + T.word[d], T.word[d + 1] - T.word[d], w);
+        __threadfence_block();
+        __syncthreads();
+    }
+}
+
+// ranks at the starts of n consecutive bitsets, and the total
+struct Starts {
+    int n;
+    int64_t word[kMaxLevels + 1];
+};
+__global__ void k_level_first(const RankWord* g, Starts S, const uint32_t* total, uint32_t* first) {
+    const int d = threadIdx.x;
+    if (d < S.n) first[d] = g[S.word[d]].rank;
+    if (d == S.n) first[d] = *total;
+}
+
+// codes of the occupied cells, by rank
+__global__ void k_occ_codes(const RankWord* occ, Tree T, uint32_t* codes) {
+    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= T.word[T.top]) return;
+    const RankWord rw = occ[w];
+    if (rw.bits == 0) return;
+    const uint32_t base = (uint32_t)(w - T.word[level_of(T.word, T.top, w)]) * 32u;
     uint32_t b = rw.bits, r = rw.rank;
     while (b) {
-        int i = __ffs(b) - 1;
-        out[r++] = (uint32_t)(w * 32 + i);
+        codes[r++] = base + (uint32_t)(__ffs(b) - 1);
         b &= b - 1;
     }
 }
 
-// bits (uint32 words) -> RankWord array (rank filled later)
-__global__ void k_pack_bits(const uint32_t* bits, int64_t nwords, RankWord* g) {
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w < nwords) g[w] = RankWord{bits[w], 0u};
+// rank of the occupied cell m of level d within its level, or ITS_NONE
+__device__ inline uint32_t occ_rank(const Tree& T, const RankWord* occ, int d, uint32_t m) {
+    const uint32_t r = bit_find(occ + T.word[d], m);
+    return r == ITS_NONE ? ITS_NONE : r - (uint32_t)T.first[d];
 }
-
-// ------------------------------------------------------------ levels -------
-// The level loop launches over a bound of the level's cell count; the count
-// itself (*cnt) is in device memory.  Entries from the count to the bound
-// are zero, so the scan over the bound gives the parents' count.
-__global__ void k_heads(const uint32_t* occ, const uint32_t* cnt, int64_t bound, uint32_t* head) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= bound) return;
-    const int64_t n = *cnt;
-    head[i] = (i < n && (i == 0 || (occ[i] >> 3) != (occ[i - 1] >> 3))) ? 1u : 0u;
-}
-__global__ void k_parents(const uint32_t* occ, const uint32_t* cnt, int64_t bound, uint32_t* prank,
-                          uint32_t* parents) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= bound || i >= (int64_t)*cnt) return;
-    uint32_t h = (i == 0 || (occ[i] >> 3) != (occ[i - 1] >> 3)) ? 1u : 0u;
-    uint32_t r = prank[i] + h - 1u;   // exclusive count of heads + own head - 1
-    prank[i] = r;
-    if (h) parents[r] = (occ[i] >> 3) & 0x0FFFFFFFu;
+// global index of the node m of level d, or ITS_NONE
+__device__ inline uint32_t node_of(const Tree& T, const RankWord* occ, const uint32_t* codes, int d, uint32_t m) {
+    if (d + 1 == T.depth) return m == codes[T.first[d]] ? (uint32_t)T.node[d] : ITS_NONE;
+    const uint32_t r = occ_rank(T, occ, d + 1, m >> 3);
+    return r == ITS_NONE ? ITS_NONE : (uint32_t)T.node[d] + 8u * r + (m & 7u);
 }
 
 struct NodeOut {
@@ -187,172 +262,162 @@ struct NodeOut {
     uint32_t* parent;
     uint32_t* childbase;
 };
-
-// nodes of one level: octets of the children of each occupied parent
-// (createNode_1/2 + createRemainNode, SVO.cu:560-672)
-// single_code: the root level's one cell code (device memory)
-__global__ void k_nodes_fill(int64_t n_nodes, const uint32_t* parents, const uint32_t* single_code, int64_t off,
-                             double gx, double gy, double gz, double w, NodeOut o) {
-    int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n_nodes) return;
-    uint32_t m = (n_nodes == 1) ? *single_code : ((parents[j >> 3] << 3) | (uint32_t)(j & 7));
-    int64_t g = off + j;
-    o.morton[g] = m;
-    o.is_leaf[g] = 1;
+// nodes of all levels: octets of the children of each occupied parent, and
+// the root (createNode_1/2 + createRemainNode, SVO.cu:560-672)
+__global__ void k_nodes(Tree T, const RankWord* occ, const uint32_t* codes, NodeOut o) {
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= T.node[T.depth]) return;
+    const int d = level_of(T.node, T.depth, g);
+    const int64_t j = g - T.node[d];
+    const bool root = d + 1 == T.depth;
+    const uint32_t m = root ? codes[T.first[d]] : ((codes[T.first[d + 1] + (j >> 3)] << 3) | (uint32_t)(j & 7));
+    const double w = T.width[d];
     uint32_t x, y, z;
     demorton3(m, x, y, z);
-    o.origin[3 * g + 0] = gx + w * (double)x;
-    o.origin[3 * g + 1] = gy + w * (double)y;
-    o.origin[3 * g + 2] = gz + w * (double)z;
+    o.morton[g] = m;
+    o.origin[3 * g + 0] = T.go[0] + w * (double)x;
+    o.origin[3 * g + 1] = T.go[1] + w * (double)y;
+    o.origin[3 * g + 2] = T.go[2] + w * (double)z;
     o.width[g] = w;
-    o.parent[g] = ITS_NONE;
-    o.childbase[g] = ITS_NONE;
+    o.parent[g] = root ? ITS_NONE : node_of(T, occ, codes, d + 1, m >> 3);
+    const uint32_t r = d > 0 ? occ_rank(T, occ, d, m) : ITS_NONE;
+    o.is_leaf[g] = r == ITS_NONE ? 1 : 0;
+    o.childbase[g] = r == ITS_NONE ? ITS_NONE : (uint32_t)T.node[d - 1] + 8u * r;
 }
 
-__global__ void k_nodes_occ(int64_t n_occ, const uint32_t* occ, const uint32_t* prank, int64_t n_nodes, int level,
-                            int64_t off, int64_t child_off, NodeOut o) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_occ) return;
-    int64_t addr = (n_nodes == 1) ? 0 : 8 * (int64_t)prank[i] + (occ[i] & 7);
-    int64_t g = off + addr;
-    if (level > 0) {
-        o.is_leaf[g] = 0;
-        uint32_t cb = (uint32_t)(child_off + 8 * i);
-        o.childbase[g] = cb;
-        for (int c = 0; c < 8; ++c) o.parent[cb + c] = (uint32_t)g;
-    }
-}
-
-// neighbour index k = (dx+1) + 3(dy+1) + 9(dz+1); child key x | y<<1 | z<<2.
-// Through the parent's neighbour's child, as findNeighbors (SVO.cu:858-890).
-__constant__ uint8_t c_lut_parent[8 * 27];
-__constant__ uint8_t c_lut_child[8 * 27];
-
-// One thread per (node, neighbour slot) of the level, so a wavefront stores
-// 64 consecutive entries of the 27-per-node table.
-__global__ void k_neighbors(int64_t n, int64_t off, const uint32_t* morton, const uint32_t* parent,
-                            const uint32_t* childbase, uint32_t* nb) {
+// Neighbour index k = (dx+1) + 3(dy+1) + 9(dz+1), as findNeighbors
+// (SVO.cu:858-890): the node at the neighbouring cell of the same level.  One
+// thread per (node, neighbour slot), so a wavefront stores 64 consecutive
+// entries of the 27-per-node table.
+__global__ void k_neighbors(Tree T, const RankWord* occ, const uint32_t* codes, const uint32_t* morton, uint32_t* nb) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 27 * n) return;
-    const int64_t i = t / 27;
-    const int k = (int)(t - 27 * i);
-    const int64_t g = off + i;
-    const uint32_t p = parent[g];
-    const int key = morton[g] & 7;
-    const uint32_t pn = nb[27 * (int64_t)p + c_lut_parent[key * 27 + k]];
+    if (t >= 27 * T.node[T.depth]) return;
+    const int64_t g = t / 27;
+    const int k = (int)(t - 27 * g);
     uint32_t v = ITS_NONE;
-    if (pn != ITS_NONE) {
-        const uint32_t cb = childbase[pn];
-        v = (cb == ITS_NONE) ? ITS_NONE : cb + c_lut_child[key * 27 + k];
+    if (k == 13) {
+        v = (uint32_t)g;
+    } else {
+        const int d = level_of(T.node, T.depth, g);
+        if (d + 1 < T.depth) {
+            uint32_t x, y, z;
+            demorton3(morton[g], x, y, z);
+            const uint32_t R = (uint32_t)(T.R0 >> d);
+            x += (uint32_t)(k % 3 - 1);
+            y += (uint32_t)((k / 3) % 3 - 1);
+            z += (uint32_t)(k / 9 - 1);
+            if (x < R && y < R && z < R) v = node_of(T, occ, codes, d, morton3(x, y, z));
+        }
     }
-    nb[27 * g + k] = v;
+    nb[t] = v;
 }
 
-__global__ void k_root_self(uint32_t* nb, int64_t top) { nb[27 * top + 13] = (uint32_t)top; }
-
-// ------------------------------------------------------------ vertices -----
+// -------------------------------------------------------------- vertices ----
 __device__ inline uint32_t lat_index(uint32_t X, uint32_t Y, uint32_t Z, uint32_t D) { return (X * D + Y) * D + Z; }
 
-__global__ void k_mark_corners(int64_t n, const uint32_t* morton, int64_t off, uint32_t D, uint32_t* bits) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+// Corners of all nodes.  The eight nodes of an octet share a block of 3 x 3 x 3
+// lattice points: one thread per octet and (x, y), which sets three
+// consecutive bits of the lattice, instead of 64 atomics for the octet's
+// nodes one by one.  The last item is the root, 2 x 2 x 2 points.
+__global__ void k_mark_corners(Tree T, const uint32_t* codes, RankWord* lat) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // octets of levels 0 .. depth - 2 are the occupied cells of levels 1 .. depth - 1
+    const int64_t octets = T.first[T.depth] - T.first[1];
+    const int64_t q = t / 9;
+    const int c = (int)(t - 9 * q);
+    if (q > octets) return;
+    const bool root = q == octets;
+    const int64_t i = root ? T.first[T.depth - 1] : T.first[1] + q;   // the cell whose corners these are
+    const int up = level_of(T.first, T.depth, i), d = root ? up : up - 1;
+    const uint32_t dx = (uint32_t)(c % 3), dy = (uint32_t)(c / 3);
+    if (root && (dx == 2 || dy == 2)) return;
     uint32_t x, y, z;
-    demorton3(morton[off + i], x, y, z);
-    for (int c = 0; c < 8; ++c) {
-        uint32_t idx = lat_index(x + (c & 1), y + ((c >> 1) & 1), z + ((c >> 2) & 1), D);
-        atomicOr(&bits[idx >> 5], 1u << (idx & 31));
+    demorton3(codes[i], x, y, z);
+    const uint32_t scale = root ? 1u : 2u, D = (uint32_t)(T.R0 >> d) + 1u;
+    const uint32_t key = lat_index(scale * x + dx, scale * y + dy, scale * z, D);
+    const uint64_t bits = (uint64_t)(root ? 3u : 7u) << (key & 31);
+    RankWord* g = lat + T.lat[d] + (key >> 5);
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t b = (uint32_t)(bits >> (32 * h));
+        if (b && (__hip_atomic_load(&g[h].bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & b) != b)
+            atomicOr(&g[h].bits, b);
     }
 }
 
-__global__ void k_emit_verts(const RankWord* g, int64_t nwords, uint32_t D, int64_t voff, int level, uint16_t* vx,
-                             uint16_t* vy, uint16_t* vz, uint8_t* vlev, uint32_t* owner) {
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= nwords) return;
-    RankWord rw = g[w];
+// lattice keys of the vertices, by rank; the ranks, counted over all levels so
+// far, become ranks within the level
+__global__ void k_vert_keys(Tree T, RankWord* lat, uint32_t* keys) {
+    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= T.lat[T.depth]) return;
+    const RankWord rw = lat[w];
+    const int d = level_of(T.lat, T.depth, w);
+    lat[w].rank = rw.rank - (uint32_t)T.vert[d];
     uint32_t b = rw.bits, r = rw.rank;
+    const uint32_t base = (uint32_t)(w - T.lat[d]) * 32u;
     while (b) {
-        int bi = __ffs(b) - 1;
-        uint32_t idx = (uint32_t)(w * 32 + bi);
-        int64_t v = voff + r++;
-        vx[v] = (uint16_t)(idx / (D * D));
-        vy[v] = (uint16_t)((idx / D) % D);
-        vz[v] = (uint16_t)(idx % D);
-        vlev[v] = (uint8_t)level;
-        owner[v] = ITS_NONE;
+        keys[r++] = base + (uint32_t)(__ffs(b) - 1);
         b &= b - 1;
     }
 }
 
-// owner = smallest global index of the nodes sharing the corner (the min over
-// d_vertSharedLUT neighbours in determineNodeVertex, SVO.cu:950-960)
-__global__ void k_owner(int64_t n, const uint32_t* morton, int64_t off, uint32_t D, const RankWord* lat, int64_t voff,
-                        uint32_t* owner, uint32_t* node_corner) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int64_t g = off + i;
-    uint32_t x, y, z;
-    demorton3(morton[g], x, y, z);
-    for (int c = 0; c < 8; ++c) {
-        uint32_t idx = lat_index(x + (c & 1), y + ((c >> 1) & 1), z + ((c >> 2) & 1), D);
-        uint32_t v = (uint32_t)(voff + bit_rank(lat, idx));
-        atomicMin(&owner[v], (uint32_t)g);
-        node_corner[8 * g + c] = v;
-    }
-}
-
-// corner position from the owner node: origin + width * (offset), the copy
-// the reference's stable sort + unique keeps (SVO.cu:1081-1082)
-__global__ void k_vxyz(int64_t nv, int64_t voff, const uint16_t* vx, const uint16_t* vy, const uint16_t* vz,
-                       const uint32_t* owner, const uint32_t* morton, const double* origin, const double* width,
-                       double* xyz) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nv) return;
-    int64_t v = voff + i;
-    uint32_t o = owner[v];
-    uint32_t x, y, z;
-    demorton3(morton[o], x, y, z);
-    double w = width[o];
-    xyz[3 * v + 0] = origin[3 * (int64_t)o + 0] + w * (double)(vx[v] - x);
-    xyz[3 * v + 1] = origin[3 * (int64_t)o + 1] + w * (double)(vy[v] - y);
-    xyz[3 * v + 2] = origin[3 * (int64_t)o + 2] + w * (double)(vz[v] - z);
-}
-
-// once per device, also when several host threads make their first call
-void upload_luts() {
-    static std::mutex mu;
-    static uint64_t done_mask = 0;   // devices holding the tables
-    int dev;
-    ITS_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lock(mu);
-    if (dev < 64 && ((done_mask >> dev) & 1u)) return;
-    uint8_t lp[8 * 27], lc[8 * 27];
-    for (int key = 0; key < 8; ++key) {
-        int c[3] = {key & 1, (key >> 1) & 1, (key >> 2) & 1};
-        for (int k = 0; k < 27; ++k) {
-            int d[3] = {k % 3 - 1, (k / 3) % 3 - 1, k / 9 - 1};
-            int pk = 0, ck = 0, mul = 1;
-            for (int a = 0; a < 3; ++a) {
-                int t = c[a] + d[a];
-                int pd = (t < 0) ? -1 : (t > 1 ? 1 : 0);
-                pk += (pd + 1) * mul;
-                ck |= (t & 1) << a;
-                mul *= 3;
-            }
-            lp[key * 27 + k] = (uint8_t)pk;
-            lc[key * 27 + k] = (uint8_t)ck;
+struct VertOut {
+    uint16_t *x, *y, *z;
+    uint8_t* level;
+    uint32_t* owner;
+    double* xyz;
+};
+// Vertices of all levels: lattice coordinates; the owner, the smallest index
+// of the nodes sharing the corner (the min over d_vertSharedLUT neighbours in
+// determineNodeVertex, SVO.cu:950-960), which within a level is the smallest
+// code; and the position from it, origin + width * (offset), the copy the
+// reference's stable sort + unique keeps (SVO.cu:1081-1082).
+__global__ void k_vertices(Tree T, const RankWord* occ, const uint32_t* codes, const uint32_t* keys, VertOut o) {
+    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= T.vert[T.depth]) return;
+    const int d = level_of(T.vert, T.depth, v);
+    const uint32_t R = (uint32_t)(T.R0 >> d), D = R + 1u, key = keys[v];
+    const uint32_t XY = key / D, Z = key - XY * D, X = XY / D, Y = XY - X * D;
+    uint32_t own = ITS_NONE, ox = 0, oy = 0, oz = 0;
+    for (int k = 0; k < 8; ++k) {
+        const uint32_t x = X - (k & 1), y = Y - ((k >> 1) & 1), z = Z - ((k >> 2) & 1);
+        if (x >= R || y >= R || z >= R) continue;
+        const uint32_t g = node_of(T, occ, codes, d, morton3(x, y, z));
+        if (g < own) {
+            own = g;
+            ox = x;
+            oy = y;
+            oz = z;
         }
     }
-    ITS_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_lut_parent), lp, sizeof lp));
-    ITS_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_lut_child), lc, sizeof lc));
-    if (dev < 64) done_mask |= 1ull << dev;
+    const double w = T.width[d];
+    o.x[v] = (uint16_t)X;
+    o.y[v] = (uint16_t)Y;
+    o.z[v] = (uint16_t)Z;
+    o.level[v] = (uint8_t)d;
+    o.owner[v] = own;
+    o.xyz[3 * v + 0] = (T.go[0] + w * (double)ox) + w * (double)(X - ox);
+    o.xyz[3 * v + 1] = (T.go[1] + w * (double)oy) + w * (double)(Y - oy);
+    o.xyz[3 * v + 2] = (T.go[2] + w * (double)oz) + w * (double)(Z - oz);
+}
+
+// ranks of n bitsets in a row and the count before each of them and in all,
+// in one read-back
+std::vector<int64_t> rank_levels(RankWord* g, const Starts& S, int64_t words, hipStream_t st) {
+    DBuf<uint32_t> first(S.n + 2);
+    uint32_t* total = first.p + S.n + 1;
+    rank_build_async(g, words, st, total);
+    hipLaunchKernelGGL(k_level_first, dim3(1), dim3(64), 0, st, (const RankWord*)g, S, (const uint32_t*)total, first.p);
+    ITS_LAUNCH_CHECK();
+    std::vector<uint32_t> h;
+    to_host(h, first.p, S.n + 1, st);
+    return std::vector<int64_t>(h.begin(), h.end());
 }
 
 }  // namespace
 
-void svo_build(its_svo s, const double* d_tris, int64_t T) {
+void svo_build(its_svo s, const double* d_tris, int64_t n_tris) {
     hipStream_t st = s->ctx->stream;
     const int R = s->R;
-    upload_luts();
     Grid g;
     for (int a = 0; a < 3; ++a) {
         g.go[a] = s->origin[a];
@@ -361,101 +426,73 @@ void svo_build(its_svo s, const double* d_tris, int64_t T) {
     g.R = R;
     s->voxel_width = g.unit[0];        // unitNodeWidth = unitVoxelSize.x()
 
-    // ---- voxelize into a Morton-ordered bitset
-    const int64_t ncell = (int64_t)R * R * R;
-    const int64_t nwords0 = std::max<int64_t>(1, (ncell + 31) / 32);
-    DBuf<uint32_t> bits(nwords0);
-    ITS_HIP(hipMemsetAsync(bits.p, 0, bits.bytes(), st));
-    if (T > 0) {
-        DBuf<uint64_t> cnt(T);
-        hipLaunchKernelGGL(k_tri_count, dim3(blocks_for(T, kT)), dim3(kT), 0, st, d_tris, T, g, cnt.p);
+    Tree T{};
+    T.R0 = R;
+    for (int a = 0; a < 3; ++a) T.go[a] = g.go[a];
+    T.top = 1;
+    while ((R >> (T.top - 1)) > 1) ++T.top;
+    ITS_REQUIRE(T.top <= kMaxLevels, ITS_E_RANGE, "octree deeper than supported");
+    Starts S{};
+    S.n = T.top;
+    for (int d = 0; d < T.top; ++d) {
+        const int64_t side = R >> d;
+        T.word[d + 1] = T.word[d] + std::max<int64_t>(1, (side * side * side + 31) / 32);
+        S.word[d] = T.word[d];
+    }
+    const int64_t words = T.word[T.top];
+
+    // ---- occupancy: voxels, then the pyramid above them
+    DBuf<RankWord> occ(words);
+    ITS_HIP(hipMemsetAsync(occ.p, 0, occ.bytes(), st));
+    if (n_tris > 0) {
+        DBuf<uint64_t> cnt(n_tris);
+        hipLaunchKernelGGL(k_tri_count, dim3(blocks_for(n_tris, kT)), dim3(kT), 0, st, d_tris, n_tris, g, cnt.p);
         ITS_LAUNCH_CHECK();
-        uint64_t total = scan_exclusive_u64(cnt.p, cnt.p, T, st);
+        const uint64_t total = scan_exclusive_u64(cnt.p, cnt.p, n_tris, st);
         if (total) {
             unsigned nb = (unsigned)std::min<uint64_t>((total + kT - 1) / kT, 1u << 20);
-            hipLaunchKernelGGL(k_voxelize, dim3(nb), dim3(kT), 0, st, d_tris, T, cnt.p, total, g, bits.p);
+            hipLaunchKernelGGL(k_voxelize, dim3(nb), dim3(kT), 0, st, d_tris, n_tris, (const uint64_t*)cnt.p, total, g,
+                               occ.p);
             ITS_LAUNCH_CHECK();
         }
     }
-    Level& l0 = s->lv[0];
-    {
-        DBuf<RankWord> occbits(nwords0);
-        hipLaunchKernelGGL(k_pack_bits, dim3(blocks_for(nwords0, kT)), dim3(kT), 0, st, bits.p, nwords0, occbits.p);
+    int d0 = 0;
+    for (; d0 + 1 < T.top && T.word[d0 + 2] - T.word[d0 + 1] > kOccTopThreads; ++d0) {
+        const int64_t nup = T.word[d0 + 2] - T.word[d0 + 1];
+        hipLaunchKernelGGL(k_occ_up, dim3(blocks_for(nup, kT)), dim3(kT), 0, st, (const RankWord*)occ.p + T.word[d0],
+                           T.word[d0 + 1] - T.word[d0], occ.p + T.word[d0 + 1], nup);
         ITS_LAUNCH_CHECK();
-        int64_t nvox = (int64_t)rank_build(occbits.p, nwords0, st);
-        s->num_voxels = nvox;
-        l0.occ.alloc(std::max<int64_t>(nvox, 1));
-        hipLaunchKernelGGL(k_emit_bits, dim3(blocks_for(nwords0, kT)), dim3(kT), 0, st, occbits.p, nwords0, l0.occ.p);
-        ITS_LAUNCH_CHECK();
-        l0.n_occ = nvox;
     }
-    bits.release();
+    hipLaunchKernelGGL(k_occ_top, dim3(1), dim3(kOccTopThreads), 0, st, T, d0, occ.p);
+    ITS_LAUNCH_CHECK();
 
-    // ---- level loop (SVO.cu:717-815): a level with a single occupied cell
-    // is the root.  Every level up to the one-cell grid (R >> d == 1) is
-    // built with its buffers sized by a bound (the level below's bound, and
-    // the level's cell count); the cell counts stay in device memory and come
-    // back in one read, which places the root.  Levels above the root are
-    // dropped.
-    int depth = 0;
-    DBuf<uint32_t> lcount;   // cells per level, device
-    if (l0.n_occ > 0) {
-        int top = 0;
-        while ((R >> top) > 1) ++top;
-        ITS_REQUIRE(top < kMaxLevels, ITS_E_RANGE, "octree deeper than supported");
-        lcount.alloc(top + 1);
-        const uint32_t n0 = (uint32_t)l0.n_occ;
-        ITS_HIP(hipMemcpyAsync(lcount.p, &n0, sizeof n0, hipMemcpyHostToDevice, st));
-        std::vector<int64_t> bound(top + 1);
-        bound[0] = l0.n_occ;
-        for (int d = 0; d < top; ++d) {
-            Level& L = s->lv[d];
-            Level& P = s->lv[d + 1];
-            const int64_t side = R >> (d + 1);
-            bound[d + 1] = std::min<int64_t>(bound[d], side * side * side);
-            L.prank.alloc(bound[d]);
-            hipLaunchKernelGGL(k_heads, dim3(blocks_for(bound[d], kT)), dim3(kT), 0, st, L.occ.p,
-                               (const uint32_t*)lcount.p + d, bound[d], L.prank.p);
-            ITS_LAUNCH_CHECK();
-            scan_exclusive_u32_async(L.prank.p, L.prank.p, bound[d], st, lcount.p + d + 1);
-            P.occ.alloc(bound[d + 1]);
-            hipLaunchKernelGGL(k_parents, dim3(blocks_for(bound[d], kT)), dim3(kT), 0, st, L.occ.p,
-                               (const uint32_t*)lcount.p + d, bound[d], L.prank.p, P.occ.p);
-            ITS_LAUNCH_CHECK();
-        }
-        std::vector<uint32_t> h;
-        to_host(h, lcount.p, top + 1, st);
-        double w = g.unit[0];
-        for (int d = 0; d <= top; ++d) {
-            Level& L = s->lv[d];
-            L.R = std::max(1, R >> d);
-            L.width = w;
-            L.n_occ = h[d];
-            depth = d + 1;
-            if (h[d] == 1) {
-                L.n_nodes = 1;
-                break;
-            }
-            ITS_REQUIRE(d < top && h[d] > 1, ITS_E_STATE, "octree level loop did not reach a single cell");
-            L.n_nodes = 8 * (int64_t)h[d + 1];
-            w *= 2.0;
-        }
-        for (int d = depth; d <= top; ++d) {   // above the root
-            s->lv[d].occ.release();
-            s->lv[d].prank.release();
-            s->lv[d].n_occ = 0;
-        }
-        s->lv[depth - 1].prank.release();
+    // ---- levels (SVO.cu:717-815): the first with a single occupied cell is
+    // the root; the levels above it are dropped
+    const std::vector<int64_t> first = rank_levels(occ.p, S, words, st);
+    for (int d = 0; d <= T.top; ++d) T.first[d] = first[d];
+    s->num_voxels = first[1];
+    s->occ_codes.alloc(std::max<int64_t>(first[T.top], 1));
+    s->depth = 0;
+    s->num_nodes = 0;
+    if (s->num_voxels == 0) return;
+    hipLaunchKernelGGL(k_occ_codes, dim3(blocks_for(words, kT)), dim3(kT), 0, st, (const RankWord*)occ.p, T,
+                       s->occ_codes.p);
+    ITS_LAUNCH_CHECK();
+    double w = g.unit[0];
+    for (int d = 0; d < T.top && s->depth == 0; ++d, w *= 2.0) {
+        Level& L = s->lv[d];
+        L.R = R >> d;
+        L.width = w;
+        T.width[d] = w;
+        L.n_occ = first[d + 1] - first[d];
+        if (L.n_occ == 1) s->depth = d + 1;
+        L.n_nodes = L.n_occ == 1 ? 1 : 8 * (first[d + 2] - first[d + 1]);
+        T.node[d + 1] = T.node[d] + L.n_nodes;
     }
-    s->depth = depth;
-    int64_t total = 0;
-    for (int d = 0; d < depth; ++d) {
-        s->esum_nodes[d] = total;
-        total += s->lv[d].n_nodes;
-    }
-    s->esum_nodes[depth] = total;
-    s->num_nodes = total;
-    if (depth == 0) return;
+    ITS_REQUIRE(s->depth > 0, ITS_E_STATE, "octree level loop did not reach a single cell");
+    const int depth = T.depth = s->depth;
+    for (int d = 0; d <= depth; ++d) s->esum_nodes[d] = T.node[d];
+    const int64_t total = s->num_nodes = T.node[depth];
 
     // ---- node arrays
     s->morton.alloc(total);
@@ -464,89 +501,49 @@ void svo_build(its_svo s, const double* d_tris, int64_t T) {
     s->node_width.alloc(total);
     s->parent.alloc(total);
     s->childbase.alloc(total);
-    NodeOut o{s->morton.p, s->is_leaf.p, s->node_origin.p, s->node_width.p, s->parent.p, s->childbase.p};
-    for (int d = 0; d < depth; ++d) {
-        Level& L = s->lv[d];
-        const uint32_t* parents = (d + 1 < depth) ? s->lv[d + 1].occ.p : nullptr;
-        hipLaunchKernelGGL(k_nodes_fill, dim3(blocks_for(L.n_nodes, kT)), dim3(kT), 0, st, L.n_nodes, parents,
-                           (const uint32_t*)L.occ.p,
-                           s->esum_nodes[d], g.go[0], g.go[1], g.go[2], L.width, o);
-        ITS_LAUNCH_CHECK();
-    }
-    for (int d = 0; d < depth; ++d) {
-        Level& L = s->lv[d];
-        hipLaunchKernelGGL(k_nodes_occ, dim3(blocks_for(L.n_occ, kT)), dim3(kT), 0, st, L.n_occ, L.occ.p,
-                           L.n_nodes == 1 ? nullptr : L.prank.p, L.n_nodes, d, s->esum_nodes[d],
-                           d > 0 ? s->esum_nodes[d - 1] : 0, o);
-        ITS_LAUNCH_CHECK();
-    }
-
-    // ---- neighbours, top-down
     s->neighbors.alloc(27 * total);
-    ITS_HIP(hipMemsetAsync(s->neighbors.p, 0xFF, s->neighbors.bytes(), st));
-    hipLaunchKernelGGL(k_root_self, dim3(1), dim3(1), 0, st, s->neighbors.p, total - 1);
+    const NodeOut o{s->morton.p, s->is_leaf.p, s->node_origin.p, s->node_width.p, s->parent.p, s->childbase.p};
+    const RankWord* d_occ = occ.p;
+    const uint32_t* codes = s->occ_codes.p;
+    hipLaunchKernelGGL(k_nodes, dim3(blocks_for(total, kT)), dim3(kT), 0, st, T, d_occ, codes, o);
     ITS_LAUNCH_CHECK();
-    for (int d = depth - 2; d >= 0; --d) {
-        Level& L = s->lv[d];
-        hipLaunchKernelGGL(k_neighbors, dim3(blocks_for(27 * L.n_nodes, kT)), dim3(kT), 0, st, L.n_nodes, s->esum_nodes[d],
-                           s->morton.p, s->parent.p, s->childbase.p, s->neighbors.p);
-        ITS_LAUNCH_CHECK();
-    }
 
-    // ---- vertices per level: every level's lattice bits and ranks are
-    // launched, then all vertex counts come back in one read
-    int64_t nv_total = 0;
-    std::vector<int64_t> lat_words(depth);
-    DBuf<uint32_t> vcount(depth);
+    // ---- corner lattices
+    S.n = depth;
     for (int d = 0; d < depth; ++d) {
-        Level& L = s->lv[d];
-        const uint32_t D = (uint32_t)L.R + 1;
-        const int64_t nbits = (int64_t)D * D * D;
-        const int64_t nwords = (nbits + 31) / 32;
-        lat_words[d] = nwords;
-        DBuf<uint32_t> lb(nwords);
-        ITS_HIP(hipMemsetAsync(lb.p, 0, lb.bytes(), st));
-        hipLaunchKernelGGL(k_mark_corners, dim3(blocks_for(L.n_nodes, kT)), dim3(kT), 0, st, L.n_nodes, s->morton.p,
-                           s->esum_nodes[d], D, lb.p);
-        ITS_LAUNCH_CHECK();
-        L.lattice.alloc(nwords);
-        hipLaunchKernelGGL(k_pack_bits, dim3(blocks_for(nwords, kT)), dim3(kT), 0, st, lb.p, nwords, L.lattice.p);
-        ITS_LAUNCH_CHECK();
-        rank_build_async(L.lattice.p, nwords, st, vcount.p + d);
+        const int64_t D = s->lv[d].R + 1;
+        T.lat[d + 1] = T.lat[d] + (D * D * D + 31) / 32;
+        S.word[d] = T.lat[d];
     }
-    {
-        std::vector<uint32_t> h(depth);
-        ITS_HIP(hipMemcpyAsync(h.data(), vcount.p, depth * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        ITS_HIP(hipStreamSynchronize(st));
-        for (int d = 0; d < depth; ++d) {
-            s->lv[d].n_verts = (int64_t)h[d];
-            s->esum_verts[d] = nv_total;
-            nv_total += s->lv[d].n_verts;
-        }
-    }
-    s->esum_verts[depth] = nv_total;
-    s->num_verts = nv_total;
-    s->vx.alloc(nv_total);
-    s->vy.alloc(nv_total);
-    s->vz.alloc(nv_total);
-    s->vlevel.alloc(nv_total);
-    s->vowner.alloc(nv_total);
-    s->vxyz.alloc(3 * nv_total);
-    s->node_corner.alloc(8 * total);
-    for (int d = 0; d < depth; ++d) {
-        Level& L = s->lv[d];
-        const uint32_t D = (uint32_t)L.R + 1;
-        hipLaunchKernelGGL(k_emit_verts, dim3(blocks_for(lat_words[d], kT)), dim3(kT), 0, st, L.lattice.p, lat_words[d],
-                           D, s->esum_verts[d], d, s->vx.p, s->vy.p, s->vz.p, s->vlevel.p, s->vowner.p);
-        ITS_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_owner, dim3(blocks_for(L.n_nodes, kT)), dim3(kT), 0, st, L.n_nodes, s->morton.p,
-                           s->esum_nodes[d], D, L.lattice.p, s->esum_verts[d], s->vowner.p, s->node_corner.p);
-        ITS_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_vxyz, dim3(blocks_for(L.n_verts, kT)), dim3(kT), 0, st, L.n_verts, s->esum_verts[d],
-                           s->vx.p, s->vy.p, s->vz.p, s->vowner.p, s->morton.p, s->node_origin.p, s->node_width.p,
-                           s->vxyz.p);
-        ITS_LAUNCH_CHECK();
-    }
+    const int64_t lat_words = T.lat[depth];
+    s->lattice.alloc(lat_words);
+    ITS_HIP(hipMemsetAsync(s->lattice.p, 0, s->lattice.bytes(), st));
+    for (int d = 0; d < depth; ++d) s->lv[d].lattice.p = s->lattice.p + T.lat[d];
+    const int64_t items = 9 * (T.first[depth] - T.first[1] + 1);
+    hipLaunchKernelGGL(k_mark_corners, dim3(blocks_for(items, kT)), dim3(kT), 0, st, T, codes, s->lattice.p);
+    ITS_LAUNCH_CHECK();
+    // queued behind the marks, in front of the read-back
+    hipLaunchKernelGGL(k_neighbors, dim3(blocks_for(27 * total, kT)), dim3(kT), 0, st, T, d_occ, codes,
+                       (const uint32_t*)s->morton.p, s->neighbors.p);
+    ITS_LAUNCH_CHECK();
+    const std::vector<int64_t> vert = rank_levels(s->lattice.p, S, lat_words, st);
+    for (int d = 0; d <= depth; ++d) s->esum_verts[d] = T.vert[d] = vert[d];
+    for (int d = 0; d < depth; ++d) s->lv[d].n_verts = vert[d + 1] - vert[d];
+    const int64_t nv = s->num_verts = vert[depth];
+
+    // ---- vertices
+    s->vx.alloc(nv);
+    s->vy.alloc(nv);
+    s->vz.alloc(nv);
+    s->vlevel.alloc(nv);
+    s->vowner.alloc(nv);
+    s->vxyz.alloc(3 * nv);
+    DBuf<uint32_t> keys(nv);
+    hipLaunchKernelGGL(k_vert_keys, dim3(blocks_for(lat_words, kT)), dim3(kT), 0, st, T, s->lattice.p, keys.p);
+    ITS_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_vertices, dim3(blocks_for(nv, kT)), dim3(kT), 0, st, T, d_occ, codes, (const uint32_t*)keys.p,
+                       VertOut{s->vx.p, s->vy.p, s->vz.p, s->vlevel.p, s->vowner.p, s->vxyz.p});
+    ITS_LAUNCH_CHECK();
     ITS_HIP(hipStreamSynchronize(st));
 }
 
@@ -643,16 +640,22 @@ void svo_from_vertices(its_svo s, const double* xyz, const uint32_t* owner, int6
         ho[j] = owner[i];
         for (int a = 0; a < 3; ++a) hxyz[3 * j + a] = xyz[3 * i + a];
     }
-    int64_t at = 0;
-    std::vector<std::vector<RankWord>> lat(depth);
+    int64_t at = 0, words = 0;
+    std::vector<int64_t> lat_off(depth);
+    for (int d = 0; d < depth; ++d) {
+        const int64_t D = (int64_t)(R >> d) + 1;
+        lat_off[d] = words;
+        words += (D * D * D + 31) / 32;
+    }
+    std::vector<RankWord> lat(words, RankWord{0, 0});
+    s->lattice.alloc(words);
     for (int d = 0; d < depth; ++d) {
         Level& L = s->lv[d];
         L.R = R >> d;
         L.width = std::ldexp(w0, d);
+        L.lattice.p = s->lattice.p + lat_off[d];
         const int64_t D = (int64_t)L.R + 1;
-        const int64_t nwords = (D * D * D + 31) / 32;
-        std::vector<RankWord>& g = lat[d];
-        g.assign(nwords, RankWord{0, 0});
+        RankWord* g = lat.data() + lat_off[d];
         s->esum_verts[d] = at;
         int64_t cnt = 0;
         while (at < n && hl[at] == d) {
@@ -663,13 +666,12 @@ void svo_from_vertices(its_svo s, const double* xyz, const uint32_t* owner, int6
         }
         L.n_verts = cnt;
         uint32_t run = 0;
-        for (RankWord& w : g) {
-            w.rank = run;
-            run += (uint32_t)__builtin_popcount(w.bits);
+        for (int64_t w = 0; w < (D * D * D + 31) / 32; ++w) {
+            g[w].rank = run;
+            run += (uint32_t)__builtin_popcount(g[w].bits);
         }
-        L.lattice.alloc(nwords);
-        ITS_HIP(hipMemcpyAsync(L.lattice.p, g.data(), nwords * sizeof(RankWord), hipMemcpyHostToDevice, st));
     }
+    ITS_HIP(hipMemcpyAsync(s->lattice.p, lat.data(), words * sizeof(RankWord), hipMemcpyHostToDevice, st));
     s->esum_verts[depth] = n;
     s->vx.alloc(n);
     s->vy.alloc(n);
