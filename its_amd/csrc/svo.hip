@@ -54,32 +54,28 @@ __global__ void k_tri_count(const double* tris, int64_t T, Grid g, uint64_t* cnt
     cnt[t] = (uint64_t)(be[0] - bo[0] + 1) * (uint64_t)(be[1] - bo[1] + 1) * (uint64_t)(be[2] - bo[2] + 1);
 }
 
+// first triangle of every 256 candidates
+__global__ void k_cand_starts(const uint64_t* off, int64_t T, uint64_t total, uint32_t* start) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= T) return;
+    const uint64_t c0 = off[t], c1 = t + 1 < T ? off[t + 1] : total;
+    for (uint64_t b = (c0 + kT - 1) / kT; b * kT < c1; ++b) start[b] = (uint32_t)t;
+}
+
 // One thread per (triangle, candidate voxel); the triangle set-up is
 // recomputed per candidate, in the reference's expression order.  A block's
 // 256 candidates belong to at most 256 consecutive triangles, since every
-// triangle has one: the block finds the range once and each thread searches
-// its part of the offsets in LDS (18 dependent global reads a thread before:
-// 108 us for 200,000 triangles at R = 256).
+// triangle has one: they start at the block's entry of start (k_cand_starts),
+// and each thread searches their offsets in LDS.
 __global__ __launch_bounds__(kT) void k_voxelize(const double* tris, int64_t T, const uint64_t* off, uint64_t total,
-                                                 Grid g, RankWord* occ) {
+                                                 const uint32_t* start, Grid g, RankWord* occ) {
     __shared__ uint64_t s_off[kT + 1];
-    __shared__ int64_t s_t[2];
-    for (uint64_t c0 = (uint64_t)blockIdx.x * kT; c0 < total; c0 += (uint64_t)gridDim.x * kT) {
+    for (uint64_t b = blockIdx.x; b * kT < total; b += gridDim.x) {
+        const uint64_t c0 = b * kT;
+        const int64_t t0 = start[b], t1 = c0 + kT < total ? (int64_t)start[b + 1] : T - 1;
+        const int nt = (int)min(t1 - t0 + 1, (int64_t)kT);
         __syncthreads();
-        if (threadIdx.x < 2) {   // last t with off[t] <= the block's first / last candidate
-            const uint64_t c = threadIdx.x == 0 ? c0 : min(c0 + kT, total) - 1;
-            int64_t lo = 0, hi = T - 1;
-            while (lo < hi) {
-                const int64_t mid = (lo + hi + 1) >> 1;
-                if (off[mid] <= c) lo = mid;
-                else hi = mid - 1;
-            }
-            s_t[threadIdx.x] = lo;
-        }
-        __syncthreads();
-        const int64_t t0 = s_t[0];
-        const int nt = (int)(s_t[1] - t0) + 1;
-        for (int q = threadIdx.x; q < nt; q += kT) s_off[q] = off[t0 + q];
+        if ((int)threadIdx.x < nt) s_off[threadIdx.x] = off[t0 + threadIdx.x];
         __syncthreads();
         const uint64_t c = c0 + threadIdx.x;
         if (c >= total) continue;
@@ -451,8 +447,12 @@ void svo_build(its_svo s, const double* d_tris, int64_t n_tris) {
         const uint64_t total = scan_exclusive_u64(cnt.p, cnt.p, n_tris, st);
         if (total) {
             unsigned nb = (unsigned)std::min<uint64_t>((total + kT - 1) / kT, 1u << 20);
-            hipLaunchKernelGGL(k_voxelize, dim3(nb), dim3(kT), 0, st, d_tris, n_tris, (const uint64_t*)cnt.p, total, g,
-                               occ.p);
+            DBuf<uint32_t> start((total + kT - 1) / kT);
+            hipLaunchKernelGGL(k_cand_starts, dim3(blocks_for(n_tris, kT)), dim3(kT), 0, st, (const uint64_t*)cnt.p,
+                               n_tris, total, start.p);
+            ITS_LAUNCH_CHECK();
+            hipLaunchKernelGGL(k_voxelize, dim3(nb), dim3(kT), 0, st, d_tris, n_tris, (const uint64_t*)cnt.p, total,
+                               (const uint32_t*)start.p, g, occ.p);
             ITS_LAUNCH_CHECK();
         }
     }
