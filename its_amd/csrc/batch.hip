@@ -33,7 +33,8 @@ struct FitDesc {
     int64_t max_iter;
     double tol;
     int64_t off[kMaxLevels + 1];
-    const uint32_t *pro_ptr, *pro_idx, *res_ptr, *res_idx, *down, *up;
+    Lists lists;
+    const uint32_t *down, *up;
     const uint8_t* finest;
     const float* invd32;
     const double* b;
@@ -59,9 +60,8 @@ __device__ inline double bsum(double v, double* sh) {
 __device__ void prolong64(const FitDesc& D, const double* x, double* g) {
     for (int d = D.L - 1; d >= 0; --d) {
         for (int64_t i = D.off[d] + threadIdx.x; i < D.off[d + 1]; i += kB) {
-            const uint32_t k0 = D.pro_ptr[i], k1 = D.pro_ptr[i + 1];
-            const double s = gather_parents(D.pro_idx, k0, k1, (const double*)g);
-            const double w = (k1 > k0) ? 1.0 / (double)(k1 - k0) : 0.0;
+            double w;
+            const double s = gather_parents<double>(D.lists.par[i], w, 0u, [&](uint32_t j) { return g[j]; });
             g[i] = x[i] + w * s;
         }
         __syncthreads();
@@ -82,7 +82,7 @@ __device__ void apply_AT(const FitDesc& D, const T* r, T* h) {
     __syncthreads();
     for (int d = 1; d < D.L; ++d) {
         for (int64_t c = D.off[d] + threadIdx.x; c < D.off[d + 1]; c += kB) {
-            h[c] += gather_children(D.res_idx, D.res_ptr[c], D.res_ptr[c + 1], (const T*)h);
+            h[c] += gather_children(D.lists, c, (const T*)h);
         }
         __syncthreads();
     }
@@ -136,9 +136,8 @@ __device__ int64_t inner_cgls(const FitDesc& D, double rel_tol, int64_t max_it, 
             for (int64_t i = D.off[d] + threadIdx.x; i < D.off[d + 1]; i += kB) {
                 const float pi = D.z[i] + (float)beta * D.p[i];
                 D.p[i] = pi;
-                const uint32_t k0 = D.pro_ptr[i], k1 = D.pro_ptr[i + 1];
-                const float s = gather_parents(D.pro_idx, k0, k1, (const float*)D.g);
-                const float w = (k1 > k0) ? 1.f / (float)(k1 - k0) : 0.f;
+                float w;
+                const float s = gather_parents<float>(D.lists.par[i], w, 0u, [&](uint32_t j) { return D.g[j]; });
                 D.g[i] = pi + w * s;
             }
             __syncthreads();
@@ -171,7 +170,7 @@ __device__ int64_t inner_cgls(const FitDesc& D, double rel_tol, int64_t max_it, 
         __syncthreads();
         for (int d = 1; d < D.L; ++d) {
             for (int64_t cc = D.off[d] + threadIdx.x; cc < D.off[d + 1]; cc += kB) {
-                D.h[cc] += gather_children(D.res_idx, D.res_ptr[cc], D.res_ptr[cc + 1], (const float*)D.h);
+                D.h[cc] += gather_children(D.lists, cc, (const float*)D.h);
             }
             __syncthreads();
         }
@@ -372,10 +371,7 @@ void batch_fit(its_batch b, double tol, int64_t max_iter, bool warm, its_lscg_st
         D.max_iter = max_iter;
         D.tol = tol;
         for (int d = 0; d <= f->L; ++d) D.off[d] = f->off[d];
-        D.pro_ptr = f->pro_ptr.p;
-        D.pro_idx = f->pro_idx.p;
-        D.res_ptr = f->res_ptr.p;
-        D.res_idx = f->res_idx.p;
+        D.lists = f->lists();
         D.down = f->down.p;
         D.up = f->up.p;
         D.finest = f->finest.p;

@@ -9,46 +9,85 @@ struct Coarse {
     uint32_t off[kMaxLevels + 1];   // global vertex offsets
 };
 
-// Operator gathers shared by the single-mesh and the batched solver.  Index
-// lists are read a chunk at a time and then the chunk's values, so a thread
-// waits for two loads per chunk instead of two per entry; the sums keep the
-// list order.  Parent lists hold at most 8 entries (one chunk of 8); child
-// lists up to 27 (one chunk of 32).
-// sum of g over the prolongation list [k0, k1) (coarse parents of a vertex)
-template <class T>
-__device__ inline T gather_parents(const uint32_t* idx, uint32_t k0, uint32_t k1, const T* g) {
-    T s = 0;
-    for (uint32_t kb = k0; kb < k1; kb += 8) {
-        uint32_t id[8];
-        T gv[8];
+// Operator lists, shared by the single-mesh and the batched solver.
+//
+// The parents of a vertex and the children of a coarse vertex are runs of
+// lattice points, and consecutive points along z that exist are consecutive
+// vertices.  A list is therefore stored by its (x, y) columns:
+//   - parents: up to 4 columns of 1 or 2 points (2 where the vertex's z is
+//     odd, bit 28 of the first column), one 16-byte word per vertex;
+//   - children, at 2 (X, Y, Z) + {-1, 0, 1}^3: 9 columns, each the first
+//     child's index with a 3-bit mask of the points that exist in bits 28 to
+//     30, in slices of 64 vertices, column by column, so that a wavefront
+//     reads whole lines.  A child's weight, 2^-(its odd coordinates), follows
+//     from its place.
+// Lists by offset and length cost two dependent reads before the entries, and
+// the entries of neighbouring vertices lay 27 apart.  256^3 knot, average of
+// the levels' launches: restriction 5.3 -> 4.3 us (one-workgroup levels 11.4
+// -> 7.1), prolongation 3.9 -> 3.5; with a branch around every read instead
+// of a safe address it was 6.9 and 11.5.  Sums run over the parents z-major
+// and over the children x-major, ascending.
+struct Lists {
+    const uint4* par;
+    const uint32_t* kid;
+    int64_t kid0;   // first vertex with children (of level 1)
+};
+constexpr uint32_t kListIdx = 0x0FFFFFFFu;
+__host__ __device__ inline int64_t kid_slot(int64_t c, int q) { return ((c >> 6) * 9 + q) * 64 + (c & 63); }
+
+// Points that do not exist are read from `safe` and not added: the loads are
+// straight-line code, all in flight at once, with no branch around each.
+// sum of g over the parents P; w = 1 / their count (0 without parents)
+template <class T, class Read>
+__device__ inline T gather_parents(uint4 P, T& w, uint32_t safe, Read&& g) {
+    const bool any = P.x != ITS_NONE, two = P.y != ITS_NONE, four = P.z != ITS_NONE, zz = any && ((P.x >> 28) & 1u);
+    const uint32_t c[4] = {P.x & kListIdx, P.y, P.z, P.w};
+    const bool has[4] = {any, two, four, four};
+    T v[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) id[q] = (kb + q < k1) ? idx[kb + q] : 0u;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) gv[q] = (kb + q < k1) ? g[id[q]] : (T)0;
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-            if (kb + q < k1) s += gv[q];
+    for (int q = 0; q < 4; ++q) {
+        v[q] = g(has[q] ? c[q] : safe);
+        v[4 + q] = g(has[q] && zz ? c[q] + 1u : safe);
     }
+    T s = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) s = has[q & 3] && (q < 4 || zz) ? s + v[q] : s;
+    w = any ? (four ? (T)0.25 : two ? (T)0.5 : (T)1) * (zz ? (T)0.5 : (T)1) : (T)0;
     return s;
 }
-// sum of 2^-k h over the restriction list [k0, k1) (fine children, with
-// log2 of the child's parent count k in bits 28 and up), weights exact
-template <class T>
-__device__ inline T gather_children(const uint32_t* ridx, uint32_t k0, uint32_t k1, const T* h) {
-    constexpr int W = 32;
-    T s = 0;
-    for (uint32_t kb = k0; kb < k1; kb += W) {
-        uint32_t v[W];
-        T hv[W];
+// sum of 2^-k h over the children in the columns e
+template <class T, class Read>
+__device__ inline T sum_children(const uint32_t e[9], uint32_t safe, Read&& h) {
+    T v[27];
 #pragma unroll
-        for (int q = 0; q < W; ++q) v[q] = (kb + q < k1) ? ridx[kb + q] : 0u;
-#pragma unroll
-        for (int q = 0; q < W; ++q) hv[q] = (kb + q < k1) ? h[v[q] & 0x0FFFFFFFu] : (T)0;
-#pragma unroll
-        for (int q = 0; q < W; ++q)
-            if (kb + q < k1) s += ldexp(hv[q], -(int)(v[q] >> 28));
+    for (int q = 0; q < 9; ++q) {
+        const uint32_t b = e[q] & kListIdx, m = e[q] >> 28;
+        const uint32_t b1 = b + (m & 1u), b2 = b1 + ((m >> 1) & 1u);
+        v[3 * q] = h((m & 1u) ? b : safe);
+        v[3 * q + 1] = h((m & 2u) ? b1 : safe);
+        v[3 * q + 2] = h((m & 4u) ? b2 : safe);
     }
+    T s = 0;
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+#pragma unroll
+        for (int z = 0; z < 3; ++z) {
+            const int k = (q / 3 != 1) + (q % 3 != 1) + (z != 1);   // odd coordinates of the child
+            const T weight = k == 0 ? (T)1 : k == 1 ? (T)0.5 : k == 2 ? (T)0.25 : (T)0.125;
+            s = ((e[q] >> (28 + z)) & 1u) ? s + v[3 * q + z] * weight : s;
+        }
     return s;
+}
+__device__ inline void load_kids(const Lists& A, int64_t c, uint32_t e[9]) {
+#pragma unroll
+    for (int q = 0; q < 9; ++q) e[q] = A.kid[kid_slot(c - A.kid0, q)];
+}
+// over the children of vertex c (of level 1 or above)
+template <class T>
+__device__ inline T gather_children(const Lists& A, int64_t c, const T* h) {
+    uint32_t e[9];
+    load_kids(A, c, e);
+    return sum_children<T>(e, 0u, [&](uint32_t y) { return h[y]; });
 }
 
 // ---------------------------------------------------------------- solver
@@ -67,22 +106,20 @@ enum FitScal { S_ABSNEW = 0, S_ALPHA, S_BETA, S_TT, S_RN2, S_THRESH, S_RN2_0, S_
 // g_i = p_i + 2^-k sum_{c in pro(i)} g_c; with UPD the new search direction
 // p_i = z_i + beta p_i first
 template <class T, bool UPD>
-__device__ inline void prolong_at(int64_t i, const uint32_t* ptr, const uint32_t* idx, T* p, const T* z, T* g,
-                                  const double* scal) {
+__device__ inline void prolong_at(int64_t i, const Lists& A, T* p, const T* z, T* g, const double* scal) {
     T pi = p[i];
     if (UPD) {
         pi = z[i] + (T)scal[S_BETA] * pi;
         p[i] = pi;
     }
-    const uint32_t k0 = ptr[i], k1 = ptr[i + 1];
-    const T s = gather_parents(idx, k0, k1, g);
-    T w = (k1 > k0) ? (T)1 / (T)(k1 - k0) : (T)0;
+    T w;
+    const T s = gather_parents<T>(A.par[i], w, 0u, [&](uint32_t j) { return g[j]; });
     g[i] = pi + w * s;
 }
 // h_c += sum_{y in res(c)} 2^-k(y) h_y
 template <class T>
-__device__ inline void restrict_at(int64_t c, const uint32_t* ptr, const uint32_t* ridx, T* h) {
-    h[c] += gather_children(ridx, ptr[c], ptr[c + 1], (const T*)h);
+__device__ inline void restrict_at(int64_t c, const Lists& A, T* h) {
+    h[c] += gather_children(A, c, (const T*)h);
 }
 // x += alpha p; r -= alpha t along the coincidence chain of i; h_i = (D^T r)_i
 __device__ inline void update_dt_at(int64_t i, const uint8_t* finest, const uint32_t* up, float* x, const float* p,
@@ -213,17 +250,9 @@ __device__ inline void scalar_beta_body(const double* part, unsigned np, double*
 // between levels, replacing one launch per level.
 constexpr int kCoarse = 12288;
 constexpr int kCoarseT = 1024;
-// The list offsets of the coarse range are staged in LDS first (one round of
-// loads) when the range holds fewer than kCoarsePtr vertices, so a level
-// waits for its list entries and values only.
-constexpr int kCoarsePtr = 2049;
-__device__ inline bool stage_ptr(const Coarse& C, const uint32_t* ptr, uint32_t* sptr) {
-    const uint32_t base = C.off[C.lc], nptr = C.off[C.L] - base + 1;
-    if (nptr > (uint32_t)kCoarsePtr) return false;
-    for (uint32_t t = threadIdx.x; t < nptr; t += blockDim.x) sptr[t] = ptr[base + t];
-    __syncthreads();
-    return true;
-}
+// vertices per thread whose lists and values a thread loads before the level
+// loop; larger ranges load them level by level
+constexpr int kCoarseHold = 2;
 // level of coarse vertex i (C.lc <= level < C.L)
 __device__ inline int coarse_level(const Coarse& C, uint32_t i) {
     int d = C.lc;
@@ -232,133 +261,98 @@ __device__ inline int coarse_level(const Coarse& C, uint32_t i) {
 }
 
 // g = G p on the coarse levels (with the search direction update when upd).
-// When the range holds at most one vertex per thread, every thread loads its
-// vertex's list and values before the level loop, which then waits only for
-// the LDS values of the level above; the sums keep the same order.
-__device__ inline void prolong_coarse_body(const Coarse& C, const uint32_t* ptr, const uint32_t* idx, float* p,
-                                           const float* z, float* g, const double* scal, int upd, float* sg,
-                                           uint32_t* sptr) {
-    const uint32_t base = C.off[C.lc];
-    if (C.off[C.L] - base <= blockDim.x) {
-        const uint32_t i = base + threadIdx.x;
-        const bool own = i < C.off[C.L];
-        const int lev = own ? coarse_level(C, i) : -1;
-        uint32_t id[8];
-        uint32_t k0 = 0, k1 = 0;
-        float pi = 0.f;
-        if (own) {
-            k0 = ptr[i];
-            k1 = ptr[i + 1];
+// When the range holds at most kCoarseHold vertices per thread, every thread
+// loads its vertices' lists and values before the level loop, which then waits
+// only for the LDS values of the level above; the sums keep the same order.
+__device__ inline void prolong_coarse_body(const Coarse& C, const Lists& A, float* p, const float* z, float* g,
+                                           const double* scal, int upd, float* sg) {
+    const uint32_t base = C.off[C.lc], end = C.off[C.L];
+    const float beta = upd ? (float)scal[S_BETA] : 0.f;
+    auto value = [&](uint32_t i) {
+        float pi = p[i];
+        if (upd) {
+            pi = z[i] + beta * pi;
+            p[i] = pi;
+        }
+        return pi;
+    };
+    auto step = [&](uint32_t i, uint4 P, float pi) {
+        float w;
+        const float s = gather_parents<float>(P, w, base, [&](uint32_t j) { return sg[j - base]; });
+        const float v = pi + w * s;
+        sg[i - base] = v;
+        g[i] = v;
+    };
+    if (end - base <= kCoarseHold * blockDim.x) {
+        int lev[kCoarseHold];
+        uint4 P[kCoarseHold];
+        float pi[kCoarseHold];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) id[q] = (k0 + q < k1) ? idx[k0 + q] : base;
-            pi = p[i];
-            if (upd) {
-                pi = z[i] + (float)scal[S_BETA] * pi;
-                p[i] = pi;
+        for (int v = 0; v < kCoarseHold; ++v) {
+            const uint32_t i = base + threadIdx.x + v * blockDim.x;
+            lev[v] = -1;
+            if (i < end) {
+                lev[v] = coarse_level(C, i);
+                P[v] = A.par[i];
+                pi[v] = value(i);
             }
         }
         for (int d = C.L - 1; d >= C.lc; --d) {
-            if (lev == d) {
-                float s = 0.f;
 #pragma unroll
-                for (int q = 0; q < 8; ++q)
-                    if (k0 + q < k1) s += sg[id[q] - base];
-                float w = (k1 > k0) ? 1.f / (float)(k1 - k0) : 0.f;
-                float v = pi + w * s;
-                sg[i - base] = v;
-                g[i] = v;
-            }
+            for (int v = 0; v < kCoarseHold; ++v)
+                if (lev[v] == d) step(base + threadIdx.x + v * blockDim.x, P[v], pi[v]);
             __syncthreads();
         }
         return;
     }
-    const bool staged = stage_ptr(C, ptr, sptr);
-    const float beta = upd ? (float)scal[S_BETA] : 0.f;
     for (int d = C.L - 1; d >= C.lc; --d) {
-        for (uint32_t i = C.off[d] + threadIdx.x; i < C.off[d + 1]; i += blockDim.x) {
-            float pi = p[i];
-            if (upd) {
-                pi = z[i] + beta * pi;
-                p[i] = pi;
-            }
-            const uint32_t k0 = staged ? sptr[i - base] : ptr[i], k1 = staged ? sptr[i + 1 - base] : ptr[i + 1];
-            float s = 0.f;
-            for (uint32_t kb = k0; kb < k1; kb += 8) {
-                uint32_t id[8];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) id[q] = (kb + q < k1) ? idx[kb + q] : base;
-#pragma unroll
-                for (int q = 0; q < 8; ++q)
-                    if (kb + q < k1) s += sg[id[q] - base];
-            }
-            float w = (k1 > k0) ? 1.f / (float)(k1 - k0) : 0.f;
-            float v = pi + w * s;
-            sg[i - base] = v;
-            g[i] = v;
-        }
+        for (uint32_t i = C.off[d] + threadIdx.x; i < C.off[d + 1]; i += blockDim.x) step(i, A.par[i], value(i));
         __syncthreads();
     }
 }
-// restriction over the coarse levels [C.lc, C.L) (C.lc >= 1); one vertex
-// per thread when the range fits, as in prolong_coarse_body
-__device__ inline void restrict_coarse_body(const Coarse& C, const uint32_t* ptr, const uint32_t* ridx, float* h,
-                                            float* sh, uint32_t* sptr) {
-    const uint32_t base = C.off[C.lc];
-    if (C.off[C.L] - base <= blockDim.x) {
-        const uint32_t c = base + threadIdx.x;
-        const bool own = c < C.off[C.L];
-        const int lev = own ? coarse_level(C, c) : -1;
-        uint32_t v[32];   // child lists: at most 27 entries
-        uint32_t k0 = 0, k1 = 0;
-        float hc0 = 0.f, hlow[32];
-        if (own) {
-            k0 = ptr[c];
-            k1 = ptr[c + 1];
+// restriction over the coarse levels [C.lc, C.L) (C.lc >= 1), as in
+// prolong_coarse_body; the lowest of them reads its children from memory
+__device__ inline void restrict_coarse_body(const Coarse& C, const Lists& A, float* h, float* sh) {
+    const uint32_t base = C.off[C.lc], end = C.off[C.L];
+    auto put = [&](uint32_t c, float hc) {
+        sh[c - base] = hc;
+        h[c] = hc;
+    };
+    if (end - base <= kCoarseHold * blockDim.x) {
+        int lev[kCoarseHold];
+        uint32_t e[kCoarseHold][9];
+        float hc[kCoarseHold];
 #pragma unroll
-            for (int q = 0; q < 32; ++q) v[q] = (k0 + q < k1) ? ridx[k0 + q] : base;
-            hc0 = h[c];
-            // children below the coarse range are final already: read them now
-#pragma unroll
-            for (int q = 0; q < 32; ++q) hlow[q] = (lev == C.lc && k0 + q < k1) ? h[v[q] & 0x0FFFFFFFu] : 0.f;
-        }
-        for (int d = C.lc; d < C.L; ++d) {
-            if (lev == d) {
-                float s = 0.f;
-#pragma unroll
-                for (int q = 0; q < 32; ++q) {
-                    const float hy = (d == C.lc) ? hlow[q] : ((k0 + q < k1) ? sh[(v[q] & 0x0FFFFFFFu) - base] : 0.f);
-                    if (k0 + q < k1) s += ldexpf(hy, -(int)(v[q] >> 28));
-                }
-                const float hc = hc0 + s;
-                sh[c - base] = hc;
-                h[c] = hc;
+        for (int v = 0; v < kCoarseHold; ++v) {
+            const uint32_t c = base + threadIdx.x + v * blockDim.x;
+            lev[v] = -1;
+            if (c < end) {
+                lev[v] = coarse_level(C, c);
+                load_kids(A, c, e[v]);
+                hc[v] = h[c];
             }
+        }
+#pragma unroll
+        for (int v = 0; v < kCoarseHold; ++v)
+            if (lev[v] == C.lc)
+                put(base + threadIdx.x + v * blockDim.x,
+                    hc[v] + sum_children<float>(e[v], base, [&](uint32_t y) { return h[y]; }));
+        __syncthreads();
+        for (int d = C.lc + 1; d < C.L; ++d) {
+#pragma unroll
+            for (int v = 0; v < kCoarseHold; ++v)
+                if (lev[v] == d)
+                    put(base + threadIdx.x + v * blockDim.x,
+                        hc[v] + sum_children<float>(e[v], base, [&](uint32_t y) { return sh[y - base]; }));
             __syncthreads();
         }
         return;
     }
-    const bool staged = stage_ptr(C, ptr, sptr);
     for (int d = C.lc; d < C.L; ++d) {
         for (uint32_t c = C.off[d] + threadIdx.x; c < C.off[d + 1]; c += blockDim.x) {
-            float s = 0.f;
-            const uint32_t k0 = staged ? sptr[c - base] : ptr[c], k1 = staged ? sptr[c + 1 - base] : ptr[c + 1];
-            for (uint32_t kb = k0; kb < k1; kb += 32) {   // child lists: at most 27 entries
-                uint32_t v[32];
-                float hy[32];
-#pragma unroll
-                for (int q = 0; q < 32; ++q) v[q] = (kb + q < k1) ? ridx[kb + q] : base;   // base: in bounds for both reads
-#pragma unroll
-                for (int q = 0; q < 32; ++q) {
-                    const uint32_t y = v[q] & 0x0FFFFFFFu;
-                    hy[q] = (kb + q < k1) ? ((d == C.lc) ? h[y] : sh[y - base]) : 0.f;
-                }
-#pragma unroll
-                for (int q = 0; q < 32; ++q)
-                    if (kb + q < k1) s += ldexpf(hy[q], -(int)(v[q] >> 28));
-            }
-            float hc = h[c] + s;
-            sh[c - base] = hc;
-            h[c] = hc;
+            uint32_t e[9];
+            load_kids(A, c, e);
+            put(c, h[c] + sum_children<float>(e, base, [&](uint32_t y) { return d == C.lc ? h[y] : sh[y - base]; }));
         }
         __syncthreads();
     }
@@ -368,8 +362,9 @@ struct Fit {
     int64_t n = 0;
     int L = 0;
     int64_t off[kMaxLevels + 1] = {0};
-    DBuf<uint32_t> pro_ptr, pro_idx;   // prolongation: coarse parents of each vertex
-    DBuf<uint32_t> res_ptr, res_idx;   // restriction: fine children of each vertex (| log2 count << 28)
+    DBuf<uint4> par;                   // prolongation: coarse parents of each vertex (Lists)
+    DBuf<uint32_t> kid;                // restriction: fine children of each vertex from level 1 on (Lists)
+    int64_t entries = 0;               // parents in all
     DBuf<uint32_t> down, up;           // finest coincident vertex; coincident vertex one level up
     DBuf<uint8_t> finest;
     DBuf<float> invd32;
@@ -387,6 +382,7 @@ struct Fit {
     int graph_chunk = 0;
     int lc = 0;            // first level handled by the one-workgroup coarse kernels
     Coarse coarse{};
+    Lists lists() const { return Lists{par.p, kid.p, L > 1 ? off[1] : n}; }
     ~Fit() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);

@@ -44,15 +44,6 @@ constexpr int kT = kFitT;
 constexpr int kRedBlocks = kFitRed;  // fixed partial count for deterministic sums
 
 // ---------------------------------------------------------------- structure
-__global__ void k_pro_count(int64_t n, const uint8_t* lev, int L, const uint16_t* vx, const uint16_t* vy,
-                            const uint16_t* vz, uint32_t* cnt) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (lev[i] == L - 1) { cnt[i] = 0; return; }
-    int k = (vx[i] & 1) + (vy[i] & 1) + (vz[i] & 1);
-    cnt[i] = 1u << k;
-}
-
 struct LatticeSet {
     const RankWord* lat[kMaxLevels];
     uint32_t D[kMaxLevels];
@@ -66,60 +57,50 @@ __device__ inline uint32_t lat_find(const LatticeSet& S, int d, uint32_t X, uint
     return r == ITS_NONE ? ITS_NONE : S.off[d] + r;
 }
 
-__global__ void k_pro_fill(int64_t n, const uint8_t* lev, int L, const uint16_t* vx, const uint16_t* vy,
-                           const uint16_t* vz, LatticeSet S, const uint32_t* ptr, uint32_t* idx, int* err) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int d = lev[i];
-    if (d == L - 1) return;
-    uint32_t X = vx[i], Y = vy[i], Z = vz[i];
-    uint32_t xs[2] = {X >> 1, (X + 1) >> 1}, ys[2] = {Y >> 1, (Y + 1) >> 1}, zs[2] = {Z >> 1, (Z + 1) >> 1};
-    int nx = (X & 1) ? 2 : 1, ny = (Y & 1) ? 2 : 1, nz = (Z & 1) ? 2 : 1;
-    uint32_t o = ptr[i];
-    for (int c = 0; c < nz; ++c)
-        for (int b = 0; b < ny; ++b)
-            for (int a = 0; a < nx; ++a) {
-                uint32_t j = lat_find(S, d + 1, xs[a], ys[b], zs[c]);
-                if (j == ITS_NONE) { atomicOr(err, 1); j = (uint32_t)i; }
-                idx[o++] = j;
+// Parent and child lists of every vertex by lookups in the lattices above and
+// below; ctl[0] += the parents, ctl[2] |= 1 where one is missing
+__global__ __launch_bounds__(kT) void k_lists(int64_t n, const uint8_t* lev, int L, const uint16_t* vx,
+                                             const uint16_t* vy, const uint16_t* vz, LatticeSet S, uint4* par,
+                                             uint32_t* kid, int* ctl) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int count = 0;
+    if (i < n) {
+        const int d = lev[i];
+        const uint32_t X = vx[i], Y = vy[i], Z = vz[i];
+        uint32_t c[4] = {ITS_NONE, ITS_NONE, ITS_NONE, ITS_NONE};
+        if (d < L - 1) {
+            const uint32_t zodd = Z & 1u;
+            bool ok = true;
+            int q = 0;
+            for (uint32_t b = 0; b <= (Y & 1u); ++b)
+                for (uint32_t a = 0; a <= (X & 1u); ++a) {
+                    uint32_t j = lat_find(S, d + 1, (X >> 1) + a, (Y >> 1) + b, Z >> 1);
+                    if (zodd) ok &= lat_find(S, d + 1, (X >> 1) + a, (Y >> 1) + b, (Z >> 1) + 1) != ITS_NONE;
+                    ok &= j != ITS_NONE;
+                    if (j == ITS_NONE) j = (uint32_t)S.off[d + 1];   // in bounds; the error ends the build
+                    c[q++] = j;
+                }
+            if (!ok) atomicOr(&ctl[2], 1);
+            c[0] |= zodd << 28;
+            count = q << zodd;
+        }
+        par[i] = make_uint4(c[0], c[1], c[2], c[3]);
+        if (d > 0)
+            for (int q = 0; q < 9; ++q) {
+                const uint32_t x = 2 * X + (uint32_t)(q / 3 - 1), y = 2 * Y + (uint32_t)(q % 3 - 1);
+                uint32_t first = 0, mask = 0;
+                for (int z = 2; z >= 0; --z) {
+                    const uint32_t j = lat_find(S, d - 1, x, y, 2 * Z + (uint32_t)(z - 1));
+                    if (j != ITS_NONE) {
+                        first = j;
+                        mask |= 1u << z;
+                    }
+                }
+                kid[kid_slot(i - (int64_t)S.off[1], q)] = first | (mask << 28);
             }
-}
-
-__global__ void k_res_count(int64_t n, const uint32_t* ptr, const uint32_t* idx, uint32_t* cnt) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    for (uint32_t k = ptr[i]; k < ptr[i + 1]; ++k) atomicAdd(&cnt[idx[k]], 1u);
-}
-__global__ void k_res_fill(int64_t n, const uint32_t* ptr, const uint32_t* idx, uint32_t* cursor, uint32_t* ridx) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t b = ptr[i], e = ptr[i + 1];
-    uint32_t lg = __ffs(e - b) - 1;   // log2 of the count
-    for (uint32_t k = b; k < e; ++k) {
-        uint32_t pos = atomicAdd(&cursor[idx[k]], 1u);
-        ridx[pos] = (uint32_t)i | (lg << 28);
     }
-}
-// deterministic order inside each restriction row
-__global__ void k_res_sort(int64_t n, const uint32_t* ptr, uint32_t* ridx) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t b = ptr[i], e = ptr[i + 1];
-    for (uint32_t k = b + 1; k < e; ++k) {
-        uint32_t v = ridx[k];
-        uint32_t key = v & 0x0FFFFFFFu;
-        uint32_t j = k;
-        while (j > b && (ridx[j - 1] & 0x0FFFFFFFu) > key) { ridx[j] = ridx[j - 1]; --j; }
-        ridx[j] = v;
-    }
-}
-
-// the list lengths into ctl[0] (parent entries) and ctl[1] (child entries);
-// error bit 4 when they differ
-__global__ void k_list_sizes(const uint32_t* npro, const uint32_t* nres, int* ctl) {
-    ctl[0] = (int)*npro;
-    ctl[1] = (int)*nres;
-    if (*npro != *nres) ctl[2] |= 4;
+    count = wave_sum(count);
+    if ((threadIdx.x & 63) == 0 && count) atomicAdd(&ctl[0], count);
 }
 
 __global__ void k_updown(int64_t n, const uint8_t* lev, int L, const uint16_t* vx, const uint16_t* vy,
@@ -210,12 +191,12 @@ __global__ void k_invdiag(int64_t n, const unsigned long long* acc, double* d64,
 // g = G p on one level: g_i = p_i + 2^-k sum_{c in pro(i)} g_c.  When upd is
 // set the first pass also forms the new search direction p = z + beta p.
 template <class T, bool UPD>
-__global__ __launch_bounds__(kT) void k_prolong(int64_t b, int64_t e, const uint32_t* ptr, const uint32_t* idx, T* p,
-                                               const T* z, T* g, const double* scal, const int* ctl) {
+__global__ __launch_bounds__(kT) void k_prolong(int64_t b, int64_t e, Lists A, T* p, const T* z, T* g,
+                                               const double* scal, const int* ctl) {
     if (UPD && ctl[0]) return;
     int64_t i = b + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= e) return;
-    prolong_at<T, UPD>(i, ptr, idx, p, z, g, scal);
+    prolong_at<T, UPD>(i, A, p, z, g, scal);
 }
 
 // t = D g and the partials of ||t||^2
@@ -244,28 +225,23 @@ __global__ __launch_bounds__(kT) void k_update_dt(int64_t n, const uint8_t* fine
 
 // h_c += sum_{y in res(c)} 2^-k(y) h_y for the vertices of one level
 template <class T>
-__global__ __launch_bounds__(kT) void k_restrict(int64_t b, int64_t e, const uint32_t* ptr, const uint32_t* ridx, T* h,
-                                                const int* ctl, int check) {
+__global__ __launch_bounds__(kT) void k_restrict(int64_t b, int64_t e, Lists A, T* h, const int* ctl, int check) {
     if (check && ctl[0]) return;
     int64_t c = b + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= e) return;
-    restrict_at<T>(c, ptr, ridx, h);
+    restrict_at<T>(c, A, h);
 }
 
-__global__ __launch_bounds__(kCoarseT) void k_prolong_coarse(Coarse C, const uint32_t* ptr, const uint32_t* idx,
-                                                            float* p, const float* z, float* g, const double* scal,
-                                                            const int* ctl, int upd) {
+__global__ __launch_bounds__(kCoarseT) void k_prolong_coarse(Coarse C, Lists A, float* p, const float* z, float* g,
+                                                            const double* scal, const int* ctl, int upd) {
     if (upd && ctl[0]) return;
     __shared__ float sg[kCoarse];
-    __shared__ uint32_t sptr[kCoarsePtr];
-    prolong_coarse_body(C, ptr, idx, p, z, g, scal, upd, sg, sptr);
+    prolong_coarse_body(C, A, p, z, g, scal, upd, sg);
 }
-__global__ __launch_bounds__(kCoarseT) void k_restrict_coarse(Coarse C, const uint32_t* ptr, const uint32_t* ridx,
-                                                             float* h, const int* ctl, int check) {
+__global__ __launch_bounds__(kCoarseT) void k_restrict_coarse(Coarse C, Lists A, float* h, const int* ctl, int check) {
     if (check && ctl[0]) return;
     __shared__ float sh[kCoarse];
-    __shared__ uint32_t sptr[kCoarsePtr];
-    restrict_coarse_body(C, ptr, ridx, h, sh, sptr);
+    restrict_coarse_body(C, A, h, sh);
 }
 
 // z = M^-1 nr and the partials of nr.nr and nr.z
@@ -341,42 +317,17 @@ Fit* fit_get(its_svo s) {
         S.D[d] = (uint32_t)s->lv[d].R + 1;
         S.off[d] = (uint32_t)s->esum_verts[d];
     }
-    // ctl during the build: [0] parent entries, [1] child entries, [2] error
-    // bits, read back together at the end, the one wait of the build
+    // ctl during the build: [0] parent entries, [2] error bits, read back at
+    // the end, the one wait of the build
     f->ctl.alloc(4);
     ITS_HIP(hipMemsetAsync(f->ctl.p, 0, 4 * sizeof(int), st));
     int* err = f->ctl.p + 2;
-    // prolongation lists: at most 8 parents per vertex; sized by that bound
-    // first, cut to their length once it is known
-    const int64_t cap = std::max<int64_t>(8 * n, 1);
-    f->pro_ptr.alloc(n + 1);
-    hipLaunchKernelGGL(k_pro_count, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, s->vlevel.p, L, s->vx.p, s->vy.p,
-                       s->vz.p, f->pro_ptr.p);
-    ITS_LAUNCH_CHECK();
-    scan_exclusive_u32_async(f->pro_ptr.p, f->pro_ptr.p, n, st, f->pro_ptr.p + n);
-    f->pro_idx.alloc(cap);
-    hipLaunchKernelGGL(k_pro_fill, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, s->vlevel.p, L, s->vx.p, s->vy.p,
-                       s->vz.p, S, f->pro_ptr.p, f->pro_idx.p, err);
-    ITS_LAUNCH_CHECK();
-    // restriction lists (transpose of prolongation)
-    f->res_ptr.alloc(n + 1);
-    ITS_HIP(hipMemsetAsync(f->res_ptr.p, 0, (n + 1) * sizeof(uint32_t), st));
-    hipLaunchKernelGGL(k_res_count, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, f->pro_ptr.p, f->pro_idx.p,
-                       f->res_ptr.p);
-    ITS_LAUNCH_CHECK();
-    scan_exclusive_u32_async(f->res_ptr.p, f->res_ptr.p, n, st, f->res_ptr.p + n);
-    f->res_idx.alloc(cap);
-    {
-        DBuf<uint32_t> cursor(n + 1);
-        ITS_HIP(hipMemcpyAsync(cursor.p, f->res_ptr.p, (n + 1) * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
-        hipLaunchKernelGGL(k_res_fill, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, f->pro_ptr.p, f->pro_idx.p,
-                           cursor.p, f->res_idx.p);
-        ITS_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_res_sort, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, f->res_ptr.p, f->res_idx.p);
-        ITS_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(k_list_sizes, dim3(1), dim3(1), 0, st, (const uint32_t*)f->pro_ptr.p + n,
-                       (const uint32_t*)f->res_ptr.p + n, f->ctl.p);
+    ITS_REQUIRE(n < (int64_t)kListIdx, ITS_E_RANGE, "more than 2^28 vertices in a fit");
+    const int64_t kids = L > 1 ? n - f->off[1] : 0;
+    f->par.alloc(std::max<int64_t>(n, 1));
+    f->kid.alloc(std::max<int64_t>((kids + 63) / 64 * 9 * 64, 1));
+    hipLaunchKernelGGL(k_lists, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, s->vlevel.p, L, s->vx.p, s->vy.p, s->vz.p,
+                       S, f->par.p, f->kid.p, f->ctl.p);
     ITS_LAUNCH_CHECK();
     // coincidence chains
     f->up.alloc(n);
@@ -408,18 +359,9 @@ Fit* fit_get(its_svo s) {
     int info[3] = {0, 0, 0};
     ITS_HIP(hipMemcpyAsync(info, f->ctl.p, sizeof info, hipMemcpyDeviceToHost, st));
     ITS_HIP(hipStreamSynchronize(st));
-    ITS_REQUIRE(info[2] == 0, ITS_E_STATE,
-                (info[2] & 4) ? "restriction size mismatch"
-                              : "octree lattice is inconsistent (missing coarse corner vertex)");
+    ITS_REQUIRE(info[2] == 0, ITS_E_STATE, "octree lattice is inconsistent (missing coarse corner vertex)");
+    f->entries = (int64_t)(uint32_t)info[0];
     ITS_HIP(hipMemsetAsync(f->ctl.p, 0, 4 * sizeof(int), st));   // the solver's flags start cleared
-    // the lists at their length (the bound-sized buffers go back to the stream's cache)
-    for (auto* lst : {&f->pro_idx, &f->res_idx}) {
-        DBuf<uint32_t> exact(std::max<int64_t>((uint32_t)info[0], 1));
-        if (info[0] > 0)
-            ITS_HIP(hipMemcpyAsync(exact.p, lst->p, (size_t)(uint32_t)info[0] * sizeof(uint32_t),
-                                   hipMemcpyDeviceToDevice, st));
-        std::swap(*lst, exact);
-    }
     for (auto* v : {&f->x, &f->r, &f->p, &f->z, &f->t, &f->g, &f->h}) v->alloc(n);
     for (auto* v : {&f->g64, &f->h64, &f->r64, &f->nr64, &f->b64, &f->tmp64}) v->alloc(n);
     f->part.alloc(2 * kRedBlocks);
@@ -437,8 +379,8 @@ void apply_A64(Fit* f, const double* x, double* y, hipStream_t st) {
     for (int d = f->L - 1; d >= 0; --d) {
         int64_t b = f->off[d], e = f->off[d + 1];
         if (e <= b) continue;
-        hipLaunchKernelGGL((k_prolong<double, false>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->pro_ptr.p,
-                           f->pro_idx.p, const_cast<double*>(x), (const double*)nullptr, g, (const double*)nullptr,
+        hipLaunchKernelGGL((k_prolong<double, false>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->lists(),
+                           const_cast<double*>(x), (const double*)nullptr, g, (const double*)nullptr,
                            (const int*)nullptr);
         ITS_LAUNCH_CHECK();
     }
@@ -452,8 +394,8 @@ void apply_AT64(Fit* f, const double* x, double* y, hipStream_t st) {
     for (int d = 1; d < f->L; ++d) {
         int64_t b = f->off[d], e = f->off[d + 1];
         if (e <= b) continue;
-        hipLaunchKernelGGL((k_restrict<double>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->res_ptr.p,
-                           f->res_idx.p, y, (const int*)nullptr, 0);
+        hipLaunchKernelGGL((k_restrict<double>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->lists(), y,
+                           (const int*)nullptr, 0);
         ITS_LAUNCH_CHECK();
     }
 }
@@ -492,8 +434,8 @@ void launch_AT32(Fit* f, hipStream_t st, int do_update, int check) {
     for (int d = 1; d < f->lc; ++d) {
         int64_t b = f->off[d], e = f->off[d + 1];
         if (e <= b) continue;
-        hipLaunchKernelGGL((k_restrict<float>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->res_ptr.p,
-                           f->res_idx.p, f->h.p, f->ctl.p, check);
+        hipLaunchKernelGGL((k_restrict<float>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->lists(), f->h.p,
+                           f->ctl.p, check);
         ITS_LAUNCH_CHECK();
     }
     if (f->lc < f->L) {
@@ -501,8 +443,8 @@ void launch_AT32(Fit* f, hipStream_t st, int do_update, int check) {
         Coarse C = f->coarse;
         if (C.lc == 0) C.lc = 1;
         if (C.lc < C.L) {
-            hipLaunchKernelGGL(k_restrict_coarse, dim3(1), dim3(kCoarseT), 0, st, C, f->res_ptr.p, f->res_idx.p, f->h.p,
-                               f->ctl.p, check);
+            hipLaunchKernelGGL(k_restrict_coarse, dim3(1), dim3(kCoarseT), 0, st, C, f->lists(), f->h.p, f->ctl.p,
+                               check);
             ITS_LAUNCH_CHECK();
         }
     }
@@ -513,15 +455,15 @@ void launch_iteration(Fit* f, hipStream_t st) {
     const int64_t n = f->n;
     const unsigned nb = red_blocks(n);
     if (f->lc < f->L) {
-        hipLaunchKernelGGL(k_prolong_coarse, dim3(1), dim3(kCoarseT), 0, st, f->coarse, f->pro_ptr.p, f->pro_idx.p,
-                           f->p.p, (const float*)f->z.p, f->g.p, (const double*)f->scal.p, (const int*)f->ctl.p, 1);
+        hipLaunchKernelGGL(k_prolong_coarse, dim3(1), dim3(kCoarseT), 0, st, f->coarse, f->lists(), f->p.p,
+                           (const float*)f->z.p, f->g.p, (const double*)f->scal.p, (const int*)f->ctl.p, 1);
         ITS_LAUNCH_CHECK();
     }
     for (int d = f->lc - 1; d >= 0; --d) {
         int64_t b = f->off[d], e = f->off[d + 1];
         if (e <= b) continue;
-        hipLaunchKernelGGL((k_prolong<float, true>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->pro_ptr.p,
-                           f->pro_idx.p, f->p.p, (const float*)f->z.p, f->g.p, (const double*)f->scal.p,
+        hipLaunchKernelGGL((k_prolong<float, true>), dim3(blocks_for(e - b, kT)), dim3(kT), 0, st, b, e, f->lists(), f->p.p,
+                           (const float*)f->z.p, f->g.p, (const double*)f->scal.p,
                            (const int*)f->ctl.p);
         ITS_LAUNCH_CHECK();
     }
@@ -596,15 +538,10 @@ __global__ void k_dual_u(int64_t n, const double* lam, const double* invd, doubl
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) u[i] = lam[i] / invd[i];
 }
-__global__ void k_dual_restrict(int64_t n, const uint32_t* ptr, const uint32_t* ridx, const double* u, double* W) {
+__global__ void k_dual_restrict(int64_t n, Lists A, const double* u, double* W) {
     int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= n) return;
-    double s = 0;
-    for (uint32_t k = ptr[c]; k < ptr[c + 1]; ++k) {
-        uint32_t v = ridx[k];
-        s += u[v & 0x0FFFFFFFu] / (double)(1u << (v >> 28));
-    }
-    W[c] = u[c] - s;
+    W[c] = u[c] - (c >= A.kid0 ? gather_children(A, c, u) : 0.0);
 }
 __global__ void k_group_count(int64_t n, const uint32_t* down, uint32_t* cnt) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -631,8 +568,8 @@ void warm_dual(its_svo s, const double* d_lam, double* d_w) {
     ITS_HIP(hipMemsetAsync(cnt.p, 0, n * sizeof(uint32_t), st));
     hipLaunchKernelGGL(k_dual_u, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, d_lam, (const double*)f->invd64.p, u.p);
     ITS_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_dual_restrict, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, (const uint32_t*)f->res_ptr.p,
-                       (const uint32_t*)f->res_idx.p, (const double*)u.p, W.p);
+    hipLaunchKernelGGL(k_dual_restrict, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, f->lists(), (const double*)u.p,
+                       W.p);
     ITS_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_group_count, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, (const uint32_t*)f->down.p, cnt.p);
     ITS_LAUNCH_CHECK();
@@ -693,13 +630,11 @@ void lscg_structure(its_svo s, its_lscg_structure* out) {
     ITS_LAUNCH_CHECK();
     unsigned long long nnz = 0;
     ITS_HIP(hipMemcpyAsync(&nnz, tot.p, sizeof nnz, hipMemcpyDeviceToHost, st));
-    uint32_t entries = 0;
-    ITS_HIP(hipMemcpyAsync(&entries, f->pro_ptr.p + n, sizeof entries, hipMemcpyDeviceToHost, st));
     ITS_HIP(hipStreamSynchronize(st));
     its_lscg_structure S{};
     S.n = n;
     S.nnz = (int64_t)nnz;
-    S.parent_entries = (int64_t)entries;
+    S.parent_entries = f->entries;
     S.levels = f->L;
     S.block_levels = f->L - f->lc;
     S.bytes_assembled_per_iteration = 16.0 * (double)nnz + 72.0 * (double)n;
@@ -707,7 +642,7 @@ void lscg_structure(its_svo s, its_lscg_structure* out) {
     // its index and gather (12 B); the update of x, r along the chains, h
     // (33 B); restriction offset and h r/w (12 B); preconditioner h, 1/d, z
     // (12 B).  Per parent entry: index and value, once down and once up (16 B).
-    S.bytes_matrix_free_per_iteration = 89.0 * (double)n + 16.0 * (double)entries;
+    S.bytes_matrix_free_per_iteration = 89.0 * (double)n + 16.0 * (double)f->entries;
     *out = S;
 }
 
@@ -740,12 +675,18 @@ void lscg_solve(its_svo s, const double* d_b, double* d_lambda, double tol, int6
     } else {
         const double inner_tol = 1e-3;
         for (;;) {
-            apply_A64(f, d_lambda, f->tmp64.p, st);
-            hipLaunchKernelGGL(k_sub64, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, d_b, f->tmp64.p, f->r64.p);
-            ITS_LAUNCH_CHECK();
+            double rn2 = rhs2;
+            if (!warm && outer == 0) {
+                // lambda = 0: the residual is b, and its normal residual A^T b is known
+                ITS_HIP(hipMemcpyAsync(f->r64.p, d_b, n * sizeof(double), hipMemcpyDeviceToDevice, st));
+            } else {
+                apply_A64(f, d_lambda, f->tmp64.p, st);
+                hipLaunchKernelGGL(k_sub64, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, d_b, f->tmp64.p, f->r64.p);
+                ITS_LAUNCH_CHECK();
+                apply_AT64(f, f->r64.p, f->nr64.p, st);
+                rn2 = dot64(f, f->nr64.p, f->nr64.p, st);
+            }
             r_current = true;
-            apply_AT64(f, f->r64.p, f->nr64.p, st);
-            double rn2 = dot64(f, f->nr64.p, f->nr64.p, st);
             rel = std::sqrt(rn2 / rhs2);
             if (rel0 < 0) rel0 = rel;
             if (rel < tol || iters >= max_iter) break;

@@ -37,7 +37,8 @@ struct MeshDesc {
     int64_t off[kMaxLevels + 1];
     Coarse coarse;    // prolongation over the coarse levels (lc < L)
     Coarse rcoarse;   // restriction over the coarse levels (from level 1 on)
-    const uint32_t *pro_ptr, *pro_idx, *res_ptr, *res_idx, *down, *up;
+    Lists lists;
+    const uint32_t *down, *up;
     const uint8_t* finest;
     const float* invd32;
     const double* b;
@@ -67,14 +68,13 @@ __global__ __launch_bounds__(kT) void kb_prolong32(const uint32_t* plan, const M
     if (M.ctl[0]) return;
     const int64_t i = M.off[d] + B.lb * kT + threadIdx.x;
     if (i >= M.off[d + 1]) return;
-    prolong_at<float, true>(i, M.pro_ptr, M.pro_idx, M.p, M.z, M.g, M.scal);
+    prolong_at<float, true>(i, M.lists, M.p, M.z, M.g, M.scal);
 }
 __global__ __launch_bounds__(kCoarseT) void kb_prolong_coarse(const uint32_t* plan, const MeshDesc* descs) {
     const MeshDesc& M = *resolve(plan, descs).D;
     if (M.ctl[0]) return;
     __shared__ float sg[kCoarse];
-    __shared__ uint32_t sptr[kCoarsePtr];
-    prolong_coarse_body(M.coarse, M.pro_ptr, M.pro_idx, M.p, M.z, M.g, M.scal, 1, sg, sptr);
+    prolong_coarse_body(M.coarse, M.lists, M.p, M.z, M.g, M.scal, 1, sg);
 }
 __global__ __launch_bounds__(kT) void kb_apply_down(const uint32_t* plan, const MeshDesc* descs) {
     const Blk B = resolve(plan, descs);
@@ -103,14 +103,13 @@ __global__ __launch_bounds__(kT) void kb_restrict32(const uint32_t* plan, const 
     if (M.ctl[0]) return;
     const int64_t c = M.off[d] + B.lb * kT + threadIdx.x;
     if (c >= M.off[d + 1]) return;
-    restrict_at<float>(c, M.res_ptr, M.res_idx, M.h);
+    restrict_at<float>(c, M.lists, M.h);
 }
 __global__ __launch_bounds__(kCoarseT) void kb_restrict_coarse(const uint32_t* plan, const MeshDesc* descs) {
     const MeshDesc& M = *resolve(plan, descs).D;
     if (M.ctl[0]) return;
     __shared__ float sh[kCoarse];
-    __shared__ uint32_t sptr[kCoarsePtr];
-    restrict_coarse_body(M.rcoarse, M.res_ptr, M.res_idx, M.h, sh, sptr);
+    restrict_coarse_body(M.rcoarse, M.lists, M.h, sh);
 }
 __global__ __launch_bounds__(kT) void kb_precond(const uint32_t* plan, const MeshDesc* descs) {
     const Blk B = resolve(plan, descs);
@@ -169,7 +168,7 @@ __global__ __launch_bounds__(kT) void kb_prolong64(const uint32_t* plan, const M
     if (!*M.act) return;
     const int64_t i = M.off[d] + B.lb * kT + threadIdx.x;
     if (i >= M.off[d + 1]) return;
-    prolong_at<double, false>(i, M.pro_ptr, M.pro_idx, M.lam, (const double*)nullptr, M.g64, (const double*)nullptr);
+    prolong_at<double, false>(i, M.lists, M.lam, (const double*)nullptr, M.g64, (const double*)nullptr);
 }
 // r64 = b - D g64
 __global__ __launch_bounds__(kT) void kb_residual64(const uint32_t* plan, const MeshDesc* descs) {
@@ -178,6 +177,14 @@ __global__ __launch_bounds__(kT) void kb_residual64(const uint32_t* plan, const 
     if (!*M.act) return;
     const int64_t i = B.lb * kT + threadIdx.x;
     if (i < M.n) M.r64[i] = M.b[i] - M.g64[M.down[i]];
+}
+// r64 = b, the residual at lambda = 0
+__global__ __launch_bounds__(kT) void kb_cold64(const uint32_t* plan, const MeshDesc* descs) {
+    const Blk B = resolve(plan, descs);
+    const MeshDesc& M = *B.D;
+    if (!*M.act) return;
+    const int64_t i = B.lb * kT + threadIdx.x;
+    if (i < M.n) M.r64[i] = M.b[i];
 }
 // A^T of b (into h64, which = 0) or of r64 (into nr64, which = 1)
 __device__ inline double* at64_dst(const MeshDesc& M, int which) { return which ? M.nr64 : M.h64; }
@@ -194,7 +201,7 @@ __global__ __launch_bounds__(kT) void kb_restrict64(const uint32_t* plan, const 
     if (!*M.act) return;
     const int64_t c = M.off[d] + B.lb * kT + threadIdx.x;
     if (c >= M.off[d + 1]) return;
-    restrict_at<double>(c, M.res_ptr, M.res_idx, at64_dst(M, which));
+    restrict_at<double>(c, M.lists, at64_dst(M, which));
 }
 // binary64 dot products: 0 h64.h64, 1 b.b, 2 nr64.nr64, 3 r64.r64
 __device__ inline const double* dot_vec(const MeshDesc& M, int pair) {
@@ -266,10 +273,7 @@ static void many_prepare(ManySolve& ms, const std::vector<its_svo>& svos, hipStr
         D.coarse = f->coarse;
         D.rcoarse = f->coarse;
         if (D.rcoarse.lc == 0) D.rcoarse.lc = 1;
-        D.pro_ptr = f->pro_ptr.p;
-        D.pro_idx = f->pro_idx.p;
-        D.res_ptr = f->res_ptr.p;
-        D.res_idx = f->res_idx.p;
+        D.lists = f->lists();
         D.down = f->down.p;
         D.up = f->up.p;
         D.finest = f->finest.p;
@@ -443,6 +447,7 @@ void lscg_solve_many(ManySolve& ms, const std::vector<its_svo>& svos, double tol
         ITS_LAUNCH_CHECK();
     }
     const double inner_tol = 1e-3;
+    bool cold = !warm;
     for (;;) {
         bool any = false;
         for (int m = 0; m < M; ++m) {
@@ -452,10 +457,18 @@ void lscg_solve_many(ManySolve& ms, const std::vector<its_svo>& svos, double tol
         if (!any) break;
         // binary64 residual and normal residual of the refining octrees
         upload(ms.act.p, act, st);
-        many_residual(L);
-        many_AT64(L, 1);
-        many_dot(L, 2, 0);
-        read_out();
+        if (cold) {
+            // lambda = 0: the residual is b, and its normal residual A^T b is known
+            hipLaunchKernelGGL(kb_cold64, dim3(ms.plan->all.count), dim3(kT), 0, st, L.at(ms.plan->all), L.descs());
+            ITS_LAUNCH_CHECK();
+            for (int m = 0; m < M; ++m) outv[2 * m] = S[m].rhs2;
+            cold = false;
+        } else {
+            many_residual(L);
+            many_AT64(L, 1);
+            many_dot(L, 2, 0);
+            read_out();
+        }
         any = false;
         for (int m = 0; m < M; ++m) {
             State& s = S[m];
