@@ -20,9 +20,9 @@
 // become the next layer's operand.  The backward pass uses the same layouts:
 // dH^T = W . dZ^T gives the lane's row again, and the weight gradients
 // dW = H^T dZ (reduction over the 32 rows of the tile) accumulate in MFMA
-// registers across all tiles of the wavefront.  Each wavefront writes its
-// gradient once; a second kernel sums the wavefront partials in a fixed
-// order, so gradients are deterministic.
+// registers across all tiles of the wavefront.  Each workgroup writes its
+// gradient once; a second kernel sums the partials in a fixed order, so
+// gradients are deterministic.
 #include <algorithm>
 #include <cmath>
 #include <random>
@@ -53,10 +53,9 @@ constexpr int W1S = IN + 8;
 // first two layers (the third stays in registers).
 template <bool TRAIN> constexpr int waves() { return TRAIN ? 2 : 4; }
 template <bool TRAIN>
-struct Tile {
+struct Tile {   // inference: the second layer's outputs take the place of the first's, which it has read by then
     __bf16 x[kRows * XS];
     __bf16 h1[kRows * HS];
-    __bf16 h2[kRows * HS];
 };
 template <>
 struct Tile<true> {
@@ -91,9 +90,33 @@ __device__ inline bf16x8 col8(const __bf16* p, int stride) {
     for (int j = 0; j < 8; ++j) v[j] = p[j * stride];
     return v;
 }
-__device__ inline float gelu(float z) { return 0.5f * z * (1.f + erff(z * 0.70710678118654752f)); }
+// erfc(|z| / sqrt 2) without branches: 2^(a R(a)) with a = |z|, R of degree 8
+// fitted here by weighted least squares on Chebyshev nodes of [0, 8] (Lawson
+// iterations; within 2.3e-9 before rounding, 1.24e-7 in binary32, as 1 + erff
+// is, 1.22e-7).  10 instructions for about 40 of erff, which runs both of its
+// ranges in a wavefront whose lanes fall on both sides: 300,000 rows forward
+// 59.6 -> 41.2 us, bound by these instructions.
+__device__ inline float erfc_abs(float z) {
+    const float a = fminf(fabsf(z), 8.f);
+    float r = 5.128700877e-07f;
+    r = fmaf(r, a, -9.560338185e-06f);
+    r = fmaf(r, a, 7.497437764e-05f);
+    r = fmaf(r, a, -2.843491093e-04f);
+    r = fmaf(r, a, 1.499301743e-05f);
+    r = fmaf(r, a, 6.931117736e-03f);
+    r = fmaf(r, a, -5.243476480e-02f);
+    r = fmaf(r, a, -4.592214525e-01f);
+    r = fmaf(r, a, -1.151104212e+00f);
+    return __builtin_amdgcn_exp2f(r * a);
+}
+// 2 GELU(z) = z + |z| erf(|z| / sqrt 2)
+__device__ inline float gelu2(float z) { return fmaf(fabsf(z), 1.f - erfc_abs(z), z); }
+__device__ inline float gelu(float z) { return 0.5f * gelu2(z); }
 __device__ inline float gelu_d(float z) {
-    return 0.5f * (1.f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
+    // 2^(-z^2 log2(e) / 2) is the exponential of the normal density
+    const float E = erfc_abs(z);
+    return fmaf(z, 0.39894228040143268f * __builtin_amdgcn_exp2f(-0.72134752044448170f * z * z),
+                0.5f * (z >= 0.f ? 2.f - E : E));
 }
 __device__ inline void wave_sync() {
     // LDS written by some lanes is read by other lanes of the same wavefront
@@ -104,15 +127,19 @@ __device__ inline void wave_sync() {
 // output n of the 32 held by a lane: m = 32-block, q, t: n = 32m + 8q + 4(lane/32) + t
 __device__ inline int out_n(int m, int q, int t, int half) { return 32 * m + 8 * q + 4 * half + t; }
 
+// Inference keeps 2 GELU in its tiles and half of every weight that follows
+// one: the same products, powers of two apart, and an instruction less per
+// activation.
 template <bool TRAIN>
 __device__ void load_weights(Shared<TRAIN>& S, const float* P) {
+    constexpr float scale = TRAIN ? 1.f : 0.5f;
     for (int i = threadIdx.x; i < IN * H; i += blockDim.x) {
         const int k = i / H, n = i % H;
         S.w1t[n * W1S + k] = (__bf16)P[oW1 + i];
     }
     for (int i = threadIdx.x; i < H * H; i += blockDim.x) {
         const int k = i / H, n = i % H;
-        const __bf16 a = (__bf16)P[oW2 + i], b = (__bf16)P[oW3 + i];
+        const __bf16 a = (__bf16)(scale * P[oW2 + i]), b = (__bf16)(scale * P[oW3 + i]);
         S.w2t[n * HS + k] = a;
         S.w3t[n * HS + k] = b;
         if (TRAIN) {
@@ -124,26 +151,36 @@ __device__ void load_weights(Shared<TRAIN>& S, const float* P) {
         S.b1[i] = P[oB1 + i];
         S.b2[i] = P[oB2 + i];
         S.b3[i] = P[oB3 + i];
-        S.w4[i] = (float)(__bf16)P[oW4 + i];
+        S.w4[i] = scale * (float)(__bf16)P[oW4 + i];
     }
     if (threadIdx.x == 0) S.b4 = P[oB4];
     __syncthreads();
 }
 
+// a lane's 32 biases, the accumulators' start
+__device__ inline f32x16 bias16(const float* b, int m, int half) {
+    f32x16 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[4 * q + t] = b[out_n(m, q, t, half)];
+    return v;
+}
 // layer with K = 64 inputs from LDS tile `hin` (row-major), weights W^T `wt`
-__device__ inline void layer64(const __bf16* wt, const __bf16* hin, int lane, f32x16 z[2]) {
+__device__ inline void layer64(const __bf16* wt, const float* b, const __bf16* hin, int lane, f32x16 z[2]) {
     const int r = lane & 31, half = lane >> 5;
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
-        f32x16 acc = {};
+        f32x16 acc = bias16(b, m, half);
 #pragma unroll
         for (int s = 0; s < 4; ++s)
             acc = mfma32(ld8(wt + (32 * m + r) * HS + 16 * s + 8 * half), ld8(hin + r * HS + 16 * s + 8 * half), acc);
         z[m] = acc;
     }
 }
-// add bias; store GELU(z) to the row-major tile `hout` (bf16); z keeps z + b
-__device__ inline void bias_gelu_store(f32x16 z[2], const float* b, __bf16* hout, int lane) {
+// GELU(z) (inference: twice that) to the row-major tile `hout` (bf16)
+template <bool TRAIN>
+__device__ inline void gelu_store(const f32x16 z[2], __bf16* hout, int lane) {
     const int r = lane & 31, half = lane >> 5;
 #pragma unroll
     for (int m = 0; m < 2; ++m)
@@ -151,10 +188,8 @@ __device__ inline void bias_gelu_store(f32x16 z[2], const float* b, __bf16* hout
         for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const int n = out_n(m, q, t, half);
-                const float v = z[m][4 * q + t] + b[n];
-                z[m][4 * q + t] = v;
-                if (hout) hout[r * HS + n] = (__bf16)gelu(v);
+                const float v = z[m][4 * q + t];
+                hout[r * HS + out_n(m, q, t, half)] = (__bf16)(TRAIN ? gelu(v) : gelu2(v));
             }
 }
 // keep / reload a lane's 32 pre-activations (binary32 tile, row-major)
@@ -241,7 +276,7 @@ __device__ inline float half_sum(float v) {
 // TRAIN = false: y[row] = net(x[row]) for rows < n.
 // TRAIN = true: also the squared-error loss against t and its gradient with
 // respect to every parameter, scaled by gscale (2/B for a mean over B rows),
-// written as one partial per wavefront: part[wave][NP + 1] (last: loss sum).
+// written as one partial per workgroup: part[block][NP + 1] (last: loss sum).
 template <bool TRAIN>
 __global__ __launch_bounds__(64 * waves<TRAIN>()) void k_mlp(const float* P, const uint16_t* X, const float* T,
                                                              int64_t n, float gscale, float* Y, float* part) {
@@ -249,6 +284,9 @@ __global__ __launch_bounds__(64 * waves<TRAIN>()) void k_mlp(const float* P, con
     load_weights<TRAIN>(S, P);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 31, half = lane >> 5;
     Tile<TRAIN>& Wt = S.wv[w];
+    __bf16* h2;
+    if constexpr (TRAIN) h2 = Wt.h2;
+    else h2 = Wt.h1;
     const int64_t wid = (int64_t)blockIdx.x * waves<TRAIN>() + w, nw = (int64_t)gridDim.x * waves<TRAIN>();
     const int64_t tiles = (n + kRows - 1) / kRows;
 
@@ -280,16 +318,17 @@ __global__ __launch_bounds__(64 * waves<TRAIN>()) void k_mlp(const float* P, con
         f32x16 z1[2], z2[2], z3[2];
 #pragma unroll
         for (int m = 0; m < 2; ++m)
-            z1[m] = mfma32(ld8(S.w1t + (32 * m + r) * W1S + 8 * half), ld8(Wt.x + r * XS + 8 * half), f32x16{});
-        bias_gelu_store(z1, S.b1, Wt.h1, lane);
+            z1[m] = mfma32(ld8(S.w1t + (32 * m + r) * W1S + 8 * half), ld8(Wt.x + r * XS + 8 * half),
+                           bias16(S.b1, m, half));
+        gelu_store<TRAIN>(z1, Wt.h1, lane);
         if constexpr (TRAIN) z_store(z1, Wt.z1, lane);
         wave_sync();
-        layer64(S.w2t, Wt.h1, lane, z2);
-        bias_gelu_store(z2, S.b2, Wt.h2, lane);
+        layer64(S.w2t, S.b2, Wt.h1, lane, z2);
+        wave_sync();
+        gelu_store<TRAIN>(z2, h2, lane);
         if constexpr (TRAIN) z_store(z2, Wt.z2, lane);
         wave_sync();
-        layer64(S.w3t, Wt.h2, lane, z3);
-        bias_gelu_store(z3, S.b3, nullptr, lane);
+        layer64(S.w3t, S.b3, h2, lane, z3);
         // output layer in binary32; training keeps h3 in the row-reduction tile
         float yp = 0.f;
 #pragma unroll
@@ -299,8 +338,8 @@ __global__ __launch_bounds__(64 * waves<TRAIN>()) void k_mlp(const float* P, con
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const int n = out_n(m, q, t, half);
-                    const float h = gelu(z3[m][4 * q + t]);
-                    yp += h * S.w4[n];
+                    const float h = TRAIN ? gelu(z3[m][4 * q + t]) : gelu2(z3[m][4 * q + t]);
+                    yp = fmaf(h, S.w4[n], yp);
                     if constexpr (TRAIN) Wt.fs[r * H + n] = h;
                 }
         const float y = yp + __shfl_xor(yp, 32) + S.b4;
@@ -363,41 +402,64 @@ __global__ __launch_bounds__(64 * waves<TRAIN>()) void k_mlp(const float* P, con
         }
     }
     if constexpr (!TRAIN) return;
-    float* out = part + wid * (NP + 1);
-    {
-        const int c16 = lane & 15, g = lane >> 4;
+    if constexpr (TRAIN) {
+        // The workgroup's two wavefronts add up in LDS (the second's tile holds
+        // its NP + 1 sums) and write one partial.
+        static_assert(waves<true>() == 2 && sizeof(Tile<true>) >= (NP + 1) * sizeof(float), "gradient fits the tile");
+        __syncthreads();   // both are done with their tiles
+        float* mine = reinterpret_cast<float*>(&S.wv[1]);
+        float* out = part + (int64_t)blockIdx.x * (NP + 1);
+        auto put = [&](int o, float v) {
+            if (w == 1) mine[o] = v;
+            else out[o] = v + mine[o];
+        };
+        auto store = [&]() {
+            const int c16 = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+            for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[oW1 + (4 * g + i) * H + 16 * c + c16] = g1[c][i];
-    }
+                for (int i = 0; i < 4; ++i) put(oW1 + (4 * g + i) * H + 16 * c + c16, g1[c][i]);
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
+            for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+                for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int k = 32 * m + 8 * (i / 4) + 4 * half + (i % 4), nn = 32 * c + r;
-                out[oW2 + k * H + nn] = g2[m][c][i];
-                out[oW3 + k * H + nn] = g3[m][c][i];
+                    for (int i = 0; i < 16; ++i) {
+                        const int k = 32 * m + 8 * (i / 4) + 4 * half + (i % 4), nn = 32 * c + r;
+                        put(oW2 + k * H + nn, g2[m][c][i]);
+                        put(oW3 + k * H + nn, g3[m][c][i]);
+                    }
+            put(oB1 + lane, gb1);
+            put(oB2 + lane, gb2);
+            put(oB3 + lane, gb3);
+            put(oW4 + lane, gw4);
+            const float sb4 = half_sum(gb4), sl = half_sum(loss);
+            if (lane == 0) {
+                put(oB4, sb4);
+                put(NP, sl);
             }
-    out[oB1 + lane] = gb1;
-    out[oB2 + lane] = gb2;
-    out[oB3 + lane] = gb3;
-    out[oW4 + lane] = gw4;
-    const float sb4 = half_sum(gb4), sl = half_sum(loss);
-    if (lane == 0) {
-        out[oB4] = sb4;
-        out[NP] = sl;
+        };
+        if (w == 1) store();
+        __syncthreads();
+        if (w == 0) store();
     }
 }
 
-// g[p] = sum over wavefronts of part[w][p], fixed order
-__global__ void k_sum_parts(const float* part, int64_t nw, float* g) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > NP) return;
+// g[p] = sum over the workgroups of part[b][p], in a fixed order: 64
+// parameters a block, 16 threads a parameter each adding every 16th partial,
+// then those 16 in turn.  One thread a parameter waited for 128 reads in a
+// row: 30 us.
+constexpr int kSumP = 64, kSumT = 16;
+__global__ __launch_bounds__(kSumP * kSumT) void k_sum_parts(const float* part, int64_t nb, float* g) {
+    __shared__ float sh[kSumT][kSumP];
+    const int q = threadIdx.x % kSumP, c = threadIdx.x / kSumP, p = blockIdx.x * kSumP + q;
     float s = 0.f;
-    for (int64_t w = 0; w < nw; ++w) s += part[w * (NP + 1) + p];
+    if (p <= NP)
+        for (int64_t b = c; b < nb; b += kSumT) s += part[b * (NP + 1) + p];
+    sh[c][q] = s;
+    __syncthreads();
+    if (c != 0 || p > NP) return;
+    for (int k = 1; k < kSumT; ++k) s += sh[k][q];
     g[p] = s;
 }
 
@@ -471,13 +533,15 @@ void mlp_forward(Mlp& m, const uint16_t* d_x, int64_t n, float* d_y, hipStream_t
 // gradient of mean((y - t)^2) into m.g (NP values, then the loss sum)
 void mlp_grad(Mlp& m, const uint16_t* d_x, const float* d_t, int64_t n, hipStream_t st) {
     ITS_REQUIRE(n > 0, ITS_E_INVALID, "empty batch");
-    const unsigned grid = mlp_grid(n, waves<true>(), 64);
-    const int64_t nw = (int64_t)grid * waves<true>();
-    m.part.ensure(nw * (NP + 1));
+    // one workgroup per CU, which its LDS fills (16,384 rows are 512 tiles, two
+    // a workgroup; on 64 workgroups 111 us)
+    const unsigned grid = mlp_grid(n, waves<true>(), (int64_t)m.ctx->prop.multiProcessorCount);
+    m.part.ensure((int64_t)grid * (NP + 1));
     hipLaunchKernelGGL(k_mlp<true>, dim3(grid), dim3(64 * waves<true>()), 0, st, (const float*)m.P.p, d_x, d_t, n, 2.f / (float)n,
                        (float*)nullptr, m.part.p);
     ITS_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_sum_parts, dim3((NP + 1 + 255) / 256), dim3(256), 0, st, (const float*)m.part.p, nw, m.g.p);
+    hipLaunchKernelGGL(k_sum_parts, dim3((NP + kSumP) / kSumP), dim3(kSumP * kSumT), 0, st, (const float*)m.part.p,
+                       (int64_t)grid, m.g.p);
     ITS_LAUNCH_CHECK();
 }
 

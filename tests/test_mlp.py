@@ -123,6 +123,42 @@ def test_gradient_matches_oracle(ctx, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 33, 64, 16389, 33000])
+def test_gradient_at_workgroup_edges(ctx, n):
+    """One tile, a second wavefront with a ragged tile or none, and one more
+    tile than the workgroups' wavefronts: the same bound as above."""
+    import torch
+    print(f"[mlp grad edges] n={n}", flush=True)
+    net, p = _net(ctx, 13)
+    xb, t = _data(14, n)
+    dx, dt = _dev(xb.view(np.int16), torch), _dev(t, torch)
+    g, loss = net.grad_device(dx.data_ptr(), dt.data_ptr(), n)
+    g2, loss2 = net.grad_device(dx.data_ptr(), dt.data_ptr(), n)
+    assert np.array_equal(g, g2) and loss == loss2
+    lr, gr, _ = M.loss_and_grad(p, M.bf16_value(xb), t, mimic=True)
+    assert abs(loss - lr) <= 1e-4 * lr
+    assert np.linalg.norm(g - gr) <= 2e-3 * np.linalg.norm(gr)
+    net.close()
+
+
+@pytest.mark.gpu
+def test_forward_far_activations(ctx):
+    """Pre-activations far into both tails of GELU (0 and the identity)."""
+    import torch
+    net, p = _net(ctx, 15)
+    xb, _ = _data(16, 4001)
+    x = M.bf16_bits((M.bf16_value(xb) * 40).astype(np.float32))
+    dx = _dev(x.view(np.int16), torch)
+    dy = torch.empty(4001, device="cuda", dtype=torch.float32)
+    net.forward_device(dx.data_ptr(), 4001, dy.data_ptr())
+    torch.cuda.synchronize()
+    yr, _ = M.forward(p, M.bf16_value(x), mimic=True)
+    err = np.abs(dy.cpu().numpy() - yr)
+    assert np.quantile(err, 0.999) <= 1e-5 * np.abs(yr).max()
+    net.close()
+
+
+@pytest.mark.gpu
 def test_training_reduces_loss(ctx):
     import torch
     net, _ = _net(ctx, 11)
