@@ -1,6 +1,7 @@
 // Internal object layout of the ITS gfx950 library (not part of the C ABI).
 #pragma once
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -25,7 +26,24 @@ struct McScratch;
 
 }  // namespace its
 
+namespace its {
+// Pinned staging of a context's copies to pageable host memory: two chunks,
+// made by the first copy that needs them, freed with the context.
+struct HostStage {
+    std::mutex mu;
+    char* buf = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    bool failed = false;   // no pinned memory: plain copies
+    ~HostStage() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+        if (buf) (void)hipHostFree(buf);
+    }
+};
+}  // namespace its
+
 struct its_ctx_s {
+    its::HostStage stage;
     int device = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -111,6 +129,8 @@ namespace its {
 inline void lambda_changing(its_svo s) { ++s->lambda_version; }
 // tunables (capi.hip)
 int64_t tune_get(int key);
+// device to caller memory; returns when the bytes are there (capi.hip)
+void copy_out(its_ctx ctx, void* h, const void* d, size_t bytes, hipStream_t st);
 // svo.hip
 void svo_build(its_svo s, const double* d_tris, int64_t T);
 void svo_from_vertices(its_svo s, const double* xyz, const uint32_t* owner, int64_t n, const double* node_width,

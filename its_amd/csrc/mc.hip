@@ -334,8 +334,7 @@ void mc_lattice(its_svo s, const double origin[3], const double width[3], const 
     int64_t dims[3] = {res[0] + 1, res[1] + 1, res[2] + 1};
     int64_t np = dims[0] * dims[1] * dims[2];
     lattice_values(s, origin, width, res, s->mc_lat, st);
-    ITS_HIP(hipMemcpyAsync(h_vals, s->mc_lat.p, np * sizeof(float), hipMemcpyDeviceToHost, st));
-    ITS_HIP(hipStreamSynchronize(st));
+    copy_out(s->ctx, h_vals, s->mc_lat.p, np * sizeof(float), st);
 }
 
 void mc_extract(its_svo s, const double origin[3], const double width[3], const int res[3], double iso, float* h_tri,
@@ -407,7 +406,7 @@ void mc_extract(its_svo s, const double origin[3], const double width[3], const 
             emit();
             ITS_HIP(hipEventRecord(ev[2], st));
         }
-        ITS_HIP(hipMemcpyAsync(h_tri, s->mc_soup.p, 3 * total * sizeof(float), hipMemcpyDeviceToHost, st));
+        copy_out(s->ctx, h_tri, s->mc_soup.p, 3 * total * sizeof(float), st);
     }
     ITS_HIP(hipStreamSynchronize(st));
     S.num_valid_voxels = nval;

@@ -156,6 +156,50 @@ def test_eval_schemes_agree(ctx, restore_tunables, dense_cells):
     g.close()
 
 
+@pytest.mark.parametrize("first,second", [(32768, 8), (8, 32768), (32768, 32768)])
+def test_field_rebuilt_on_the_same_octree(ctx, restore_tunables, first, second):
+    """New coefficients and another collapse level on an octree that has its
+    field's cells already: the values of an octree that meets both first."""
+    from its_amd import _capi
+    F = fitted("bunny", 64)
+    c = F.case
+    q = _queries(c, 20011, 6)
+    lam2 = np.random.default_rng(7).standard_normal(len(F.lam))
+    _capi.tune_set(_capi.TUNE_DENSE_CELLS, first)
+    g = _gpu(ctx, F)
+    g.eval(q, c.end)
+    _capi.tune_set(_capi.TUNE_DENSE_CELLS, second)
+    g.set_lambda(lam2)
+    fresh = _capi.Octree(ctx, c.tris, c.origin, c.width, c.R)
+    fresh.set_lambda(lam2)
+    for mode in (_capi.EVAL_SUPPORT, _capi.EVAL_RAW):
+        assert np.array_equal(g.eval(q, c.end, mode), fresh.eval(q, c.end, mode))
+    g.close()
+    fresh.close()
+
+
+@pytest.fixture(scope="module")
+def direct_copies(ctx):
+    """Values of 4,194,309 points, in pieces too small for staged copies."""
+    F = fitted("icosphere", 32)
+    c = F.case
+    g = _gpu(ctx, F)
+    q = np.random.default_rng(8).uniform(c.origin + 0.01, c.end - 0.01, size=(4194309, 3)).astype(np.float32)
+    ref = np.concatenate([g.eval(q[i:i + 32767], c.end) for i in range(0, len(q), 32767)])
+    yield c, g, q, ref
+    g.close()
+
+
+@pytest.mark.parametrize("n", [1048575, 1048576, 1048577, 1049600, 2097152, 4194309])
+def test_eval_staged_copies(direct_copies, n):
+    """Copies out of 4 MB and more go through the pinned chunks: the least one
+    and the size below, ragged last chunks, whole chunks, and the largest chunk
+    with a remainder."""
+    c, g, q, ref = direct_copies
+    print(f"[staged copy] n={n}", flush=True)
+    assert np.array_equal(g.eval(q[:n], c.end), ref[:n])
+
+
 @pytest.mark.parametrize("name,R", [("bunny", 64), ("torus", 32)])
 def test_eval_boundary_points(ctx, name, R):
     """Points on the box faces (open box in SUPPORT mode, closed in DENSE),
