@@ -347,8 +347,11 @@ int its_batch_eval_device_noalloc(its_batch b, const float* d_x, const float* d_
  *   walks its own query (default 1).
  * ITS_TUNE_BATCH_MAX_VERTS: meshes of a batch with at most this many
  *   unknowns may share the one-launch fit (default 65536).
- * ITS_TUNE_SDF_RAY: 1 = for a closed, consistently oriented mesh the sign of
- *   the signed distance comes from the crossings of a ray where exact
+ * ITS_TUNE_SDF_RAY: 1 = for a closed, consistently oriented mesh, and for one
+ *   with a short boundary (at most one uncancelled half edge per two triangles,
+ *   and 4,096), the sign of
+ *   the signed distance comes from the crossings of a ray, and the angles of
+ *   the boundary, where exact
  *   orientation tests decide it (the winding-number fan sum for the other
  *   points); 0 = the fan sum for every point (default 1; same results).
  * No reference counterpart (the reference hard-codes its launch shapes). */

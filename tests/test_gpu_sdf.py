@@ -5,6 +5,7 @@ import pytest
 
 import oracle as O
 from helpers import case, exact_winding_number, fitted
+from its_amd import meshes
 
 pytestmark = pytest.mark.gpu
 
@@ -216,3 +217,63 @@ def test_sdf_packets(ctx, name, N):
     np.testing.assert_array_equal(np.signbit(d[clear]), np.signbit(one[clear]))
     k = rng.choice(np.nonzero(np.isfinite(P).all(1) & (np.abs(P) < 1e3).all(1))[0], 300, replace=False)
     assert np.abs(np.abs(d[k]) - np.abs(O.signed_distance(V, F, P[k]))).max() <= 1e-12
+
+
+def _rim_mesh(kind):
+    rng = np.random.default_rng(21)
+    if kind in ("limit", "over", "long", "too_long"):
+        # two rings of n quads: 4n triangles, 2n boundary half edges; the ray and
+        # the rim take one per two triangles, and 4,096, at most
+        n = {"limit": 300, "over": 300, "long": 2048, "too_long": 2049}[kind]
+        a = 2 * np.pi * np.arange(n) / n
+        V = np.concatenate([np.stack([np.cos(a), np.sin(a), z + 0 * a], 1) for z in (-0.7, 0.1, 0.8)])
+        V = V + rng.uniform(-1e-3, 1e-3, V.shape)
+        i, j = np.arange(n), (np.arange(n) + 1) % n
+        F = np.concatenate([np.stack(t, 1) for o in (0, n) for t in ((i + o, j + o, j + o + n), (i + o, j + o + n, i + o + n))])
+        return V, np.ascontiguousarray(F[1 if kind == "over" else 0:], np.int32)
+    V, F = meshes.noisy_icosphere(seed=2, level=3)
+    if kind == "patch":
+        F = F[np.linalg.norm(V[F].mean(1) - V[5], axis=1) > 0.2]
+    elif kind == "holes":
+        F = F[rng.random(len(F)) > 0.05]
+    elif kind == "flipped":
+        flip = rng.random(len(F)) < 0.03
+        F = np.where(flip[:, None], F[:, ::-1], F)
+    elif kind == "doubled":   # 60 triangles twice, three degenerate ones
+        F = np.concatenate([F[100:], F[300:360], [[5, 5, 9], [7, 8, 8], [4, 4, 4]]])
+    return V, np.ascontiguousarray(F, np.int32)
+
+
+@pytest.mark.parametrize("N", [1, 63, 2000, 40001])
+@pytest.mark.parametrize("kind", ["patch", "holes", "flipped", "doubled", "limit", "over", "long", "too_long"])
+def test_sdf_rim_signs(ctx, kind, N):
+    """Meshes with a boundary: distances are the fan walk's bit for bit, signs
+    those of the winding number summed over all triangles in binary64, wherever
+    that is farther than 1e-4 from 1/2 (binary32 sums of 1,000 angles)."""
+    import torch
+    from its_amd import _capi
+    V, F = _rim_mesh(kind)
+    rng = np.random.default_rng(N)
+    lo, hi = V.min(0), V.max(0)
+    P = rng.uniform(lo - 0.1 * (hi - lo), hi + 0.1 * (hi - lo), (N, 3))
+    near = rng.random(N) < 0.5
+    P[near] = V[rng.integers(len(V), size=near.sum())] + rng.normal(0, 0.01, (near.sum(), 3))
+    print(f"[rim] {kind} T={len(F)} N={N}", flush=True)
+    d = ctx.signed_distance(V, F, P)
+    old = _capi.tune_get(_capi.TUNE_SDF_RAY)
+    _capi.tune_set(_capi.TUNE_SDF_RAY, 0)
+    fan = ctx.signed_distance(V, F, P)
+    _capi.tune_set(_capi.TUNE_SDF_RAY, old)
+    T, Q = torch.from_numpy(V[F]).cuda(), torch.from_numpy(P).cuda()
+    w = torch.zeros(N, dtype=torch.float64, device="cuda")
+    for s in range(0, N, 4000):
+        a, b, c = (T[None, :, k] - Q[s:s + 4000, None] for k in range(3))
+        la, lb, lc = a.norm(dim=2), b.norm(dim=2), c.norm(dim=2)
+        det = (a * torch.linalg.cross(b, c)).sum(2)
+        den = la * lb * lc + (a * b).sum(2) * lc + (b * c).sum(2) * la + (c * a).sum(2) * lb
+        w[s:s + 4000] = torch.atan2(det, den).sum(1) / (2 * np.pi)
+    w = w.cpu().numpy()
+    assert np.array_equal(np.abs(d), np.abs(fan))
+    sure = (np.abs(w - 0.5) > 1e-4) & (np.abs(d) > 1e-9)
+    assert sure.mean() > 0.9
+    assert np.array_equal(np.signbit(d)[sure], (w > 0.5)[sure])
