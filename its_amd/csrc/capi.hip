@@ -154,6 +154,8 @@ int its_ctx_create(int device, its_ctx* out) {
     ITS_HIP(hipEventCreate(&c->ev0));
     ITS_HIP(hipEventCreate(&c->ev1));
     for (hipEvent_t& e : c->mc_ev) ITS_HIP(hipEventCreate(&e));
+    ITS_HIP(hipHostMalloc((void**)&c->pinned, 16 * sizeof(int), hipHostMallocDefault));
+    ITS_HIP(hipEventCreateWithFlags(&c->pinned_ev, hipEventDisableTiming));
     ITS_HIP(hipGetDeviceProperties(&c->prop, device));
     // stream-ordered allocations come from the library's own pool on this
     // device, which keeps freed blocks; the default pool is left as it is
@@ -172,6 +174,8 @@ int its_ctx_destroy(its_ctx ctx) {
     if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
+    if (ctx->pinned_ev) (void)hipEventDestroy(ctx->pinned_ev);
+    if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     for (hipEvent_t e : ctx->mc_ev)
         if (e) (void)hipEventDestroy(e);
     const int dev = ctx->device;
@@ -460,7 +464,7 @@ int its_sdf_at_vertices(its_ctx ctx, its_svo s, const double* V, int64_t nV, con
     const int64_t n = s->num_verts;
     s->rhs.ensure(std::max<int64_t>(n, 1));
     s->rhs_tri.ensure(std::max<int64_t>(n, 1));
-    signed_distance(st, dV.p, nV, dF.p, nF, s->vxyz.p, n, s->rhs.p, s->rhs_tri.p);
+    signed_distance(ctx, dV.p, nV, dF.p, nF, s->vxyz.p, n, s->rhs.p, s->rhs_tri.p);
     s->rhs_nrm.ensure(std::max<int64_t>(n, 1));
     nearest_normals(st, dV.p, dF.p, s->rhs_tri.p, n, s->rhs_nrm.p);
     ITS_HIP(hipStreamSynchronize(st));
@@ -485,7 +489,7 @@ int its_signed_distance(its_ctx ctx, const double* V, int64_t nV, const int32_t*
     DBuf<int32_t> dF = upload(F, 3 * (size_t)nF, st);
     DBuf<double> dP = upload(pts, 3 * (size_t)N, st);
     DBuf<double> dO(N);
-    signed_distance(st, dV.p, nV, dF.p, nF, dP.p, N, dO.p, nullptr);
+    signed_distance(ctx, dV.p, nV, dF.p, nF, dP.p, N, dO.p, nullptr);
     ITS_HIP(hipMemcpyAsync(out, dO.p, N * sizeof(double), hipMemcpyDeviceToHost, st));
     ITS_HIP(hipStreamSynchronize(st));
     ITS_API_END

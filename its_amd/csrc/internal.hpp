@@ -44,6 +44,8 @@ struct HostStage {
 
 struct its_ctx_s {
     its::HostStage stage;
+    int* pinned = nullptr;             // 16 words of pinned host memory, for counts read beside running kernels
+    hipEvent_t pinned_ev = nullptr;    // the last copy to it
     int device = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -158,7 +160,7 @@ void mc_extract(its_svo s, const double origin[3], const double width[3], const 
                 float* h_tri, int64_t capacity, its_mc_stats* st);
 void mc_lattice(its_svo s, const double origin[3], const double width[3], const int res[3], float* h_vals);
 // sdf.hip
-void signed_distance(hipStream_t st, const double* d_V, int64_t nV, const int32_t* d_F, int64_t nF,
+void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* d_F, int64_t nF,
                      const double* d_pts, int64_t N, double* d_out, int32_t* d_tri);
 // stable radix sort of the low `bits` bits, in place
 void sort_u64(DBuf<uint64_t>& keys, int64_t n, int bits, hipStream_t st);

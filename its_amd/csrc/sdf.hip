@@ -258,7 +258,7 @@ __device__ inline uint32_t quant_code(const Quant& q, const double x[3]) {
 
 struct TreeView {
     Shape s;
-    Quant q;
+    const Quant* q;
     const double* tris;      // 9 per sorted triangle
     const float4* sph;       // bounding sphere per sorted triangle
     const float4* nrm;       // unit normal per sorted triangle (zero: none)
@@ -298,8 +298,40 @@ __global__ void k_centroid_box(const double* V, const int32_t* F, int64_t nF, do
     if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = sh[threadIdx.x][0];
 }
 
+// Morton quantisation over the boxes of k_centroid_box; one workgroup of kT
+__global__ __launch_bounds__(kT) void k_quant(const double* part, int nb, Quant* q) {
+    __shared__ double sh[6][kT];
+    for (int x = 0; x < 3; ++x) {
+        double lo = INFINITY, hi = -INFINITY;
+        for (int b = threadIdx.x; b < nb; b += kT) {
+            lo = fmin(lo, part[6 * b + x]);
+            hi = fmax(hi, part[6 * b + 3 + x]);
+        }
+        sh[x][threadIdx.x] = lo;
+        sh[3 + x][threadIdx.x] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    for (int x = 0; x < 3; ++x) {
+        double lo = INFINITY, hi = -INFINITY;
+        for (int k = threadIdx.x; k < kT; k += 64) {
+            lo = fmin(lo, sh[x][k]);
+            hi = fmax(hi, sh[3 + x][k]);
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, o));
+            hi = fmax(hi, __shfl_xor(hi, o));
+        }
+        if (threadIdx.x == 0) {
+            q->lo[x] = lo;
+            q->scale[x] = (hi > lo) ? 1024.0 / (hi - lo) : 0.0;
+        }
+    }
+}
+
 // centroid code of every triangle, with its index as the sort's value
-__global__ void k_tri_keys(const double* V, const int32_t* F, int64_t nF, Quant q, uint32_t* code, uint32_t* idx) {
+__global__ void k_tri_keys(const double* V, const int32_t* F, int64_t nF, const Quant* q, uint32_t* code,
+                           uint32_t* idx) {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nF) return;
     const double* a = V + 3 * (int64_t)F[3 * t];
@@ -307,7 +339,7 @@ __global__ void k_tri_keys(const double* V, const int32_t* F, int64_t nF, Quant 
     const double* c = V + 3 * (int64_t)F[3 * t + 2];
     double m[3];
     for (int x = 0; x < 3; ++x) m[x] = (a[x] + b[x] + c[x]) / 3.0;
-    code[t] = quant_code(q, m);
+    code[t] = quant_code(*q, m);
     idx[t] = (uint32_t)t;
 }
 
@@ -420,27 +452,17 @@ struct RimEdge {
 // Longest boundary that the ray and the rim (k_rim) take: see signed_distance.
 constexpr int kRimMost = 4096;
 
-// open[0] = 1 unless every undirected edge has exactly two half edges of
-// opposite directions (a degenerate edge also opens the mesh); open[1] = the
-// number of half edges left when opposite ones have cancelled, at least if
-// above kRimMost, and rim = these half edges if not, in any order.
-__global__ void k_closed_check(const uint64_t* keys, const uint32_t* vals, int64_t M, uint64_t none, int vb,
-                               const double* V, int* open, RimEdge* rim) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int coef = 0;   // min -> max half edges less max -> min ones
-    if (i < M) {
-        if (keys[i] == none) {
-            open[0] = 1;
-        } else if (edge_head(keys, i, none)) {
-            const bool pair = i + 1 < M && keys[i + 1] == keys[i] && (i + 2 >= M || keys[i + 2] != keys[i]);
-            if (!pair || ((vals[i] ^ vals[i + 1]) & 1u) == 0u) {
-                open[0] = 1;
-                for (int64_t j = i; j < M && keys[j] == keys[i]; ++j) coef += (vals[j] & 1u) ? -1 : 1;
-            }
-        }
-    }
+// The undirected edges' half edges, counted: open[0] = 1 unless every edge has
+// exactly two half edges of opposite directions (a degenerate edge also opens
+// the mesh); open[1] = the number of half edges left when opposite ones have
+// cancelled, at least if above kRimMost, and rim = these half edges if not, in
+// any order.  Called by whole wavefronts: key, number and sum (min -> max less
+// max -> min) of an edge per lane, 0 half edges for none.
+__device__ inline void boundary_edge(uint64_t key, uint32_t number, int sum, int vb, const double* V, int* open,
+                                     RimEdge* rim) {
+    if (number != 0 && (number != 2 || sum != 0)) open[0] = 1;
     // places on the list: one atomic per wavefront, none once it is too long
-    const int lane = threadIdx.x & 63, copies = min(abs(coef), kRimMost + 1);
+    const int lane = threadIdx.x & 63, copies = min(abs(sum), kRimMost + 1);
     const int upto = wave_incl_scan(copies), total = __shfl(upto, 63);
     if (total == 0) return;
     int first = 0;
@@ -450,14 +472,65 @@ __global__ void k_closed_check(const uint64_t* keys, const uint32_t* vals, int64
     }
     first = __shfl(first, 63) + upto - copies;
     if (copies == 0 || first + copies > kRimMost) return;
-    const int64_t lo = (int64_t)(keys[i] >> vb), hi = (int64_t)(keys[i] & ((1ull << vb) - 1ull));
-    const double* a = V + 3 * (coef > 0 ? lo : hi);
-    const double* b = V + 3 * (coef > 0 ? hi : lo);
+    const int64_t lo = (int64_t)(key >> vb), hi = (int64_t)(key & ((1ull << vb) - 1ull));
+    const double* a = V + 3 * (sum > 0 ? lo : hi);
+    const double* b = V + 3 * (sum > 0 ? hi : lo);
     for (int c = 0; c < copies; ++c)
         for (int x = 0; x < 3; ++x) {
             rim[first + c].a[x] = a[x];
             rim[first + c].b[x] = b[x];
         }
+}
+
+// Edges by a hash table: whether a mesh is closed needs no order.  A sort of
+// the half edges, which only the fans need, took 12 to 15 launches (60,000 half
+// edges: 47 us; the table 14, and 57 at 600,000, bound by the atomics).  A slot
+// holds key + 1 (0: empty), and in one word the number of half edges and,
+// above it, their sum.  Linear probing; the table has at least 1.5 slots a
+// half edge, so an empty slot ends every probe.
+struct EdgeSlot {
+    unsigned long long key, stat;
+};
+__global__ void k_edge_insert(const int32_t* F, int64_t nF, int vb, EdgeSlot* slots, int bits, int* open) {
+    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (h >= 3 * nF) return;
+    const int64_t t = h / 3;
+    const int e = (int)(h - 3 * t);
+    const uint32_t a = (uint32_t)F[3 * t + e], b = (uint32_t)F[3 * t + (e + 1) % 3];
+    if (a == b) {
+        open[0] = 1;
+        return;
+    }
+    const unsigned long long key = (((unsigned long long)std::min(a, b) << vb) | std::max(a, b)) + 1ull;
+    const unsigned long long mask = (1ull << bits) - 1ull;
+    unsigned long long at = (key * 0x9E3779B97F4A7C15ull) >> (64 - bits);
+    for (;; at = (at + 1ull) & mask) {
+        unsigned long long k = __hip_atomic_load(&slots[at].key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (k == 0ull) {
+            k = atomicCAS(&slots[at].key, 0ull, key);
+            if (k == 0ull) k = key;
+        }
+        if (k == key) break;
+    }
+    atomicAdd(&slots[at].stat, (a > b ? 0xFFFFFFFF00000001ull : 0x0000000100000001ull));
+}
+__global__ void k_edge_check(const EdgeSlot* slots, int64_t n, int vb, const double* V, int* open, RimEdge* rim) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    EdgeSlot s{0ull, 0ull};
+    if (i < n) s = slots[i];
+    boundary_edge(s.key - 1ull, (uint32_t)s.stat, (int)(uint32_t)(s.stat >> 32), vb, V, open, rim);
+}
+
+// the same from the sorted half edges
+__global__ void k_closed_check(const uint64_t* keys, const uint32_t* vals, int64_t M, uint64_t none, int vb,
+                               const double* V, int* open, RimEdge* rim) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t number = 0;
+    int sum = 0;
+    if (i < M && keys[i] == none) open[0] = 1;
+    if (i < M && edge_head(keys, i, none))
+        for (int64_t j = i; j < M && keys[j] == keys[i]; ++j, ++number) sum += (vals[j] & 1u) ? -1 : 1;
+    boundary_edge(i < M ? keys[i] : 0ull, number, sum, vb, V, open, rim);
 }
 
 __global__ void k_fan_node_count(const uint64_t* keys, const uint32_t* vals, int64_t M, Shape s, uint64_t none,
@@ -713,25 +786,27 @@ void radix_sort(DBuf<K>& keys, DBuf<V>* vals, int64_t n, int bits, hipStream_t s
 
 struct TriTree {
     Shape s{};
-    Quant q{};
     int64_t nodes = 0, fans = 0;
+    DBuf<Quant> q;
     DBuf<double> tris;
     DBuf<float> fan;
     DBuf<float4> sph, nrm, node;
     DBuf<int32_t> tid;
     DBuf<uint32_t> code, cell_lb;
     int cell_bits = 0;
-    bool closed = false;   // every undirected edge: exactly two half edges, opposite directions
-    // half edges sorted by undirected edge (for the fans) and the open flag
+    // half edges sorted by undirected edge, for the fans
     DBuf<uint64_t> hkeys;
     DBuf<uint32_t> hvals;
-    DBuf<int> is_open;       // flag, boundary half edges (k_closed_check)
+    DBuf<int32_t> pos;       // sorted position per triangle
+    // open flag, boundary half edges (boundary_edge); points passed on by the
+    // two packet kernels, undecided points
+    DBuf<int> counts;
     DBuf<RimEdge> rim;
     int64_t M = 0;
     uint64_t none = 0;
     int vb = 0;
     TreeView view() const {
-        return TreeView{s, q, tris.p, sph.p, nrm.p, tid.p, code.p, node.p, fan.p, cell_lb.p, cell_bits};
+        return TreeView{s, q.p, tris.p, sph.p, nrm.p, tid.p, code.p, node.p, fan.p, cell_lb.p, cell_bits};
     }
 };
 
@@ -748,6 +823,20 @@ __global__ void k_cell_lb(const uint32_t* code, int64_t T, int bits, uint32_t* l
     }
     lb[C] = (uint32_t)a;
 }
+
+void sort_half_edges(TriTree& tr, hipStream_t st, const int32_t* d_F) {
+    const int64_t M = tr.M;
+    tr.hkeys.alloc(M);
+    tr.hvals.alloc(M);
+    hipLaunchKernelGGL(k_half_edges, dim3(blocks_for(M, kT)), dim3(kT), 0, st, d_F, M / 3, (const int32_t*)tr.pos.p,
+                       tr.vb, tr.none, tr.hkeys.p, tr.hvals.p);
+    ITS_LAUNCH_CHECK();
+    radix_sort(tr.hkeys, &tr.hvals, M, std::min(64, 2 * tr.vb), st);
+}
+
+// Most half edges for the hash table: 2^24 slots, 256 MB, the size of the
+// Infinity Cache.
+constexpr int64_t kHashEdges = int64_t(1) << 23;
 
 void tree_build(TriTree& tr, hipStream_t st, const double* d_V, int64_t nV, const int32_t* d_F, int64_t nF) {
     ITS_REQUIRE(nF > 0 && nF < (1ll << 30) && nV < (1ll << 31), ITS_E_RANGE, "mesh too large for the triangle tree (2^30 triangles, 2^31 vertices)");
@@ -769,29 +858,24 @@ void tree_build(TriTree& tr, hipStream_t st, const double* d_V, int64_t nV, cons
     DBuf<double> part(6 * (size_t)nb);
     hipLaunchKernelGGL(k_centroid_box, dim3(nb), dim3(kT), 0, st, d_V, d_F, nF, part.p);
     ITS_LAUNCH_CHECK();
-    std::vector<double> hp;
-    to_host(hp, part.p, 6 * (size_t)nb, st);
-    ITS_HIP(hipStreamSynchronize(st));
-    for (int a = 0; a < 3; ++a) {
-        double lo = INFINITY, hi = -INFINITY;
-        for (int b = 0; b < nb; ++b) { lo = std::min(lo, hp[6 * b + a]); hi = std::max(hi, hp[6 * b + 3 + a]); }
-        tr.q.lo[a] = lo;
-        tr.q.scale[a] = (hi > lo) ? 1024.0 / (hi - lo) : 0.0;
-    }
+    tr.q.alloc(1);
+    hipLaunchKernelGGL(k_quant, dim3(1), dim3(kT), 0, st, (const double*)part.p, nb, tr.q.p);
+    ITS_LAUNCH_CHECK();
 
     // sort triangles by centroid code (stable: ties by index)
     tr.code.alloc(nF);
     DBuf<uint32_t> tidx(nF);
-    hipLaunchKernelGGL(k_tri_keys, dim3(blocks_for(nF, kT)), dim3(kT), 0, st, d_V, d_F, nF, tr.q, tr.code.p, tidx.p);
+    hipLaunchKernelGGL(k_tri_keys, dim3(blocks_for(nF, kT)), dim3(kT), 0, st, d_V, d_F, nF, (const Quant*)tr.q.p, tr.code.p,
+                       tidx.p);
     ITS_LAUNCH_CHECK();
     radix_sort(tr.code, &tidx, nF, 30, st);
     tr.tris.alloc(9 * (size_t)nF);
     tr.sph.alloc(nF);
     tr.nrm.alloc(nF);
     tr.tid.alloc(nF);
-    DBuf<int32_t> pos(nF);
+    tr.pos.alloc(nF);
     hipLaunchKernelGGL(k_tri_gather, dim3(blocks_for(nF, kT)), dim3(kT), 0, st, (const uint32_t*)tidx.p, nF, d_V, d_F,
-                       tr.tris.p, tr.sph.p, tr.nrm.p, tr.tid.p, pos.p);
+                       tr.tris.p, tr.sph.p, tr.nrm.p, tr.tid.p, tr.pos.p);
     ITS_LAUNCH_CHECK();
     // code-prefix table with about one prefix per triangle (3 to 21 bits)
     tr.cell_bits = 3;
@@ -812,30 +896,39 @@ void tree_build(TriTree& tr, hipStream_t st, const double* d_V, int64_t nV, cons
     }
 
     // half edges grouped by undirected edge: whether the mesh is closed, and
-    // the boundaries of the fans
+    // its boundary
     const int64_t M = 3 * nF;
     const int vb = bits_for((uint64_t)(nV - 1));
-    const uint64_t none = (2 * vb >= 64) ? ~0ull : ((1ull << (2 * vb)) - 1);
     tr.M = M;
     tr.vb = vb;
-    tr.none = none;
-    tr.hkeys.alloc(M);
-    tr.hvals.alloc(M);
-    hipLaunchKernelGGL(k_half_edges, dim3(blocks_for(M, kT)), dim3(kT), 0, st, d_F, nF, (const int32_t*)pos.p, vb, none,
-                       tr.hkeys.p, tr.hvals.p);
-    ITS_LAUNCH_CHECK();
-    radix_sort(tr.hkeys, &tr.hvals, M, std::min(64, 2 * vb), st);
-    tr.is_open.alloc(2);
+    tr.none = (2 * vb >= 64) ? ~0ull : ((1ull << (2 * vb)) - 1);
+    tr.counts.alloc(5);
     tr.rim.alloc(kRimMost);
-    ITS_HIP(hipMemsetAsync(tr.is_open.p, 0, tr.is_open.bytes(), st));
-    hipLaunchKernelGGL(k_closed_check, dim3(blocks_for(M, kT)), dim3(kT), 0, st, (const uint64_t*)tr.hkeys.p,
-                       (const uint32_t*)tr.hvals.p, M, none, vb, d_V, tr.is_open.p, tr.rim.p);
-    ITS_LAUNCH_CHECK();
+    ITS_HIP(hipMemsetAsync(tr.counts.p, 0, tr.counts.bytes(), st));
+    if (M <= kHashEdges) {
+        int bits = 1;
+        while ((int64_t(1) << bits) < M + M / 2) ++bits;
+        const int64_t n = int64_t(1) << bits;
+        DBuf<EdgeSlot> slots(n);
+        ITS_HIP(hipMemsetAsync(slots.p, 0, slots.bytes(), st));
+        hipLaunchKernelGGL(k_edge_insert, dim3(blocks_for(M, kT)), dim3(kT), 0, st, d_F, nF, vb, slots.p, bits,
+                           tr.counts.p);
+        ITS_LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_edge_check, dim3(blocks_for(n, kT)), dim3(kT), 0, st, (const EdgeSlot*)slots.p, n, vb,
+                           d_V, tr.counts.p, tr.rim.p);
+        ITS_LAUNCH_CHECK();
+    } else {
+        sort_half_edges(tr, st, d_F);
+        hipLaunchKernelGGL(k_closed_check, dim3(blocks_for(M, kT)), dim3(kT), 0, st, (const uint64_t*)tr.hkeys.p,
+                           (const uint32_t*)tr.hvals.p, M, tr.none, vb, d_V, tr.counts.p, tr.rim.p);
+        ITS_LAUNCH_CHECK();
+    }
 }
 
 // Boundary fans of the tree's nodes, for the winding-number walk; built only
 // when some point needs that walk.
-void fans_build(TriTree& tr, hipStream_t st, const double* d_V) {
+void fans_build(TriTree& tr, hipStream_t st, const double* d_V, const int32_t* d_F) {
+    if (!tr.hkeys.p) sort_half_edges(tr, st, d_F);
     const Shape& s = tr.s;
     const int64_t M = tr.M;
     const int vb = tr.vb;
@@ -1116,7 +1209,7 @@ __global__ void k_pt_seed(TreeView t, const double* pts, int64_t N, uint32_t* ke
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
-    const uint32_t c = quant_code(t.q, p);
+    const uint32_t c = quant_code(*t.q, p);
     const uint32_t C = c >> (30 - t.cell_bits);
     int64_t a = t.cell_lb[C], b = t.cell_lb[C + 1];
     while (a < b) {
@@ -1666,8 +1759,8 @@ __device__ inline int tri_ray(const double* T, const double p[3], const Ray& R, 
 // number), so one walk serves them all.
 // decided[i] = 1 and the sign is applied when every orientation was certain
 // and the lists fitted; otherwise decided[i] = 0 and the fan walk takes the
-// point.  With cross given (a mesh with a boundary) the crossings and the ray's
-// axis and direction are left there instead, and k_rim applies the sign.
+// point.  With cross given (an open mesh) the crossings and the ray's axis and
+// direction are left there instead, and k_rim applies the sign.
 template <int P, int FRONT>
 __global__ __launch_bounds__(64, 5) void k_ray_packet(TreeView t, const double* pts, Work work, double* out,
                                                    uint8_t* decided, int* cross, unsigned* undecided, uint32_t* rest,
@@ -1962,11 +2055,15 @@ __global__ __launch_bounds__(kT) void k_sdf_wind(TreeView t, const double* pts, 
 }
 }  // namespace
 
-void signed_distance(hipStream_t st, const double* d_V, int64_t nV, const int32_t* d_F, int64_t nF,
+void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* d_F, int64_t nF,
                      const double* d_pts, int64_t N, double* d_out, int32_t* d_tri) {
     if (N <= 0) return;
+    const hipStream_t st = ctx->stream;
     TriTree tr;
     tree_build(tr, st, d_V, nV, d_F, nF);
+    // the boundary, read while the distance kernels run
+    ITS_HIP(hipMemcpyAsync(ctx->pinned, tr.counts.p, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
+    ITS_HIP(hipEventRecord(ctx->pinned_ev, st));
     // grid-strided launches: as many blocks as the CUs hold at once
     int dev = 0, cus = 256;
     ITS_HIP(hipGetDevice(&dev));
@@ -1988,26 +2085,21 @@ void signed_distance(hipStream_t st, const double* d_V, int64_t nV, const int32_
     hipLaunchKernelGGL(k_pt_seed, dim3(blocks_for(N, kT)), dim3(kT), 0, st, tr.view(), d_pts, N, key.p, order.p, d_out,
                        seed_at.p);
     ITS_LAUNCH_CHECK();
-    DBuf<unsigned> counts(3);   // points passed on by the two packet kernels, undecided points
-    ITS_HIP(hipMemsetAsync(counts.p, 0, counts.bytes(), st));
+    unsigned* counts = (unsigned*)tr.counts.p + 2;   // passed on, twice, and undecided
     const unsigned pgrid = (unsigned)((N + kPk - 1) / kPk);
     Work all{N, nullptr, nullptr}, left = all;
     if (packets) {
         radix_sort(key, &order, N, kSeedKeyBits, st);
         rest.alloc(N);
         all.list = order.p;
-        left = Work{N, rest.p, counts.p};
+        left = Work{N, rest.p, counts};
         hipLaunchKernelGGL(dist1, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, (const int32_t*)seed_at.p, d_out,
-                           d_tri, rest.p, counts.p);
+                           d_tri, rest.p, counts);
         ITS_LAUNCH_CHECK();
     }
     hipLaunchKernelGGL(dist2, dim3(grid_of((const void*)dist2, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left,
                        (const int32_t*)seed_at.p, d_out, d_tri, (uint32_t*)nullptr, (unsigned*)nullptr);
     ITS_LAUNCH_CHECK();
-    int boundary[2];   // k_closed_check
-    ITS_HIP(hipMemcpyAsync(boundary, tr.is_open.p, sizeof boundary, hipMemcpyDeviceToHost, st));
-    ITS_HIP(hipStreamSynchronize(st));
-    tr.closed = boundary[0] == 0;
     // Signs by the ray, and the rim where there is a boundary, for the points
     // that they decide; the fans are built and walked only for the others.
     // The rim's time grows with the boundary, the fan walk's hardly, so long
@@ -2018,31 +2110,35 @@ void signed_distance(hipStream_t st, const double* d_V, int64_t nV, const int32_
     // 60,000 points: 1.23 and 1.97; torus of 8,638 with 3,566: about equal).
     DBuf<uint8_t> decided;
     DBuf<int> cross;
-    int64_t undecided = N;
-    if (boundary[1] <= std::min<int64_t>(kRimMost, nF / 2) && tune_get(ITS_TUNE_SDF_RAY)) {
+    const int most = (int)std::min<int64_t>(kRimMost, nF / 2);
+    ITS_HIP(hipEventSynchronize(ctx->pinned_ev));
+    const bool open = ctx->pinned[0] != 0;
+    const int rim = ctx->pinned[1];
+    const bool by_ray = rim <= most && tune_get(ITS_TUNE_SDF_RAY);
+    bool fans = true;
+    if (by_ray) {
         decided.alloc(N);
-        if (!tr.closed) cross.alloc(N);
+        if (open) cross.alloc(N);
         if (packets) {
-            left.list_n = counts.p + 1;
+            left.list_n = counts + 1;
             hipLaunchKernelGGL(ray1, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, d_out, decided.p,
-                               cross.p, counts.p + 2, rest.p, counts.p + 1);
+                               cross.p, counts + 2, rest.p, counts + 1);
             ITS_LAUNCH_CHECK();
         }
         hipLaunchKernelGGL(ray2, dim3(grid_of((const void*)ray2, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left, d_out,
-                           decided.p, cross.p, counts.p + 2, (uint32_t*)nullptr, (unsigned*)nullptr);
+                           decided.p, cross.p, counts + 2, (uint32_t*)nullptr, (unsigned*)nullptr);
         ITS_LAUNCH_CHECK();
-        if (!tr.closed) {
-            hipLaunchKernelGGL(k_rim, dim3(blocks_for(N, 64)), dim3(64 * kRimWaves), 0, st,
-                               (const RimEdge*)tr.rim.p, boundary[1], d_pts, N, d_out, decided.p,
-                               (const int*)cross.p, counts.p + 2);
+        if (open) {
+            hipLaunchKernelGGL(k_rim, dim3(blocks_for(N, 64)), dim3(64 * kRimWaves), 0, st, (const RimEdge*)tr.rim.p,
+                               rim, d_pts, N, d_out, decided.p, (const int*)cross.p, counts + 2);
             ITS_LAUNCH_CHECK();
         }
-        undecided = read1(counts.p + 2, st);
+        fans = read1(counts + 2, st) != 0;
     }
-    if (undecided > 0) {
-        fans_build(tr, st, d_V);
+    if (fans) {
+        fans_build(tr, st, d_V, d_F);
         hipLaunchKernelGGL(k_sdf_wind, dim3(grid_of((const void*)k_sdf_wind, kT, (N + kWavesPerBlock - 1) / kWavesPerBlock)), dim3(kT), 0, st, tr.view(), d_pts, N, d_out,
-                           (const uint8_t*)decided.p);
+                           by_ray ? (const uint8_t*)decided.p : (const uint8_t*)nullptr);
         ITS_LAUNCH_CHECK();
     }
     ITS_HIP(hipStreamSynchronize(st));

@@ -277,3 +277,24 @@ def test_sdf_rim_signs(ctx, kind, N):
     sure = (np.abs(w - 0.5) > 1e-4) & (np.abs(d) > 1e-9)
     assert sure.mean() > 0.9
     assert np.array_equal(np.signbit(d)[sure], (w > 0.5)[sure])
+
+
+@pytest.mark.parametrize("hole", [False, True])
+def test_sdf_many_half_edges(ctx, hole):
+    """Above 2^23 half edges they are sorted, not hashed, to find the boundary:
+    the ray's signs are the fan walk's."""
+    from its_amd import _capi
+    V, F = meshes.torus(1700, 850)
+    assert 3 * len(F) > 1 << 23
+    if hole:
+        F = np.ascontiguousarray(F[np.linalg.norm(V[F].mean(1) - V[1000], axis=1) > 0.01])
+    rng = np.random.default_rng(5)
+    P = V[rng.integers(len(V), size=3000)] + rng.normal(0, 0.02, (3000, 3))
+    print(f"[many half edges] T={len(F)}", flush=True)
+    d = ctx.signed_distance(V, F, P)
+    old = _capi.tune_get(_capi.TUNE_SDF_RAY)
+    _capi.tune_set(_capi.TUNE_SDF_RAY, 0)
+    fan = ctx.signed_distance(V, F, P)
+    _capi.tune_set(_capi.TUNE_SDF_RAY, old)
+    assert np.array_equal(d, fan)
+    assert 0.3 < np.signbit(d).mean() < 0.7
