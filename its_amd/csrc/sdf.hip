@@ -1158,7 +1158,7 @@ __device__ void dist_dfs(const TreeView& t, int leaf, int lane, const double p[3
 // results are theirs bit for bit.  Bound by vector instructions (about 3,800
 // per packet of 16 points, 65 % of the issue slots; a wavefront per point took
 // over 1,200 per point): 200,000 triangles and 554,122 octree vertices,
-// distances 2,736 -> 370 us and 350 us for the 2 % of points on the second
+// distances 2,736 -> 370 us and 305 us for the 2 % of points on the second
 // pass, crossings 1,692 -> 270 us, seeds 58 us and their sort 75 us.
 //
 // P points per packet: 16 on the first pass, over all points.  Packets whose
