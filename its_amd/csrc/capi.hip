@@ -466,7 +466,7 @@ int its_sdf_at_vertices(its_ctx ctx, its_svo s, const double* V, int64_t nV, con
     s->rhs_tri.ensure(std::max<int64_t>(n, 1));
     signed_distance(ctx, dV.p, nV, dF.p, nF, s->vxyz.p, n, s->rhs.p, s->rhs_tri.p);
     s->rhs_nrm.ensure(std::max<int64_t>(n, 1));
-    nearest_normals(st, dV.p, dF.p, s->rhs_tri.p, n, s->rhs_nrm.p);
+    nearest_normals(st, dV.p, dF.p, nF, s->rhs_tri.p, n, s->rhs_nrm.p);
     ITS_HIP(hipStreamSynchronize(st));
     s->has_rhs = true;
     if (b && n) {

@@ -164,8 +164,8 @@ void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* 
                      const double* d_pts, int64_t N, double* d_out, int32_t* d_tri);
 // stable radix sort of the low `bits` bits, in place
 void sort_u64(DBuf<uint64_t>& keys, int64_t n, int bits, hipStream_t st);
-void nearest_normals(hipStream_t st, const double* d_V, const int32_t* d_F, const int32_t* d_tri, int64_t N,
-                     float4* d_nrm);
+void nearest_normals(hipStream_t st, const double* d_V, const int32_t* d_F, int64_t nF, const int32_t* d_tri,
+                     int64_t N, float4* d_nrm);
 void eval_batch(its_svo const* svos, int64_t count, const int64_t* off, const float* x, const float* y,
                 const float* z, float out_val, float* f, hipStream_t st);
 // the same launch with its tables in the file-scope scratch array of eval.hip

@@ -1424,7 +1424,7 @@ __global__ __launch_bounds__(64, 5) void k_dist_packet(TreeView t, const double*
     __shared__ uint32_t cand[kTriQueue];     // (frontier slot * 8 + triangle) * P + point
     __shared__ double sp[3][P];
     __shared__ float sub[P];               // upper bounds with margin
-    __shared__ float4 sseed[P];            // bounding spheres of the points' seed triangles
+    __shared__ float4 sseed[P];            // bounding spheres of the points' seed triangles (centre at infinity: no bound)
     __shared__ unsigned long long sbest[P];   // bits of the best squared distance (order of non-negative doubles)
     __shared__ int32_t sid[P];
     const int lane = threadIdx.x, pt = lane & (P - 1), slot = lane / P;
@@ -1451,13 +1451,18 @@ __global__ __launch_bounds__(64, 5) void k_dist_packet(TreeView t, const double*
     if (slot == 0) {
         const int32_t j = seed_at[i];
         for (int a = 0; a < 3; ++a) sp[a][pt] = p[a];
-        sseed[pt] = t.sph[j];
+        // A triangle with a unit normal has a distance to every point, no larger
+        // than its centre's.  A face (a, a, c) has none (0 / 0) for the points
+        // on the c side of a: it never wins, so its centre bounds nothing.
+        const float4 S = t.sph[j], nr = t.nrm[j];
+        const bool sound = nr.x * nr.x + nr.y * nr.y + nr.z * nr.z > 0.5f;
+        sseed[pt] = sound ? S : make_float4(INFINITY, 0.f, 0.f, S.w);
         sbest[pt] = (unsigned long long)__double_as_longlong(seed_d2);
         sid[pt] = seed_d2 < INFINITY ? t.tid[j] : 0x7fffffff;
     }
     lds_fence();
     // A point's Morton position can miss a triangle that a neighbour's found:
-    // the centres of all the packet's seeds bound its distance too.
+    // the centres of all the packet's sound seeds bound its distance too.
     for (int q = slot; q < P; q += SUB) {
         const float4 S = sseed[q];
         const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z;
@@ -2145,11 +2150,17 @@ void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* 
 }
 
 namespace {
-// unit normal of each point's nearest triangle (zero for a degenerate one)
-__global__ void k_tri_normal(int64_t N, const double* V, const int32_t* F, const int32_t* tri, float4* nrm) {
+// unit normal of each point's nearest triangle (zero for a degenerate one, and
+// for a point to which no triangle has a distance)
+__global__ void k_tri_normal(int64_t N, const double* V, const int32_t* F, int64_t nF, const int32_t* tri,
+                             float4* nrm) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     const int32_t t = tri[i];
+    if (t < 0 || t >= nF) {
+        nrm[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        return;
+    }
     const double* a = V + 3 * (int64_t)F[3 * (int64_t)t];
     const double* b = V + 3 * (int64_t)F[3 * (int64_t)t + 1];
     const double* c = V + 3 * (int64_t)F[3 * (int64_t)t + 2];
@@ -2160,10 +2171,10 @@ __global__ void k_tri_normal(int64_t N, const double* V, const int32_t* F, const
 }
 }  // namespace
 
-void nearest_normals(hipStream_t st, const double* d_V, const int32_t* d_F, const int32_t* d_tri, int64_t N,
-                     float4* d_nrm) {
+void nearest_normals(hipStream_t st, const double* d_V, const int32_t* d_F, int64_t nF, const int32_t* d_tri,
+                     int64_t N, float4* d_nrm) {
     if (N <= 0) return;
-    hipLaunchKernelGGL(k_tri_normal, dim3(blocks_for(N, kT)), dim3(kT), 0, st, N, d_V, d_F, d_tri, d_nrm);
+    hipLaunchKernelGGL(k_tri_normal, dim3(blocks_for(N, kT)), dim3(kT), 0, st, N, d_V, d_F, nF, d_tri, d_nrm);
     ITS_LAUNCH_CHECK();
 }
 

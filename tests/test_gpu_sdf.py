@@ -219,6 +219,48 @@ def test_sdf_packets(ctx, name, N):
     assert np.abs(np.abs(d[k]) - np.abs(O.signed_distance(V, F, P[k]))).max() <= 1e-12
 
 
+def _collapsed_mesh(order):
+    """Closed sphere and one face on the chord between two far vertices i and
+    j, of no area: a repeated corner (the distance to it is 0 / 0 for half of
+    space in one of the orders) or three collinear ones."""
+    V, F = meshes.icosphere(3)
+    i, j = 0, int(np.argmin(V @ V[0]))
+    V = np.concatenate([V, [0.3 * V[i] + 0.7 * V[j]]])
+    face = {"iij": [i, i, j], "ijj": [i, j, j], "iji": [i, j, i], "line": [i, len(V) - 1, j]}[order]
+    return np.ascontiguousarray(V), np.concatenate([F, [face]]).astype(np.int32), i, j
+
+
+@pytest.mark.parametrize("N", [2000, 40001])
+@pytest.mark.parametrize("order", ["iij", "ijj", "iji", "line"])
+def test_sdf_collapsed_face(ctx, order, N):
+    """Points around a face of no area far from all others, one by one and in
+    packets, against the brute-force oracle: the face bounds no distance that
+    it does not have."""
+    V, F, i, j = _collapsed_mesh(order)
+    rng = np.random.default_rng(N)
+    P = V[i] + rng.uniform(-0.05, 1.05, (N, 1)) * (V[j] - V[i]) + 0.02 * rng.standard_normal((N, 3))
+    P[: N // 2] = V[F[-1]].mean(0) + 0.02 * rng.standard_normal((N // 2, 3))   # around its centre
+    print(f"[sdf collapsed] {order} N={N}", flush=True)
+    d = ctx.signed_distance(V, F, P)
+    ref = O.signed_distance(V, F, P)
+    assert np.isfinite(d).all()
+    assert np.abs(np.abs(d) - np.abs(ref)).max() <= 1e-12
+
+
+@pytest.mark.parametrize("order", ["iij", "line"])
+def test_sdf_collapsed_face_at_vertices(ctx, order):
+    """The same at the octree's vertices, some of which lie along the face."""
+    from its_amd import _capi
+    V, F, _, _ = _collapsed_mesh(order)
+    V = O.normalize(V)
+    o, _, w = O.uniform_bbox(V)
+    g = _capi.Octree(ctx, meshes.triangles(V, F), o, w, 32)
+    print(f"[sdf collapsed] {order} n={g.num_verts}", flush=True)
+    b = g.sdf_at_vertices(V, F)
+    assert np.isfinite(b).all()
+    assert np.abs(np.abs(b) - np.abs(O.signed_distance(V, F, g.verts()[0]))).max() <= 1e-12
+
+
 def _rim_mesh(kind):
     rng = np.random.default_rng(21)
     if kind in ("limit", "over", "long", "too_long"):
