@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "its_c.h"
+#include "launch.hpp"
 
 namespace its {
 

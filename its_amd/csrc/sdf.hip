@@ -1206,75 +1206,75 @@ constexpr int kSeedKeyBits = 24;
 // d2_out, at_out: exact squared distance and sorted position of the triangle near p
 __global__ void k_pt_seed(TreeView t, const double* pts, int64_t N, uint32_t* key, uint32_t* idx, double* d2_out,
                           int32_t* at_out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
-    const uint32_t c = quant_code(*t.q, p);
-    const uint32_t C = c >> (30 - t.cell_bits);
-    int64_t a = t.cell_lb[C], b = t.cell_lb[C + 1];
-    while (a < b) {
-        const int64_t m = (a + b) >> 1;
-        if (t.code[m] < c) a = m + 1; else b = m;
-    }
-    const int64_t lo = max((int64_t)0, min(a, (int64_t)t.s.T) - kSeedWindow / 2);
-    const int64_t hi = min((int64_t)t.s.T, lo + kSeedWindow);
-    const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
-    float near2 = INFINITY;
-    int64_t j = min(a, (int64_t)t.s.T - 1);
-    for (int64_t k = lo; k < hi; ++k) {
-        const float4 S = t.sph[k];
-        const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z;
-        const float d2 = dx * dx + dy * dy + dz * dz;
-        if (d2 < near2) {
-            near2 = d2;
-            j = k;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (int64_t)gridDim.x * blockDim.x) {
+        const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
+        const uint32_t c = quant_code(*t.q, p);
+        const uint32_t C = c >> (30 - t.cell_bits);
+        int64_t a = t.cell_lb[C], b = t.cell_lb[C + 1];
+        while (a < b) {
+            const int64_t m = (a + b) >> 1;
+            if (t.code[m] < c) a = m + 1; else b = m;
         }
-    }
-    const NodeRec root = load_node(t, t.s.off[t.s.H]);
-    const float ext = fmaxf(root.hi.x - root.lo.x, fmaxf(root.hi.y - root.lo.y, root.hi.z - root.lo.z));
-    // Away from the surface the Morton position says little (a tenth of the
-    // seeds are over twice as far as the nearest triangle), and the reach of
-    // a packet grows with it: such a point also descends the tree, to the
-    // child whose box is nearer by its nearest and farthest corner together,
-    // and looks at that bucket.
-    if (near2 > ext * ext * (1.f / (128.f * 128.f))) {
-        int k = 0;
-        for (int h = t.s.H; h > 0; --h) {
-            float m[2] = {INFINITY, INFINITY};
-            for (int c = 0; c < 2; ++c) {
-                if (2 * k + c >= t.s.count[h - 1]) break;
-                const NodeRec r = load_node(t, t.s.off[h - 1] + 2 * k + c);
-                const float l[3] = {r.lo.x, r.lo.y, r.lo.z}, u[3] = {r.hi.x, r.hi.y, r.hi.z};
-                m[c] = 0.f;
-                for (int x = 0; x < 3; ++x) {
-                    const float e = fmaxf(fmaxf(l[x] - pf[x], pf[x] - u[x]), 0.f);
-                    const float f = fmaxf(fabsf(pf[x] - l[x]), fabsf(pf[x] - u[x]));
-                    m[c] += e * e + f * f;
-                }
-            }
-            k = 2 * k + (m[1] < m[0] ? 1 : 0);
-        }
-        for (int q = k * kBucket; q < min((k + 1) * kBucket, t.s.T); ++q) {
-            const float4 S = t.sph[q];
+        const int64_t lo = max((int64_t)0, min(a, (int64_t)t.s.T) - kSeedWindow / 2);
+        const int64_t hi = min((int64_t)t.s.T, lo + kSeedWindow);
+        const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
+        float near2 = INFINITY;
+        int64_t j = min(a, (int64_t)t.s.T - 1);
+        for (int64_t k = lo; k < hi; ++k) {
+            const float4 S = t.sph[k];
             const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z;
             const float d2 = dx * dx + dy * dy + dz * dz;
             if (d2 < near2) {
                 near2 = d2;
-                j = q;
+                j = k;
             }
         }
+        const NodeRec root = load_node(t, t.s.off[t.s.H]);
+        const float ext = fmaxf(root.hi.x - root.lo.x, fmaxf(root.hi.y - root.lo.y, root.hi.z - root.lo.z));
+        // Away from the surface the Morton position says little (a tenth of the
+        // seeds are over twice as far as the nearest triangle), and the reach of
+        // a packet grows with it: such a point also descends the tree, to the
+        // child whose box is nearer by its nearest and farthest corner together,
+        // and looks at that bucket.
+        if (near2 > ext * ext * (1.f / (128.f * 128.f))) {
+            int k = 0;
+            for (int h = t.s.H; h > 0; --h) {
+                float m[2] = {INFINITY, INFINITY};
+                for (int c = 0; c < 2; ++c) {
+                    if (2 * k + c >= t.s.count[h - 1]) break;
+                    const NodeRec r = load_node(t, t.s.off[h - 1] + 2 * k + c);
+                    const float l[3] = {r.lo.x, r.lo.y, r.lo.z}, u[3] = {r.hi.x, r.hi.y, r.hi.z};
+                    m[c] = 0.f;
+                    for (int x = 0; x < 3; ++x) {
+                        const float e = fmaxf(fmaxf(l[x] - pf[x], pf[x] - u[x]), 0.f);
+                        const float f = fmaxf(fabsf(pf[x] - l[x]), fabsf(pf[x] - u[x]));
+                        m[c] += e * e + f * f;
+                    }
+                }
+                k = 2 * k + (m[1] < m[0] ? 1 : 0);
+            }
+            for (int q = k * kBucket; q < min((k + 1) * kBucket, t.s.T); ++q) {
+                const float4 S = t.sph[q];
+                const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z;
+                const float d2 = dx * dx + dy * dy + dz * dz;
+                if (d2 < near2) {
+                    near2 = d2;
+                    j = q;
+                }
+            }
+        }
+        const double* T = t.tris + 9 * j;
+        double best = point_tri_dist2(p, T, T + 3, T + 6);
+        if (!(best <= INFINITY)) best = INFINITY;   // a degenerate triangle never wins
+        // distance classes: below 1/128 of the box, then one per power of two
+        const float rel = sqrtf((float)best) * 128.f;
+        uint32_t cls = 0;
+        for (float lim = ext; cls < 7 && !(rel < lim); lim *= 2.f) ++cls;
+        key[i] = (cls << 21) | (c >> 9);   // kSeedKeyBits bits
+        idx[i] = (uint32_t)i;
+        d2_out[i] = best;
+        at_out[i] = (int32_t)j;
     }
-    const double* T = t.tris + 9 * j;
-    double best = point_tri_dist2(p, T, T + 3, T + 6);
-    if (!(best <= INFINITY)) best = INFINITY;   // a degenerate triangle never wins
-    // distance classes: below 1/128 of the box, then one per power of two
-    const float rel = sqrtf((float)best) * 128.f;
-    uint32_t cls = 0;
-    for (float lim = ext; cls < 7 && !(rel < lim); lim *= 2.f) ++cls;
-    key[i] = (cls << 21) | (c >> 9);   // kSeedKeyBits bits
-    idx[i] = (uint32_t)i;
-    d2_out[i] = best;
-    at_out[i] = (int32_t)j;
 }
 
 // bucket j of the frontier: its nodes are of `level`, each standing for the
@@ -1935,7 +1935,8 @@ __global__ __launch_bounds__(64 * kRimWaves) void k_rim(const RimEdge* __restric
     __shared__ long long sum[kRimWaves][64];
     __shared__ int bad[kRimWaves][64];
     const int lane = threadIdx.x & 63, wave = wave_uniform((int)(threadIdx.x >> 6));
-    const int64_t i = (int64_t)blockIdx.x * 64 + lane, at = i < N ? i : N - 1;
+    for (int64_t i0 = (int64_t)blockIdx.x * 64; i0 < N; i0 += (int64_t)gridDim.x * 64) {
+    const int64_t i = i0 + lane, at = i < N ? i : N - 1;
     const double p[3] = {pts[3 * at], pts[3 * at + 1], pts[3 * at + 2]};
     const int c = cross[at], w = (c >> 1) & 3;
     const float sg = (c & 1) ? 1.f : -1.f;
@@ -1960,10 +1961,11 @@ __global__ __launch_bounds__(64 * kRimWaves) void k_rim(const RimEdge* __restric
             unsure = true;
         acc += (long long)(int)(atan2_fit(num, den) * 134217728.f);
     }
+    __syncthreads();   // the points before have been read
     sum[wave][lane] = acc;
     bad[wave][lane] = unsure ? 1 : 0;
     __syncthreads();
-    if (wave != 0) return;
+    if (wave != 0) continue;
     for (int k = 1; k < kRimWaves; ++k) {
         acc += sum[k][lane];
         unsure = unsure || bad[k][lane] != 0;
@@ -1973,9 +1975,9 @@ __global__ __launch_bounds__(64 * kRimWaves) void k_rim(const RimEdge* __restric
     if (!(fabs(wn - 0.5) > 1e-5 + 1e-7 * n)) unsure = true;
     const uint64_t mu = __ballot(mine && unsure);
     if (mu != 0ull && lane == 0) atomicAdd(undecided, (unsigned)__popcll(mu));
-    if (!mine) return;
-    if (unsure) decided[i] = 0;
-    else if (wn > 0.5) out[i] = -out[i];
+    if (mine && unsure) decided[i] = 0;
+    else if (mine && wn > 0.5) out[i] = -out[i];
+    }
 }
 
 __global__ __launch_bounds__(kT) void k_sdf_wind(TreeView t, const double* pts, int64_t N, double* out,
@@ -2087,11 +2089,11 @@ void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* 
     const bool packets = N >= kPacketPoints && N < (int64_t(1) << 32);
     DBuf<uint32_t> key(N), order(N), rest;
     DBuf<int32_t> seed_at(N);
-    hipLaunchKernelGGL(k_pt_seed, dim3(blocks_for(N, kT)), dim3(kT), 0, st, tr.view(), d_pts, N, key.p, order.p, d_out,
+    hipLaunchKernelGGL(k_pt_seed, dim3(strided_blocks(N, kT, kT)), dim3(kT), 0, st, tr.view(), d_pts, N, key.p, order.p, d_out,
                        seed_at.p);
     ITS_LAUNCH_CHECK();
     unsigned* counts = (unsigned*)tr.counts.p + 2;   // passed on, twice, and undecided
-    const unsigned pgrid = (unsigned)((N + kPk - 1) / kPk);
+    const unsigned pgrid = strided_blocks(N, kPk, 64);   // a packet a block
     Work all{N, nullptr, nullptr}, left = all;
     if (packets) {
         radix_sort(key, &order, N, kSeedKeyBits, st);
@@ -2134,7 +2136,8 @@ void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* 
                            decided.p, cross.p, counts + 2, (uint32_t*)nullptr, (unsigned*)nullptr);
         ITS_LAUNCH_CHECK();
         if (open) {
-            hipLaunchKernelGGL(k_rim, dim3(blocks_for(N, 64)), dim3(64 * kRimWaves), 0, st, (const RimEdge*)tr.rim.p,
+            hipLaunchKernelGGL(k_rim, dim3(grid_of((const void*)k_rim, 64 * kRimWaves, (N + 63) / 64)),
+                               dim3(64 * kRimWaves), 0, st, (const RimEdge*)tr.rim.p,
                                rim, d_pts, N, d_out, decided.p, (const int*)cross.p, counts + 2);
             ITS_LAUNCH_CHECK();
         }

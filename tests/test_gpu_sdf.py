@@ -321,6 +321,45 @@ def test_sdf_rim_signs(ctx, kind, N):
     assert np.array_equal(np.signbit(d)[sure], (w > 0.5)[sure])
 
 
+def test_sdf_rim_many_points(ctx):
+    """More points than the rim kernel's resident blocks take at once: the
+    same points in calls that need one round, bit for bit."""
+    V, F = _rim_mesh("patch")
+    rng = np.random.default_rng(8)
+    N = 300_007
+    P = rng.uniform(V.min(0) - 0.1, V.max(0) + 0.1, (N, 3))
+    print(f"[rim] patch T={len(F)} N={N}", flush=True)
+    d = ctx.signed_distance(V, F, P)
+    one = np.concatenate([ctx.signed_distance(V, F, p) for p in np.array_split(P, 10)])
+    clear = np.abs(d) > 1e-9
+    np.testing.assert_array_equal(np.abs(d), np.abs(one))
+    np.testing.assert_array_equal(np.signbit(d[clear]), np.signbit(one[clear]))
+
+
+def test_sdf_points_beyond_a_launch(ctx):
+    """2^29 + 3 points (13 GB) around a mesh with a boundary: more work items
+    than one launch dimension holds, for the rim kernel.  The points are one
+    set of 2^20 over and over, so the results are that set's."""
+    import psutil
+    if psutil.virtual_memory().available < 40 << 30:
+        pytest.skip("needs 40 GiB of host memory")
+    V, F = _rim_mesh("patch")
+    rng = np.random.default_rng(4)
+    B, N = 1 << 20, (1 << 29) + 3
+    T = rng.uniform(V.min(0) - 0.2, V.max(0) + 0.2, (B, 3))
+    base = ctx.signed_distance(V, F, T)
+    P = np.empty((N, 3))
+    for s in range(0, N, B):
+        P[s:s + B] = T[:min(B, N - s)]
+    print(f"[sdf] N={N}", flush=True)
+    d = ctx.signed_distance(V, F, P)
+    clear = np.abs(base) > 1e-9
+    for s in range(0, N, B):
+        n = min(B, N - s)
+        assert np.array_equal(np.abs(d[s:s + n]), np.abs(base[:n]))
+        assert np.array_equal(d[s:s + n][clear[:n]], base[:n][clear[:n]])
+
+
 @pytest.mark.parametrize("hole", [False, True])
 def test_sdf_many_half_edges(ctx, hole):
     """Above 2^23 half edges they are sorted, not hashed, to find the boundary:
