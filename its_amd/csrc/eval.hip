@@ -135,20 +135,20 @@ __device__ inline float with_link(float v, const RankWord* below, uint32_t m, in
 // once, whole lines at a time, links included.
 __global__ void k_fill_blocks(int64_t n, FieldLevels F, const RankWord* cells, const uint32_t* code,
                               const double* lambda, float* blocks) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const int64_t i = t >> 3;
-    const int k = (int)(t & 7);
-    const int d = level_of(F.first, F.n, i);
-    const uint32_t m = code[i];
-    uint32_t x, y, z;
-    demorton3(m, x, y, z);
-    const uint32_t D = (uint32_t)max(1, F.R0 >> d) + 1u;
-    const uint32_t key = ((x + (k & 1)) * D + (y + ((k >> 1) & 1))) * D + (z + ((k >> 2) & 1));
-    const uint32_t r = bit_find(F.lattice[d], key);
-    float v = r != ITS_NONE ? (float)lambda[F.voff[d] + r] : 0.f;
-    if (d > 0 && d < F.lc) v = with_link(v, cells + F.word[d - 1], m, k);
-    blocks[t] = v;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t i = t >> 3;
+        const int k = (int)(t & 7);
+        const int d = level_of(F.first, F.n, i);
+        const uint32_t m = code[i];
+        uint32_t x, y, z;
+        demorton3(m, x, y, z);
+        const uint32_t D = (uint32_t)max(1, F.R0 >> d) + 1u;
+        const uint32_t key = ((x + (k & 1)) * D + (y + ((k >> 1) & 1))) * D + (z + ((k >> 2) & 1));
+        const uint32_t r = bit_find(F.lattice[d], key);
+        float v = r != ITS_NONE ? (float)lambda[F.voff[d] + r] : 0.f;
+        if (d > 0 && d < F.lc) v = with_link(v, cells + F.word[d - 1], m, k);
+        blocks[t] = v;
+    }
 }
 
 struct EvalParams {
@@ -962,7 +962,7 @@ void field_build(its_svo s) {
     ITS_REQUIRE(s->orphan_level + 1 >= lc, ITS_E_STATE, "marked cell without a marked parent");
     const int64_t n = 8 * s->cell_first[s->depth];
     if (n > 0) {
-        hipLaunchKernelGGL(k_fill_blocks, dim3(blocks_for(n, kT)), dim3(kT), 0, st, n, field_levels(s, lc),
+        hipLaunchKernelGGL(k_fill_blocks, dim3(strided_blocks(n, kT, kT)), dim3(kT), 0, st, n, field_levels(s, lc),
                            (const RankWord*)s->cells.p, (const uint32_t*)s->cell_code.p, (const double*)s->lambda64.p,
                            (float*)s->blocks.p);
         ITS_LAUNCH_CHECK();

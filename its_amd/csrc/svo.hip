@@ -286,26 +286,27 @@ __global__ void k_nodes(Tree T, const RankWord* occ, const uint32_t* codes, Node
 // thread per (node, neighbour slot), so a wavefront stores 64 consecutive
 // entries of the 27-per-node table.
 __global__ void k_neighbors(Tree T, const RankWord* occ, const uint32_t* codes, const uint32_t* morton, uint32_t* nb) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 27 * T.node[T.depth]) return;
-    const int64_t g = t / 27;
-    const int k = (int)(t - 27 * g);
-    uint32_t v = ITS_NONE;
-    if (k == 13) {
-        v = (uint32_t)g;
-    } else {
-        const int d = level_of(T.node, T.depth, g);
-        if (d + 1 < T.depth) {
-            uint32_t x, y, z;
-            demorton3(morton[g], x, y, z);
-            const uint32_t R = (uint32_t)(T.R0 >> d);
-            x += (uint32_t)(k % 3 - 1);
-            y += (uint32_t)((k / 3) % 3 - 1);
-            z += (uint32_t)(k / 9 - 1);
-            if (x < R && y < R && z < R) v = node_of(T, occ, codes, d, morton3(x, y, z));
+    const int64_t n = 27 * T.node[T.depth], step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += step) {
+        const int64_t g = t / 27;
+        const int k = (int)(t - 27 * g);
+        uint32_t v = ITS_NONE;
+        if (k == 13) {
+            v = (uint32_t)g;
+        } else {
+            const int d = level_of(T.node, T.depth, g);
+            if (d + 1 < T.depth) {
+                uint32_t x, y, z;
+                demorton3(morton[g], x, y, z);
+                const uint32_t R = (uint32_t)(T.R0 >> d);
+                x += (uint32_t)(k % 3 - 1);
+                y += (uint32_t)((k / 3) % 3 - 1);
+                z += (uint32_t)(k / 9 - 1);
+                if (x < R && y < R && z < R) v = node_of(T, occ, codes, d, morton3(x, y, z));
+            }
         }
+        nb[t] = v;
     }
-    nb[t] = v;
 }
 
 // -------------------------------------------------------------- vertices ----
@@ -523,7 +524,7 @@ void svo_build(its_svo s, const double* d_tris, int64_t n_tris) {
     hipLaunchKernelGGL(k_mark_corners, dim3(blocks_for(items, kT)), dim3(kT), 0, st, T, codes, s->lattice.p);
     ITS_LAUNCH_CHECK();
     // queued behind the marks, in front of the read-back
-    hipLaunchKernelGGL(k_neighbors, dim3(blocks_for(27 * total, kT)), dim3(kT), 0, st, T, d_occ, codes,
+    hipLaunchKernelGGL(k_neighbors, dim3(strided_blocks(27 * total, kT, kT)), dim3(kT), 0, st, T, d_occ, codes,
                        (const uint32_t*)s->morton.p, s->neighbors.p);
     ITS_LAUNCH_CHECK();
     const std::vector<int64_t> vert = rank_levels(s->lattice.p, S, lat_words, st);
