@@ -54,12 +54,23 @@ __global__ void k_tri_count(const double* tris, int64_t T, Grid g, uint64_t* cnt
     cnt[t] = (uint64_t)(be[0] - bo[0] + 1) * (uint64_t)(be[1] - bo[1] + 1) * (uint64_t)(be[2] - bo[2] + 1);
 }
 
-// first triangle of every 256 candidates
-__global__ void k_cand_starts(const uint64_t* off, int64_t T, uint64_t total, uint32_t* start) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= T) return;
-    const uint64_t c0 = off[t], c1 = t + 1 < T ? off[t + 1] : total;
-    for (uint64_t b = (c0 + kT - 1) / kT; b * kT < c1; ++b) start[b] = (uint32_t)t;
+// First triangle of every 256 candidates: the last whose offset is not beyond
+// theirs.  One thread per entry, so that a triangle with many candidates takes no
+// longer than the others.  One thread per triangle, writing its run of entries,
+// took 2.5 us where this takes 7.3 (200,000 small triangles at 256^3), but 1.4 ms
+// for 3 on a slanted tetrahedron at 256^3 and 79 ms for 0.02 at 1024^3.
+__global__ void k_cand_starts(const uint64_t* off, int64_t T, uint64_t entries, uint32_t* start) {
+    const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; b < entries; b += step) {
+        const uint64_t c = b * kT;
+        int64_t lo = 0, hi = T - 1;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi + 1) >> 1;
+            if (off[mid] <= c) lo = mid;
+            else hi = mid - 1;
+        }
+        start[b] = (uint32_t)lo;
+    }
 }
 
 // One thread per (triangle, candidate voxel); the triangle set-up is
@@ -448,9 +459,10 @@ void svo_build(its_svo s, const double* d_tris, int64_t n_tris) {
         const uint64_t total = scan_exclusive_u64(cnt.p, cnt.p, n_tris, st);
         if (total) {
             unsigned nb = (unsigned)std::min<uint64_t>((total + kT - 1) / kT, 1u << 20);
-            DBuf<uint32_t> start((total + kT - 1) / kT);
-            hipLaunchKernelGGL(k_cand_starts, dim3(blocks_for(n_tris, kT)), dim3(kT), 0, st, (const uint64_t*)cnt.p,
-                               n_tris, total, start.p);
+            const int64_t entries = (int64_t)((total + kT - 1) / kT);
+            DBuf<uint32_t> start(entries);
+            hipLaunchKernelGGL(k_cand_starts, dim3(strided_blocks(entries, kT, kT)), dim3(kT), 0, st,
+                               (const uint64_t*)cnt.p, n_tris, (uint64_t)entries, start.p);
             ITS_LAUNCH_CHECK();
             hipLaunchKernelGGL(k_voxelize, dim3(nb), dim3(kT), 0, st, d_tris, n_tris, (const uint64_t*)cnt.p, total,
                                (const uint32_t*)start.p, g, occ.p);

@@ -49,6 +49,24 @@ def test_svo_bit_exact(ctx, name, R):
     np.testing.assert_array_equal(vox, O.voxelize(c.tris, c.origin, c.width, R))
 
 
+@pytest.mark.parametrize("sizes", [(1, 0), (0, 300), (1, 300), (3, 40)])
+def test_voxels_of_large_and_small_triangles(ctx, sizes):
+    """Slanted triangles across the whole grid (up to 1,024 runs of 256
+    candidates each) among small ones (many to a run): the oracle's voxels."""
+    from its_amd import _capi
+    large, small = sizes
+    rng = np.random.default_rng(10 * large + small)
+    far = np.array([[0, 0, 0], [1, 1, 0.1], [0.9, 0.1, 1]])
+    tri = [far + 0.02 * rng.standard_normal((3, 3)) for _ in range(large)]
+    tri += [rng.uniform(0, 1, (1, 3)) + 0.01 * rng.standard_normal((3, 3)) for _ in range(small)]
+    tris = np.array([tri[k] for k in rng.permutation(len(tri))])
+    o = np.full(3, -0.1)
+    w = np.full(3, 1.2)
+    print(f"[svo] {large} large and {small} small triangles", flush=True)
+    g = _capi.Octree(ctx, tris, o, w, 64)
+    np.testing.assert_array_equal(g.voxels(), O.voxelize(tris, o, w, 64))
+
+
 def test_svo_structural_invariants(ctx):
     """Size-independent checks at the full depth-8 torus-knot size (200k triangles)."""
     from its_amd import _capi
