@@ -18,6 +18,7 @@
 #include <thread>
 #include <vector>
 
+#include "batch_split.hpp"
 #include "fit.hpp"
 #include "lscg_batch.hpp"
 
@@ -287,47 +288,6 @@ static void sync_octree_streams(its_batch b) {
     }
 }
 
-namespace {
-// Which of the meshes that may share the one-launch fit do (cand, sizes
-// ascending on return): the largest go to the many-mesh solver while that
-// makes the slower of the two, which run side by side, faster.  Estimates, in
-// ms, from measured fits:
-//   - one workgroup takes 0.17 + 0.2 per 1,000 unknowns, 256 meshes at a
-//     time (0.19 ms at 160 unknowns, 0.66 at 3,668, 1.97 at 14,110, 6.1 at
-//     31,101 with more iterations, 8.7 at 55,852);
-//   - the many-mesh solver takes 0.055 depth^2 for its chain of launches
-//     (0.83 ms at depth 3, 1.8 at 6, 2.7 at 7) and 1.1 per million unknowns
-//     in all (5.8 ms for 256 meshes of 14,110).
-// 24 meshes of 14,282 to 131,176 unknowns: all under the cap in one launch
-// 6.1 ms, chosen so 5.0; 6 meshes of 7,165 to 55,852: 8.7 and 2.7.
-int one_launch_count(its_batch b, std::vector<int>& cand, const std::vector<int>& big) {
-    std::stable_sort(cand.begin(), cand.end(),
-                     [&](int x, int y) { return b->svos[x]->num_verts < b->svos[y]->num_verts; });
-    double unknowns = 0;
-    int depth = 0;
-    for (int m : big) {
-        unknowns += (double)b->svos[m]->num_verts;
-        depth = std::max(depth, b->svos[m]->depth);
-    }
-    int best = (int)cand.size();
-    double best_ms = INFINITY;
-    for (int k = (int)cand.size(); k >= 0; --k) {   // the k smallest in one launch
-        if (k < (int)cand.size()) {
-            unknowns += (double)b->svos[cand[k]]->num_verts;
-            depth = std::max(depth, b->svos[cand[k]]->depth);
-        }
-        const double one = k ? (0.17 + 2e-4 * (double)b->svos[cand[k - 1]]->num_verts) * ((k + 255) / 256) : 0.0;
-        const double many = unknowns > 0 ? 0.055 * depth * depth + 1.1e-6 * unknowns : 0.0;
-        const double ms = std::max(one, many);
-        if (ms < best_ms) {
-            best_ms = ms;
-            best = k;
-        }
-    }
-    return best;
-}
-}  // namespace
-
 // Fit every mesh of the batch.  Of the meshes with at most
 // ITS_TUNE_BATCH_MAX_VERTS unknowns, the smaller ones are solved together by
 // the one-launch kernel (graph-captured, replayed on later calls) on the
@@ -347,7 +307,14 @@ void batch_fit(its_batch b, double tol, int64_t max_iter, bool warm, its_lscg_st
         ITS_REQUIRE(!warm || s->has_lambda, ITS_E_STATE, "warm batch fit needs coefficients on every mesh");
         (s->num_verts <= cap ? small : big).push_back(m);
     }
-    const int one = one_launch_count(b, small, big);
+    std::stable_sort(small.begin(), small.end(),
+                     [&](int x, int y) { return b->svos[x]->num_verts < b->svos[y]->num_verts; });
+    auto sizes = [&](const std::vector<int>& meshes) {
+        std::vector<SplitMesh> v;
+        for (int m : meshes) v.push_back(SplitMesh{b->svos[m]->num_verts, b->svos[m]->depth});
+        return v;
+    };
+    const int one = one_launch_count(sizes(small), sizes(big), kManyMost);
     big.insert(big.end(), small.begin() + one, small.end());
     small.resize(one);
     std::sort(small.begin(), small.end());   // batch order, whatever the split

@@ -28,8 +28,7 @@ namespace {
 
 constexpr int kT = kFitT;
 constexpr int kChunk = 4;        // binary32 iterations per graph launch
-constexpr int kMeshBits = 12;    // block table entry: octree << 20 | block
-constexpr int kBlockBits = 20;
+constexpr int kBlockBits = 32 - kMeshBits;
 
 struct MeshDesc {
     int64_t n;
@@ -255,7 +254,7 @@ struct Launcher {
 static void many_prepare(ManySolve& ms, const std::vector<its_svo>& svos, hipStream_t st) {
     AllocStream as(st);
     const int M = (int)svos.size();
-    ITS_REQUIRE(M > 0 && M < (1 << kMeshBits), ITS_E_RANGE, "too many octrees for one many-mesh solve");
+    ITS_REQUIRE(M > 0 && M <= kManyMost, ITS_E_RANGE, "too many octrees for one many-mesh solve");
     std::vector<MeshDesc> h(M);
     ms.ctl.ensure(4 * (size_t)M);
     ms.act.ensure(M);

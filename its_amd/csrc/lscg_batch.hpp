@@ -7,6 +7,9 @@
 
 namespace its {
 
+constexpr int kMeshBits = 12;                      // block table entry: octree << 20 | block
+constexpr int kManyMost = (1 << kMeshBits) - 1;    // octrees of one solve
+
 // Device state of a many-octree solve, kept between calls: the descriptors,
 // block tables and the captured iteration graph are rebuilt only when the
 // set of octrees or one of their solver states changes.
