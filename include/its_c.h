@@ -288,13 +288,15 @@ int its_lscg_solve_mlp(its_ctx ctx, its_svo svo, its_mlp net, const double* b, d
  *      one model per process) ----
  * A batch holds octrees, each with its right-hand side
  * (its_sdf_at_vertices).  its_batch_fit solves small meshes (at most
- * ITS_TUNE_BATCH_MAX_VERTS unknowns, and among those the ones that would not
- * hold the others up) in one persistent launch (one workgroup
+ * ITS_TUNE_BATCH_MAX_VERTS unknowns) in one persistent launch (one workgroup
  * per mesh runs that mesh's whole mixed-precision LSCG, the algorithm and
- * stopping rule of its_lscg_solve), captured once as a hipGraph and replayed
- * on later calls; the larger meshes run at the same time through the
- * many-mesh solver (one launch per solver pass for all of them; per mesh the
- * coefficients and statistics of its_lscg_solve, bit for bit).
+ * stopping rule of its_lscg_solve, with its result to the solver tolerance),
+ * captured once as a hipGraph and replayed on later calls; the larger meshes
+ * run at the same time through the many-mesh solver (one launch per solver
+ * pass for all of them; per mesh the coefficients and statistics of
+ * its_lscg_solve, bit for bit).  With the cap at its default, meshes below it
+ * that would hold the launch up also go to the many-mesh solver: which ones
+ * depends on all sizes and depths of the batch.  its_batch_solvers tells.
  * stats: one per mesh; seconds: wall time of the fit.  warm != 0 starts
  * every mesh from its current coefficients.  The coefficients stay on the
  * octrees; their evaluation fields are rebuilt by its_batch_fields (octrees
@@ -310,6 +312,10 @@ int its_batch_destroy(its_batch b);
  * their streams before reading them. */
 int its_batch_add(its_batch b, its_svo svo);
 int its_batch_fit(its_batch b, double tol, int64_t max_iter, int warm, its_lscg_stats* stats, double* seconds);
+/* one_launch[m] = 1 where the last its_batch_fit solved mesh m in the one
+ * launch, 0 where the many-mesh solver did; ITS_E_STATE without a fit of the
+ * present meshes */
+int its_batch_solvers(its_batch b, uint8_t* one_launch);
 int its_batch_fields(its_batch b);
 int its_batch_eval_device(its_batch b, const float* d_x, const float* d_y, const float* d_z, const int64_t* offsets,
                           float out_val, float* d_f, double* seconds);
@@ -346,7 +352,9 @@ int its_batch_eval_device_noalloc(its_batch b, const float* d_x, const float* d_
  *   gathered per wavefront in LDS and walked 64 at a time; 0 = every thread
  *   walks its own query (default 1).
  * ITS_TUNE_BATCH_MAX_VERTS: meshes of a batch with at most this many
- *   unknowns may share the one-launch fit (default 65536).
+ *   unknowns share the one-launch fit.  At the default, 65536, some of them may
+ *   go to the many-mesh solver (its_batch_fit); at any other value this size
+ *   alone decides, and no mesh's solver depends on the rest of the batch.
  * ITS_TUNE_SDF_RAY: 1 = for a closed, consistently oriented mesh, and for one
  *   with a short boundary (at most one uncancelled half edge per two triangles,
  *   and 4,096), the sign of

@@ -147,6 +147,7 @@ SIGNATURES = {
     "its_batch_destroy": [vp],
     "its_batch_add": [vp, vp],
     "its_batch_fit": [vp, C.c_double, C.c_int64, C.c_int, vp, C.POINTER(C.c_double)],
+    "its_batch_solvers": [vp, vp],
     "its_batch_fields": [vp],
     "its_batch_eval_device": [vp, vp, vp, vp, np.ctypeslib.ndpointer(dtype=np.int64, flags="C_CONTIGUOUS"), C.c_float,
                               vp, C.POINTER(C.c_double)],
@@ -582,6 +583,12 @@ class Batch:
         sec = C.c_double(0)
         check(lib().its_batch_fit(self._h, tol, int(max_iter), 1 if warm else 0, C.cast(st, vp), C.byref(sec)))
         return [s.as_dict() for s in st], sec.value
+
+    def one_launch(self):
+        """Per mesh: whether the last fit solved it in the one launch (else the many-mesh solver)."""
+        out = np.zeros(max(len(self.octrees), 1), np.uint8)
+        check(lib().its_batch_solvers(self._h, out.ctypes.data_as(vp)))
+        return out[: len(self.octrees)].astype(bool)
 
     def fields(self):
         check(lib().its_batch_fields(self._h))

@@ -250,6 +250,7 @@ struct its_batch_s {
     hipStream_t side = nullptr;       // the one-launch fit runs here, beside the large meshes
     std::vector<its::FitDesc> host;   // the descriptors the graph was captured with
     its::ManySolve large;             // the large meshes' solve, on the context stream
+    std::vector<uint8_t> one_launch;  // per mesh: solved in the one launch by the last fit
     ~its_batch_s() {
         // no stream may still use the buffers freed below
         if (side) (void)hipStreamSynchronize(side);
@@ -288,10 +289,10 @@ static void sync_octree_streams(its_batch b) {
     }
 }
 
-// Fit every mesh of the batch.  Of the meshes with at most
-// ITS_TUNE_BATCH_MAX_VERTS unknowns, the smaller ones are solved together by
-// the one-launch kernel (graph-captured, replayed on later calls) on the
-// batch's own stream; larger meshes, whose solve on one workgroup would bound
+// Fit every mesh of the batch.  Meshes with at most ITS_TUNE_BATCH_MAX_VERTS
+// unknowns (of these the smaller ones, with the cap at its default) are solved
+// together by the one-launch kernel (graph-captured, replayed on later calls) on
+// the batch's own stream; larger meshes, whose solve on one workgroup would bound
 // the launch, run at the same time on the context stream through the
 // many-mesh solver (one launch per solver pass for all of them).  seconds:
 // wall time of the whole fit.
@@ -307,18 +308,21 @@ void batch_fit(its_batch b, double tol, int64_t max_iter, bool warm, its_lscg_st
         ITS_REQUIRE(!warm || s->has_lambda, ITS_E_STATE, "warm batch fit needs coefficients on every mesh");
         (s->num_verts <= cap ? small : big).push_back(m);
     }
-    std::stable_sort(small.begin(), small.end(),
-                     [&](int x, int y) { return b->svos[x]->num_verts < b->svos[y]->num_verts; });
-    auto sizes = [&](const std::vector<int>& meshes) {
-        std::vector<SplitMesh> v;
-        for (int m : meshes) v.push_back(SplitMesh{b->svos[m]->num_verts, b->svos[m]->depth});
-        return v;
-    };
-    const int one = one_launch_count(sizes(small), sizes(big), kManyMost);
-    big.insert(big.end(), small.begin() + one, small.end());
-    small.resize(one);
-    std::sort(small.begin(), small.end());   // batch order, whatever the split
-    std::sort(big.begin(), big.end());
+    if (cap == kBatchMaxVerts) {   // a caller's own cap is the whole rule
+        std::stable_sort(small.begin(), small.end(),
+                         [&](int x, int y) { return b->svos[x]->num_verts < b->svos[y]->num_verts; });
+        auto sizes = [&](const std::vector<int>& meshes) {
+            std::vector<SplitMesh> v;
+            for (int m : meshes) v.push_back(SplitMesh{b->svos[m]->num_verts, b->svos[m]->depth});
+            return v;
+        };
+        const int one = one_launch_count(sizes(small), sizes(big), kManyMost);
+        big.insert(big.end(), small.begin() + one, small.end());
+        small.resize(one);
+        std::sort(small.begin(), small.end());   // batch order, whatever the split
+        std::sort(big.begin(), big.end());
+    }
+    b->one_launch.clear();   // until the fit has run
     const int ns = (int)small.size();
     std::vector<FitDesc> h(ns);
     b->stats.ensure(8 * (int64_t)std::max(ns, 1));
@@ -422,6 +426,14 @@ void batch_fit(its_batch b, double tol, int64_t max_iter, bool warm, its_lscg_st
         b->svos[m]->has_lambda = true;
         b->svos[m]->field_ready = false;
     }
+    b->one_launch.assign(count, 0);
+    for (int m : small) b->one_launch[m] = 1;
+}
+
+void batch_solvers(its_batch b, uint8_t* one_launch) {
+    ITS_REQUIRE(!b->svos.empty() && b->one_launch.size() == b->svos.size(), ITS_E_STATE,
+                "the batch's meshes have not been fitted");
+    std::copy(b->one_launch.begin(), b->one_launch.end(), one_launch);
 }
 
 // Rebuild the evaluation fields after a batch fit, each on its octree's

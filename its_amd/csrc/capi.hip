@@ -16,7 +16,7 @@ namespace its {
 static thread_local std::string g_last_error;
 void set_last_error(const std::string& msg) { g_last_error = msg; }
 
-static int64_t g_tune[ITS_TUNE_COUNT] = {32768, 64, 2048, 1, 1, 65536, 1};
+static int64_t g_tune[ITS_TUNE_COUNT] = {32768, 64, 2048, 1, 1, kBatchMaxVerts, 1};
 int64_t tune_get(int key) { return g_tune[key]; }
 
 // A copy to pageable memory runs at 18 GB/s here (29.3 MB in 1.63 ms), one to
@@ -841,6 +841,12 @@ int its_batch_fit(its_batch b, double tol, int64_t max_iter, int warm, its_lscg_
     DeviceGuard g(batch_ctx(b)->device);
     AllocStream as(batch_ctx(b)->stream);
     batch_fit(b, tol, max_iter, warm != 0, stats, seconds);
+    ITS_API_END
+}
+int its_batch_solvers(its_batch b, uint8_t* one_launch) {
+    ITS_API_BEGIN
+    ITS_REQUIRE(b && one_launch, ITS_E_INVALID, "bad arguments");
+    batch_solvers(b, one_launch);
     ITS_API_END
 }
 int its_batch_fields(its_batch b) {

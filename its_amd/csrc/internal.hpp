@@ -129,6 +129,8 @@ struct its_svo_s {
 namespace its {
 // call before writing lambda64 or rebuilding the field
 inline void lambda_changing(its_svo s) { ++s->lambda_version; }
+// default of ITS_TUNE_BATCH_MAX_VERTS, with which a batch is also split by estimates (batch_split.hpp)
+constexpr int64_t kBatchMaxVerts = 65536;
 // tunables (capi.hip)
 int64_t tune_get(int key);
 // device to caller memory; returns when the bytes are there (capi.hip)
@@ -185,6 +187,7 @@ void face_corners(const double* d_V, const int32_t* d_F, int64_t nF, double* d_t
 bool value_range(const float* d_f, int64_t n, float range[2], hipStream_t st);
 // batch.hip
 its_batch batch_new(its_ctx ctx);
+void batch_solvers(its_batch b, uint8_t* one_launch);
 void batch_delete(its_batch b);
 void batch_add(its_batch b, its_svo s);
 void batch_fit(its_batch b, double tol, int64_t max_iter, bool warm, its_lscg_stats* out, double* seconds);
