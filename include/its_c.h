@@ -152,7 +152,8 @@ int its_collocation_mul(its_ctx ctx, its_svo svo, const double* x, double* y, in
  * the matrix-free operator's parent lists, the levels (and how many of them
  * the one-workgroup kernels take), and the bytes one CGLS iteration moves:
  * 16 B per non-zero + 72 B per row for the assembled matrix, and this
- * library's matrix-free count (89 B per vertex + 16 B per parent entry). */
+ * library's matrix-free count (89 B per vertex + 44 B per vertex above the
+ * finest level + 8 B per parent entry). */
 typedef struct {
     int64_t n;
     int64_t nnz;

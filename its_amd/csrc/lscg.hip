@@ -638,11 +638,13 @@ void lscg_structure(its_svo s, its_lscg_structure* out) {
     S.levels = f->L;
     S.block_levels = f->L - f->lc;
     S.bytes_assembled_per_iteration = 16.0 * (double)nnz + 72.0 * (double)n;
-    // per vertex: prolongation p r/w, z, list offset, g (20 B); t = D g with
+    // per vertex: prolongation p r/w, z, parent columns, g (32 B); t = D g with
     // its index and gather (12 B); the update of x, r along the chains, h
-    // (33 B); restriction offset and h r/w (12 B); preconditioner h, 1/d, z
-    // (12 B).  Per parent entry: index and value, once down and once up (16 B).
-    S.bytes_matrix_free_per_iteration = 89.0 * (double)n + 16.0 * (double)f->entries;
+    // (33 B); preconditioner h, 1/d, z (12 B).  Per vertex with children: their
+    // nine columns and h r/w (44 B).  Per parent entry: the value, once down and
+    // once up (8 B).
+    const double kids = f->L > 1 ? (double)(n - f->off[1]) : 0.0;
+    S.bytes_matrix_free_per_iteration = 89.0 * (double)n + 44.0 * kids + 8.0 * (double)f->entries;
     *out = S;
 }
 

@@ -80,3 +80,11 @@ def test_assembled_nnz_matches_oracle(ctx, name, R):
     st = g.lscg_structure()
     assert st["n"] == F.A.n and st["nnz"] == F.A.nnz
     assert st["bytes_assembled_per_iteration"] == 16.0 * F.A.nnz + 72.0 * F.A.n
+    # the operator's lists: 2 parents per odd lattice coordinate below the root
+    # level; a 16-byte word of parent columns per vertex, nine 4-byte columns
+    # per vertex with children
+    key, level = g.vert_lattice()
+    odd = (key & 1).sum(1)[level < g.depth - 1]
+    assert st["parent_entries"] == (1 << odd).sum()
+    assert st["bytes_matrix_free_per_iteration"] == (
+        (16 + 73) * F.A.n + (36 + 8) * (level > 0).sum() + 8 * (1 << odd).sum())
