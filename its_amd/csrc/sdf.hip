@@ -1917,13 +1917,17 @@ __global__ __launch_bounds__(64, 5) void k_ray_packet(TreeView t, const double* 
 // sg the ray's direction on its axis and alpha taken without cancellation.  It
 // jumps by 2 pi where the ray crosses the edge, as the count does.  Left to the
 // fan walk (decided = 0): points whose ray passes an edge so closely that
-// binary32 may jump on the other side, and winding numbers within the sum's
-// error of 1/2 (1e-7 an edge, and 1e-5).  Angles are summed in multiples of
-// 2^-27, so the sum does not depend on the edges' order.
+// binary32 may jump on the other side, and winding numbers within 1e-5 and 1e-7
+// an edge of 1/2, the sum's error away from the boundary.  One angle's error
+// grows with the inverse of the point's distance to its edge: at 1e-3 of the
+// edge's length it is mostly 1e-6 turns, but up to 3e-4, at 1e-4 up to 7e-3, so a
+// point that close to the boundary and that close to 1/2 can get either sign, as
+// it can from the fans, whose formula is no better there.  Angles are summed in
+// multiples of 2^-27, so the sum does not depend on the edges' order.
 //
 // 64 points a block; its wavefronts share the edges, which are uniform and come
-// by scalar loads.  Bound by vector instructions: 0.2 ns per (point, edge) in
-// all, 100 us per 100 edges at 500,000 points.  Knot tube with a hole, 20,000
+// by scalar loads.  Bound by vector instructions: 2 ps per (point, edge) over
+// the chip, 100 us per 100 edges at 500,000 points.  Knot tube with a hole, 20,000
 // triangles at 128^3: crossings 63 us and this kernel 13, where the fan walk took 1,065
 // and its fans 350 with their host step.
 constexpr int kRimWaves = 8;
