@@ -187,13 +187,15 @@ def test_sdf_ray_signs(ctx, name):
 
 
 @pytest.mark.parametrize("N", [32767, 32768, 32769, 50021])
-@pytest.mark.parametrize("name", ["icosphere", "open", "single", "nine"])
+@pytest.mark.parametrize("name", ["icosphere", "open", "single", "nine", "collapsed"])
 def test_sdf_packets(ctx, name, N):
     """Point sets walked in packets of 16 (from 32,768 points) against the
     same points in calls small enough to be walked one by one: identical bit
-    for bit, since both take the exact minimum and exact crossings.  Dense
-    points on the surface, a few far ones and coordinates that are huge,
-    infinite or NaN; meshes of one bucket, two buckets and many levels."""
+    for bit, since both take the exact minimum and exact crossings; and a
+    sample of them against the brute-force oracle.  Dense points on the
+    surface, a few far ones and coordinates that are huge, infinite or NaN;
+    meshes of one bucket, two buckets and many levels, and one with faces of no
+    area on chords of the sphere, with points around their centres."""
     from its_amd import meshes
     V, F = meshes.noisy_icosphere(seed=3, level=3)
     V = np.ascontiguousarray(V)
@@ -203,9 +205,18 @@ def test_sdf_packets(ctx, name, N):
         F = F[:1]
     elif name == "nine":
         F = F[:9]
+    chords = []
+    if name == "collapsed":
+        far = [(0, int(np.argmin(V @ V[0]))), (7, int(np.argmin(V @ V[7]))), (9, int(np.argmin(V @ V[9])))]
+        V = np.concatenate([V, [0.5 * (V[far[2][0]] + V[far[2][1]])]])
+        chords = [[far[0][0], far[0][0], far[0][1]], [far[1][0], far[1][1], far[1][1]],
+                  [far[2][0], len(V) - 1, far[2][1]]]
+        F = np.concatenate([F, chords])
     F = np.ascontiguousarray(F, np.int32)
     rng = np.random.default_rng(N)
     P = V[rng.integers(0, len(V), N)] + 0.03 * rng.standard_normal((N, 3))
+    for q, f in enumerate(chords):
+        P[30 + q::20] = V[f].mean(0) + 0.02 * rng.standard_normal(P[30 + q::20].shape)
     P[::97] = rng.uniform(-8, 8, size=(len(P[::97]), 3))
     P[5], P[777], P[-1] = [1e30, 0, 0], [np.inf, 0, 0], [np.nan, 0.1, 0.2]
     P[20:25] = V[F[0, 0]]   # ties between the triangles of a vertex
@@ -215,7 +226,8 @@ def test_sdf_packets(ctx, name, N):
     clear = np.abs(d) > 1e-9   # nearer, a point that rays leave undecided takes the binary32 fan sum
     np.testing.assert_array_equal(np.abs(d), np.abs(one))
     np.testing.assert_array_equal(np.signbit(d[clear]), np.signbit(one[clear]))
-    k = rng.choice(np.nonzero(np.isfinite(P).all(1) & (np.abs(P) < 1e3).all(1))[0], 300, replace=False)
+    k = rng.choice(np.nonzero(np.isfinite(P).all(1) & (np.abs(P) < 1e3).all(1))[0], 2000, replace=False)
+    assert np.isfinite(d[k]).all()
     assert np.abs(np.abs(d[k]) - np.abs(O.signed_distance(V, F, P[k]))).max() <= 1e-12
 
 
@@ -289,11 +301,11 @@ def _rim_mesh(kind):
 @pytest.mark.parametrize("N", [1, 63, 2000, 40001])
 @pytest.mark.parametrize("kind", ["patch", "holes", "flipped", "doubled", "limit", "over", "long", "too_long"])
 def test_sdf_rim_signs(ctx, kind, N):
-    """Meshes with a boundary: distances are the fan walk's bit for bit, signs
-    those of the winding number summed over all triangles in binary64, wherever
-    that is farther than 1e-4 from 1/2 (binary32 sums of 1,000 angles)."""
+    """Meshes with a boundary: distances are the brute-force oracle's (on a
+    sample), signs those of the winding number summed over all triangles in
+    binary64, wherever that is farther than 1e-4 from 1/2 (binary32 sums of 1,000
+    angles)."""
     import torch
-    from its_amd import _capi
     V, F = _rim_mesh(kind)
     rng = np.random.default_rng(N)
     lo, hi = V.min(0), V.max(0)
@@ -302,10 +314,6 @@ def test_sdf_rim_signs(ctx, kind, N):
     P[near] = V[rng.integers(len(V), size=near.sum())] + rng.normal(0, 0.01, (near.sum(), 3))
     print(f"[rim] {kind} T={len(F)} N={N}", flush=True)
     d = ctx.signed_distance(V, F, P)
-    old = _capi.tune_get(_capi.TUNE_SDF_RAY)
-    _capi.tune_set(_capi.TUNE_SDF_RAY, 0)
-    fan = ctx.signed_distance(V, F, P)
-    _capi.tune_set(_capi.TUNE_SDF_RAY, old)
     T, Q = torch.from_numpy(V[F]).cuda(), torch.from_numpy(P).cuda()
     w = torch.zeros(N, dtype=torch.float64, device="cuda")
     for s in range(0, N, 4000):
@@ -315,7 +323,9 @@ def test_sdf_rim_signs(ctx, kind, N):
         den = la * lb * lc + (a * b).sum(2) * lc + (b * c).sum(2) * la + (c * a).sum(2) * lb
         w[s:s + 4000] = torch.atan2(det, den).sum(1) / (2 * np.pi)
     w = w.cpu().numpy()
-    assert np.array_equal(np.abs(d), np.abs(fan))
+    assert np.isfinite(d).all()
+    k = rng.choice(N, min(N, 1000), replace=False)
+    assert np.abs(np.abs(d[k]) - np.abs(O.signed_distance(V, F, P[k]))).max() <= 1e-12
     sure = (np.abs(w - 0.5) > 1e-4) & (np.abs(d) > 1e-9)
     assert sure.mean() > 0.9
     assert np.array_equal(np.signbit(d)[sure], (w > 0.5)[sure])
