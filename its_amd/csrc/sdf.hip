@@ -1919,11 +1919,13 @@ __global__ __launch_bounds__(64, 5) void k_ray_packet(TreeView t, const double* 
 // fan walk (decided = 0): points whose ray passes an edge so closely that
 // binary32 may jump on the other side, and winding numbers within 1e-5 and 1e-7
 // an edge of 1/2, the sum's error away from the boundary.  One angle's error
-// grows with the inverse of the point's distance to its edge: at 1e-3 of the
-// edge's length it is mostly 1e-6 turns, but up to 3e-4, at 1e-4 up to 7e-3, so a
-// point that close to the boundary and that close to 1/2 can get either sign, as
-// it can from the fans, whose formula is no better there.  Angles are summed in
-// multiples of 2^-27, so the sum does not depend on the edges' order.
+// grows with the inverse of the point's distance to its edge: a million random
+// edges in binary32 against binary64 gave at most 1.3e-5 turns at 1e-3 of the
+// edge's length (mostly 6e-7) and 1.3e-4 at 1e-4, and rays that pass the edge
+// closely do worse.  So a point that close to the boundary and that close to 1/2
+// can get either sign, as it can from the fans, whose formula is no better there.
+// Angles are summed in multiples of 2^-27: the sum does not depend on the edges'
+// order.
 //
 // 64 points a block; its wavefronts share the edges, which are uniform and come
 // by scalar loads.  Bound by vector instructions: 2 ps per (point, edge) over
