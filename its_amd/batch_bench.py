@@ -9,8 +9,10 @@ lists and preconditioner per mesh, from several host threads with a
 context each (--build-threads); the fit of
 all meshes (its_batch_fit: the smaller meshes in one persistent
 graph-captured launch, the larger ones beside it through the many-mesh
-solver, one launch per solver pass for all of them); the evaluation fields
-with the autotuned collapse bound of each depth (its_batch_fields);
+solver, one launch per solver pass for all of them; its graphs are captured by
+a first call, reported beside the replay that counts); the evaluation fields
+with the autotuned collapse bound of each depth (its_batch_fields), first on
+octrees that have none, which counts, and once more as a rebuild;
 the evaluation of all meshes' queries in one launch (its_batch_eval_device).
 The same fits and evaluations also run mesh by mesh through the single-mesh
 entry points for comparison.  Prints one JSON line.
@@ -128,41 +130,47 @@ def main(argv=None):
     log(f"[batch] built {a.meshes} on {nthr} threads in {t_build_wall:.2f} s (summed per-call: octrees "
         f"{t_build:.2f} s, right-hand sides {t_rhs:.2f} s, solver setup {t_setup:.2f} s)")
 
-    # fit: mesh by mesh, then all in one launch
-    for it in items:
-        it["g"].lscg(it["b"], tol=1e-6)              # solver structures and graphs
-    seq_fit = 0.0
-    seq_stats = []
-    for it in items:
-        lam, st = it["g"].lscg(it["b"], tol=1e-6)
-        seq_fit += st["seconds"]
-        seq_stats.append(st)
-    batch = _capi.Batch(ctx)
-    for it in items:
-        batch.add(it["g"])
-    batch.fit(tol=1e-6)                              # captures the graph
-    stats, t_fit = batch.fit(tol=1e-6)
-    log(f"[batch] fit: one launch {t_fit * 1e3:.1f} ms vs mesh by mesh {seq_fit * 1e3:.1f} ms")
-
     # evaluation fields with the collapse bound of each depth: one
     # its_batch_fields call per bound (octrees of different contexts are
     # built side by side)
-    s0 = time.perf_counter()
-    groups = {}
+    def fields():
+        s0 = time.perf_counter()
+        groups = {}
+        for it in items:
+            bound = (table[it["depth"]]["dense_cells"] if table and it["depth"] in table
+                     else _capi.tune_get(_capi.TUNE_DENSE_CELLS))
+            groups.setdefault(int(bound), []).append(it)
+        old_bound = _capi.tune_get(_capi.TUNE_DENSE_CELLS)
+        for bound, group in sorted(groups.items()):
+            _capi.tune_set(_capi.TUNE_DENSE_CELLS, bound)
+            fb = _capi.Batch(ctx)
+            for it in group:
+                fb.add(it["g"])
+            fb.fields()
+            fb.close()
+        _capi.tune_set(_capi.TUNE_DENSE_CELLS, old_bound)
+        return time.perf_counter() - s0
+
+    # fit: all meshes together, and their first fields
+    batch = _capi.Batch(ctx)
     for it in items:
-        bound = (table[it["depth"]]["dense_cells"] if table and it["depth"] in table
-                 else _capi.tune_get(_capi.TUNE_DENSE_CELLS))
-        groups.setdefault(int(bound), []).append(it)
-    old_bound = _capi.tune_get(_capi.TUNE_DENSE_CELLS)
-    for bound, group in sorted(groups.items()):
-        _capi.tune_set(_capi.TUNE_DENSE_CELLS, bound)
-        fb = _capi.Batch(ctx)
-        for it in group:
-            fb.add(it["g"])
-        fb.fields()
-        fb.close()
-    _capi.tune_set(_capi.TUNE_DENSE_CELLS, old_bound)
-    t_fields = time.perf_counter() - s0
+        batch.add(it["g"])
+    _, t_fit_first = batch.fit(tol=1e-6)             # captures the graphs
+    stats, t_fit = batch.fit(tol=1e-6)
+    one_launch = int(batch.one_launch().sum())
+    t_fields = fields()
+    # mesh by mesh, for comparison; it leaves its own fields on the octrees
+    for it in items:
+        it["g"].lscg(it["b"], tol=1e-6)              # solver graphs
+    seq_fit = 0.0
+    for it in items:
+        lam, st = it["g"].lscg(it["b"], tol=1e-6)
+        seq_fit += st["seconds"]
+    batch.fit(tol=1e-6)
+    t_rebuild = fields()
+    log(f"[batch] fit: together {t_fit * 1e3:.1f} ms ({one_launch} meshes in one launch; first call "
+        f"{t_fit_first * 1e3:.1f} ms) vs mesh by mesh {seq_fit * 1e3:.1f} ms; fields {t_fields * 1e3:.1f} ms, "
+        f"rebuilt {t_rebuild * 1e3:.1f} ms")
     if table:
         autotune.apply(8, table)
 
@@ -209,9 +217,8 @@ def main(argv=None):
                 cb.add(it["g"])
             cb.fit(tol=1e-6)
             best = min(cb.fit(tol=1e-6)[1] for _ in range(3))
+            cap_sweep[cap] = {"fit_s": best, "one_launch_meshes": int(cb.one_launch().sum())}
             cb.close()
-            cap_sweep[cap] = {"fit_s": best, "one_launch_meshes": int(sum(1 for it in items
-                                                                            if it["g"].num_verts <= cap))}
             log(f"[batch] cap {cap}: fit {best * 1e3:.1f} ms ({cap_sweep[cap]['one_launch_meshes']} meshes "
                 f"in the one-launch kernel)")
         _capi.tune_set(_capi.TUNE_BATCH_MAX_VERTS, cap0)
@@ -223,20 +230,19 @@ def main(argv=None):
                     f"depth 5-8, {nq} queries per mesh",
         "meshes": a.meshes, "triangles_total": int(sum(it["T"] for it in items)), "unknowns_total": int(n_tot),
         "depth_counts": {d: int(sum(1 for it in items if it["depth"] == d)) for d in range(5, 9)},
-        "fit_one_launch_s": t_fit, "fit_mesh_by_mesh_s": seq_fit, "fit_speedup": seq_fit / t_fit,
+        "fit_one_launch_s": t_fit, "fit_first_call_s": t_fit_first, "fit_mesh_by_mesh_s": seq_fit, "fit_speedup": seq_fit / t_fit,
         "eval_one_launch_s": t_eval, "eval_mesh_by_mesh_s": t_seq_eval, "eval_speedup": t_seq_eval / t_eval,
         "eval_bit_identical": same,
         "all_converged": bool(all(s["converged"] for s in stats)),
         "max_iterations": int(max(s["iterations"] for s in stats)),
         "build_threads": nthr, "build_rhs_wall_s": t_build_wall,
-        "build_s_summed": t_build, "rhs_s_summed": t_rhs, "solver_setup_s_summed": t_setup, "fields_s": t_fields,
+        "build_s_summed": t_build, "rhs_s_summed": t_rhs, "solver_setup_s_summed": t_setup, "fields_s": t_fields, "fields_rebuild_s": t_rebuild,
         "meshes_per_s_fit_eval": a.meshes / gpu_total,
         "meshes_per_s_end_to_end": a.meshes / (t_build_wall + t_fit + t_fields + t_eval),
         "latency_ms_per_mesh_end_to_end": (t_build_wall + t_fit + t_fields + t_eval) / a.meshes * 1e3,
         "autotune_table": os.path.basename(a.table) if table else None,
         "one_launch_cap": _capi.tune_get(_capi.TUNE_BATCH_MAX_VERTS),
-        "one_launch_meshes": int(sum(1 for it in items
-                                     if it["g"].num_verts <= _capi.tune_get(_capi.TUNE_BATCH_MAX_VERTS))),
+        "one_launch_meshes": one_launch,
         "cap_sweep": cap_sweep,
     }
     print(json.dumps(res))
