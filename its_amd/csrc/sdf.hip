@@ -1158,14 +1158,13 @@ __device__ void dist_dfs(const TreeView& t, int leaf, int lane, const double p[3
 // results are theirs bit for bit.  Bound by vector instructions (about 3,800
 // per packet of 16 points, 65 % of the issue slots; a wavefront per point took
 // over 1,200 per point): 200,000 triangles and 554,122 octree vertices,
-// distances 2,736 -> 370 us and 305 us for the 2 % of points on the second
+// distances 2,736 -> 370 us and 169 us for the 2 % of points on the second
 // pass, crossings 1,692 -> 270 us, seeds 58 us and their sort 75 us.
 //
-// P points per packet: 16 on the first pass, over all points.  Packets whose
-// frontier would overflow put their points on a list, which the second pass
-// walks one point at a time (P = 1, 64 buckets a round).  There a frontier
-// that would overflow stays at its level, and all buckets below its nodes are
-// tested.
+// Packets whose frontier would overflow put their points on a list, which the
+// second pass walks one point a wavefront (k_dist_point, k_ray_point), down to
+// leaves of 64 triangles.  There a frontier that would overflow stays at its
+// level, and all leaves below its nodes are tested.
 constexpr int kPk = 16;
 constexpr int kFrontPacket = 384, kFrontPoint = 512;   // nodes per frontier of the two passes
 constexpr int kPairQueue = 128;  // (point, bucket): below 64 before a round, up to 64 a round
@@ -1291,9 +1290,8 @@ __device__ inline void queue_push(uint32_t* queue, int& n, bool take, uint32_t v
 }
 
 // The walk starts at the lowest level of at most this many nodes, all loaded
-// at once.  Packets go down to the buckets.  A single point stops at nodes
-// of 64 triangles, whose buckets are then tested 64 a round: three rounds of
-// the frontier that would each wait for a load are left out.
+// at once.  Packets go down to the buckets.  A single point (P = 1) stops at the
+// leaves, nodes of 64 triangles.
 constexpr int start_nodes(int P) { return P > 1 ? 256 : 512; }
 constexpr int stop_level(int P) { return P > 1 ? 0 : 3; }
 static_assert(start_nodes(1) <= kFrontPoint, "the start level always fits");
@@ -1320,7 +1318,7 @@ struct BoxStage {
 // points, the list of the level above with one.
 constexpr int kPkRefine = 40;
 template <int P, int FRONT, class Keep, class Need>
-__device__ inline int packet_frontier(const TreeView& t, int start, int lane, uint32_t (*fk)[FRONT], BoxStage& box,
+__device__ inline int packet_frontier(const TreeView& t, int start, int lane, uint32_t (*fk)[FRONT], BoxStage* box,
                                       int& cur, int& level, Keep&& keep, Need&& need) {
     constexpr int SUB = 64 / P, kQ = start_nodes(P) / 64, stop = stop_level(P);
     const uint64_t below = (1ull << lane) - 1ull;
@@ -1350,12 +1348,12 @@ __device__ inline int packet_frontier(const TreeView& t, int start, int lane, ui
             int m = 0;
             for (int j0 = 0; j0 < n; j0 += 64) {
                 const uint32_t k = j0 + lane < n ? fk[cur][j0 + lane] : 0u;
-                box.fill(t, t.s.off[h] + (int)k, lane);
+                box->fill(t, t.s.off[h] + (int)k, lane);
                 uint64_t used = 0;   // nodes of this round that some point needs
                 const int rounds = (min(64, n - j0) + SUB - 1) / SUB;
                 for (int r = 0; r < rounds; ++r) {
                     const int b = r * SUB + slot;
-                    const uint64_t votes = __ballot(need(box.lo[b], box.hi[b]));
+                    const uint64_t votes = __ballot(need(box->lo[b], box->hi[b]));
 #pragma unroll
                     for (int q = 0; q < SUB; ++q)
                         if ((votes >> (q * P)) & ((1ull << P) - 1ull)) used |= 1ull << (r * SUB + q);
@@ -1397,6 +1395,138 @@ __device__ inline int packet_frontier(const TreeView& t, int start, int lane, ui
     return n;
 }
 
+// The frontier of a single point
+template <class Keep>
+__device__ inline int point_frontier(const TreeView& t, int start, int lane, uint32_t (*fk)[kFrontPoint], int& cur,
+                                     int& level, Keep&& keep) {
+    return packet_frontier<1, kFrontPoint>(t, start, lane, fk, nullptr, cur, level, keep, keep);
+}
+
+// The second pass: one point a wavefront.  Its frontier's nodes, of `level`, each
+// stand for the 2^(level - leaf) leaves below.  64 leaves are tested a round,
+// one per lane: box(lo, hi) gives a number, and keep(number) tells whether the
+// leaf is needed, now and after the exact tests before it.  The triangles of
+// the leaves that are, one per lane and kLeaves leaves at a time, go through tri
+// to a queue, and exact takes them 64 at a time.
+//
+// Leaves, and not the packets' pairs of point and bucket: with one point those
+// read 8 spheres per lane from 64 places of memory at once, and a bucket's box
+// saves little where most triangles below a leaf are needed.  Bound by vector
+// instructions, mostly the exact tests', and by latency for few points.
+// 300,000 points in the middle of a torus of 20,000 triangles, as far from all
+// of it: 14.6 ms in pairs, 8.0 so (the whole call); 300,000 around a mesh of two
+// parts far apart: 16.9 and 8.4; the second pass of the 554,122 vertices of the
+// 200,000-triangle knot: 306 and 169 us.  Two leaves at a time were 1 % slower
+// over 245 sets of points, and so was the exact distance of the seed's leaf
+// before the frontier.
+constexpr int kLeaves = 4;
+constexpr int kLeafQueue = 64 + 64 * kLeaves;   // below 64 before a round
+template <class Box, class Keep, class Tri, class Exact>
+__device__ inline void point_leaves(const TreeView& t, const uint32_t* list, int n, int level, int leaf, int lane,
+                                    uint32_t* queue, Box&& box, Keep&& keep, Tri&& tri, Exact&& exact) {
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int shift = level - leaf, nl = n << shift;
+    int qn = 0;
+    auto flush = [&](int cnt) {   // the last cnt queued triangles
+        lds_fence();
+        qn -= cnt;
+        const uint32_t k = queue[qn + (lane < cnt ? lane : 0)];
+        lds_fence();
+        exact((int64_t)k, lane < cnt);
+    };
+    for (int j0 = 0; j0 < nl; j0 += 64) {
+        const int j = j0 + lane;
+        int l = 0;
+        bool have = false;
+        float far = 0.f;
+        if (j < nl) {
+            l = (int)((list[j >> shift] << shift) | (uint32_t)(j & ((1 << shift) - 1)));
+            have = l < t.s.count[leaf];
+            if (have) {
+                const NodeRec r = load_node(t, t.s.off[leaf] + l);
+                far = box(r.lo, r.hi);
+            }
+        }
+        uint64_t left = __ballot(have && keep(far));
+        while (left != 0ull) {
+            int k[kLeaves];
+            bool pass[kLeaves];
+            float4 S[kLeaves];
+#pragma unroll
+            for (int q = 0; q < kLeaves; ++q) {
+                const int b = left != 0ull ? __ffsll((unsigned long long)left) - 1 : 0;
+                const int64_t lk = __builtin_amdgcn_readlane(l, b);
+                k[q] = (int)node_first(leaf, lk) + lane;
+                pass[q] = left != 0ull && k[q] < node_last(t.s, leaf, lk);
+                S[q] = t.sph[pass[q] ? k[q] : 0];
+                left &= left - 1ull;
+            }
+#pragma unroll
+            for (int q = 0; q < kLeaves; ++q)
+                queue_push(queue, qn, pass[q] && tri(k[q], S[q]), (uint32_t)k[q], below);
+            if (qn < 64) continue;
+            while (qn >= 64) flush(64);
+            left &= __ballot(keep(far));
+        }
+    }
+    if (qn > 0) flush(qn);
+}
+
+// out holds the seeds' squared distances on entry
+__global__ __launch_bounds__(64, 5) void k_dist_point(TreeView t, const double* pts, Work work, const int32_t* seed_at,
+                                                     double* out, int32_t* tri_out) {
+    __shared__ uint32_t fk[2][kFrontPoint];
+    __shared__ uint32_t queue[kLeafQueue];
+    const int lane = threadIdx.x;
+    const int64_t N = work.size();
+    const NodeRec root = load_node(t, t.s.off[t.s.H]);
+    const float rs = root_scale(root);
+    const int leaf = std::min(kLeafLevel, (int)t.s.H);
+    const int start = start_level(t.s, leaf, start_nodes(1));
+    for (int64_t g = blockIdx.x; g < N; g += gridDim.x) {
+        const int64_t i = work.point(N - 1 - g);
+        const double p[3] = {wave_uniform(pts[3 * i]), wave_uniform(pts[3 * i + 1]), wave_uniform(pts[3 * i + 2])};
+        const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
+        const float pm = fmaxf(fabsf(pf[0]), fmaxf(fabsf(pf[1]), fabsf(pf[2])));
+        const float M = bound_margin(pm + 4.f * rs);   // covers any centre and radius of the tree
+        const int seed = wave_uniform(seed_at[i]);
+        double best = wave_uniform(out[i]);
+        int32_t bt = best < INFINITY ? t.tid[seed] : 0x7fffffff;
+        if (isfinite(pf[0]) && isfinite(pf[1]) && isfinite(pf[2])) {
+            auto upper = [M](double d2) { return wave_uniform_f(sqrtf((float)d2) * 1.000001f + M); };
+            float ubm = upper(best);   // upper bound of the distance, with the margin
+            // points much farther than a triangle's size also test the planes
+            const float near = 4.f * t.sph[seed].w;
+            auto box = [&](float4 lo, float4 hi) {
+                const float ex = fmaxf(fmaxf(lo.x - pf[0], pf[0] - hi.x), 0.f);
+                const float ey = fmaxf(fmaxf(lo.y - pf[1], pf[1] - hi.y), 0.f);
+                const float ez = fmaxf(fmaxf(lo.z - pf[2], pf[2] - hi.z), 0.f);
+                return ex * ex + ey * ey + ez * ez;
+            };
+            auto keep = [&](float d2) { return !(d2 > ubm * ubm); };
+            int cur = 0, level = 0;
+            const int n = point_frontier(t, start, lane, fk, cur, level,
+                                         [&](float4 lo, float4 hi) { return keep(box(lo, hi)); });
+            point_leaves(t, fk[cur], n, level, leaf, lane, queue, box, keep, [&](int k, float4 S) {
+                const float dx = pf[0] - S.x, dy = pf[1] - S.y, dz = pf[2] - S.z, lim = ubm + S.w;
+                if (dx * dx + dy * dy + dz * dz > lim * lim) return false;
+                if (!(ubm > near)) return true;
+                const float4 nr = t.nrm[k];
+                return !(fabsf(nr.x * dx + nr.y * dy + nr.z * dz) > ubm);
+            }, [&](int64_t k, bool take) {
+                tri_nearest(t, k, take, p, best, bt);
+                ubm = fminf(ubm, upper(best));
+            });
+        } else {   // a coordinate beyond binary32, or NaN
+            dist_dfs(t, leaf, lane, p, pf, pm, best, bt);
+        }
+        if (lane == 0) {
+            out[i] = sqrt(best);
+            if (tri_out) tri_out[i] = bt;
+        }
+    }
+}
+
 // points of a packet that goes to the second pass
 __device__ inline void packet_pass_on(bool valid, int64_t i, int lane, uint32_t* rest, unsigned* rest_n) {
     const uint64_t m = __ballot(valid);
@@ -1406,18 +1536,20 @@ __device__ inline void packet_pass_on(bool valid, int64_t i, int lane, uint32_t*
     if (valid) rest[base + __popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)i;
 }
 
-// Point sets below this take the second pass alone: 2,000 packets or fewer
-// leave most of the chip's 1,024 SIMDs with one wavefront or none, and 16
-// times as many wavefronts hide more (20,000 uniform points around a
-// 10,000-triangle torus: 0.61 ms in packets, 0.47 one by one; 100,000: 0.74
-// in packets).
-constexpr int64_t kPacketPoints = 32768;
+// Point sets below this take the second pass alone: 3,000 packets or fewer
+// leave most of the chip's 1,024 SIMDs with few wavefronts or none, 16 times as
+// many wavefronts hide more, and the points' sort takes 9 launches.  In packets
+// and one by one, whole call in ms: 24,000 points in the box of a
+// 10,000-triangle torus 0.50 and 0.37, 48,000 0.56 and 0.50, 64,000 0.59 and
+// 0.57, 100,000 0.68 and 0.74; near its surface 48,000 0.48 and 0.44, 64,000
+// 0.49 and 0.50; 200,000-triangle knot, near the surface, 48,000 1.02 and 1.01,
+// 64,000 1.02 and 1.11.
+constexpr int64_t kPacketPoints = 49152;
 
 // out holds the seeds' squared distances on entry
-template <int P, int FRONT>
 __global__ __launch_bounds__(64, 5) void k_dist_packet(TreeView t, const double* pts, Work work, const int32_t* seed_at,
                                                     double* out, int32_t* tri_out, uint32_t* rest, unsigned* rest_n) {
-    constexpr int SUB = 64 / P;   // buckets tested at once
+    constexpr int P = kPk, FRONT = kFrontPacket, SUB = 64 / P;   // buckets tested at once
     __shared__ uint32_t fk[2][FRONT];
     __shared__ BoxStage box;
     __shared__ uint32_t pairs[kPairQueue];   // frontier slot * P + point
@@ -1487,24 +1619,14 @@ __global__ __launch_bounds__(64, 5) void k_dist_packet(TreeView t, const double*
     };
     int cur = 0;
     int level = 0;
-    const int n = wild ? -1 : packet_frontier<P, FRONT>(t, start, lane, fk, box, cur, level, [&](float4 lo, float4 hi) {
+    const int n = wild ? -1 : packet_frontier<P, FRONT>(t, start, lane, fk, &box, cur, level, [&](float4 lo, float4 hi) {
         const float ex = fmaxf(fmaxf(lo.x - bhi[0], blo[0] - hi.x), 0.f);
         const float ey = fmaxf(fmaxf(lo.y - bhi[1], blo[1] - hi.y), 0.f);
         const float ez = fmaxf(fmaxf(lo.z - bhi[2], blo[2] - hi.z), 0.f);
         return !(ex * ex + ey * ey + ez * ez > reach2);
     }, needs);
     if (n < 0) {
-        if (P > 1) {
-            packet_pass_on(valid && slot == 0, i, lane, rest, rest_n);
-        } else {   // the node-by-node walk of the one point
-            double best = seed_d2;
-            int32_t bt = sid[0];
-            dist_dfs(t, std::min(kLeafLevel, (int)t.s.H), lane, p, pf, pm, best, bt);
-            if (lane == 0) {
-                out[i] = sqrt(best);
-                if (tri_out) tri_out[i] = bt;
-            }
-        }
+        packet_pass_on(valid && slot == 0, i, lane, rest, rest_n);
         continue;
     }
     // points much farther than a triangle's size also test the planes
@@ -1567,22 +1689,13 @@ __global__ __launch_bounds__(64, 5) void k_dist_packet(TreeView t, const double*
             }
             const unsigned long long bits = (unsigned long long)__double_as_longlong(d2), pre = sbest[o];
             lds_fence();
-            if (P == 1) {   // one point: a butterfly instead of 64 atomics on one word
-                wave_argmin(d2, id);
-                if (lane == 0) {
-                    const unsigned long long now = (unsigned long long)__double_as_longlong(d2);
-                    if (now < pre || (now == pre && id < sid[0])) sid[0] = id;
-                    sbest[0] = now < pre ? now : pre;
-                }
-            } else {
-                if (take) atomicMin(&sbest[o], bits);
-                lds_fence();
-                const unsigned long long now = sbest[o];
-                const bool win = take && bits == now;
-                if (win && now < pre) sid[o] = 0x7fffffff;   // a smaller distance: the old index does not count
-                lds_fence();
-                if (win) atomicMin(&sid[o], id);
-            }
+            if (take) atomicMin(&sbest[o], bits);
+            lds_fence();
+            const unsigned long long now = sbest[o];
+            const bool win = take && bits == now;
+            if (win && now < pre) sid[o] = 0x7fffffff;   // a smaller distance: the old index does not count
+            lds_fence();
+            if (win) atomicMin(&sid[o], id);
             lds_fence();
             ubm = fminf(ubm, upper(__longlong_as_double((long long)sbest[pt])));
             sub[pt] = ubm;   // the same value from every lane of the point
@@ -1766,11 +1879,10 @@ __device__ inline int tri_ray(const double* T, const double p[3], const Ray& R, 
 // and the lists fitted; otherwise decided[i] = 0 and the fan walk takes the
 // point.  With cross given (an open mesh) the crossings and the ray's axis and
 // direction are left there instead, and k_rim applies the sign.
-template <int P, int FRONT>
 __global__ __launch_bounds__(64, 5) void k_ray_packet(TreeView t, const double* pts, Work work, double* out,
                                                    uint8_t* decided, int* cross, unsigned* undecided, uint32_t* rest,
                                                    unsigned* rest_n) {
-    constexpr int SUB = 64 / P;   // buckets tested at once
+    constexpr int P = kPk, FRONT = kFrontPacket, SUB = 64 / P;   // buckets tested at once
     __shared__ uint32_t fk[2][FRONT];
     __shared__ BoxStage box;
     __shared__ uint32_t pairs[kPairQueue];   // frontier slot * P + point
@@ -1826,17 +1938,12 @@ __global__ __launch_bounds__(64, 5) void k_ray_packet(TreeView t, const double* 
     };
     int cur = 0;
     int level = 0;
-    const int n = wild ? -1 : packet_frontier<P, FRONT>(t, start, lane, fk, box, cur, level, [&](float4 lo, float4 hi) {
+    const int n = wild ? -1 : packet_frontier<P, FRONT>(t, start, lane, fk, &box, cur, level, [&](float4 lo, float4 hi) {
         return !(sel3(hi, R.u) < ulo || sel3(lo, R.u) > uhi || sel3(hi, R.v) < vlo || sel3(lo, R.v) > vhi ||
                  box_far(lo, hi) < wlo);
     }, needs);
     if (n < 0) {
-        if (P > 1) {
-            packet_pass_on(valid && slot == 0, i, lane, rest, rest_n);
-        } else if (lane == 0) {
-            decided[i] = 0;
-            atomicAdd(undecided, 1u);
-        }
+        packet_pass_on(valid && slot == 0, i, lane, rest, rest_n);
         continue;
     }
     int qp = 0, qt = 0;
@@ -1903,6 +2010,63 @@ __global__ __launch_bounds__(64, 5) void k_ray_packet(TreeView t, const double* 
         if (cross) cross[i] = scross[pt] * 8 + R.w * 2 + (fwd ? 1 : 0);
         else if (!unsure && scross[pt] >= 1) out[i] = -out[i];   // winding number > 1/2
     }
+    }
+}
+
+// The same for one point a wavefront
+__global__ __launch_bounds__(64, 5) void k_ray_point(TreeView t, const double* pts, Work work, double* out,
+                                                    uint8_t* decided, int* cross, unsigned* undecided) {
+    __shared__ uint32_t fk[2][kFrontPoint];
+    __shared__ uint32_t queue[kLeafQueue];
+    const int lane = threadIdx.x;
+    const int64_t N = work.size();
+    const NodeRec root = load_node(t, t.s.off[t.s.H]);
+    const float rs = root_scale(root);
+    const int leaf = std::min(kLeafLevel, (int)t.s.H);
+    const int start = start_level(t.s, leaf, start_nodes(1));
+    for (int64_t g = blockIdx.x; g < N; g += gridDim.x) {
+        const int64_t i = work.point(N - 1 - g);
+        const double p[3] = {wave_uniform(pts[3 * i]), wave_uniform(pts[3 * i + 1]), wave_uniform(pts[3 * i + 2])};
+        const float pf[3] = {(float)p[0], (float)p[1], (float)p[2]};
+        Ray R = choose_ray(p, root.lo, root.hi);
+        bool unsure = !(isfinite(pf[0]) && isfinite(pf[1]) && isfinite(pf[2]));
+        int c = 0;
+        if (!unsure) {
+            R.w = wave_uniform(R.w);
+            R.sg = wave_uniform(R.sg);
+            R.u = R.w == 2 ? 0 : R.w + 1;
+            R.v = R.u == 2 ? 0 : R.u + 1;
+            const float dir = R.sg > 0 ? 1.f : -1.f;
+            const float pm = fmaxf(fabsf(pf[0]), fmaxf(fabsf(pf[1]), fabsf(pf[2])));
+            const float M = bound_margin(pm + 4.f * rs);
+            const float4 pf4 = make_float4(pf[0], pf[1], pf[2], 0.f);
+            const float pu = sel3(pf4, R.u), pv = sel3(pf4, R.v), pw = sel3(pf4, R.w) * dir;   // pw: place along the ray
+            // does the ray meet the box?
+            auto meets = [&](float4 lo, float4 hi) {
+                const float last = R.sg > 0 ? sel3(hi, R.w) : -sel3(lo, R.w);
+                return !(sel3(hi, R.u) < pu - M || sel3(lo, R.u) > pu + M || sel3(hi, R.v) < pv - M ||
+                         sel3(lo, R.v) > pv + M || last < pw - M);
+            };
+            int cur = 0, level = 0;
+            const int n = point_frontier(t, start, lane, fk, cur, level, meets);
+            point_leaves(t, fk[cur], n, level, leaf, lane, queue,
+                         [&](float4 lo, float4 hi) { return meets(lo, hi) ? 0.f : 1.f; },
+                         [](float miss) { return miss == 0.f; }, [&](int, float4 S) {
+                // wholly beside the ray or behind its start: no crossing
+                const float du = pu - sel3(S, R.u), dv = pv - sel3(S, R.v), lim = S.w + M;
+                return !(du * du + dv * dv > lim * lim) && !(pw - sel3(S, R.w) * dir > lim);
+            }, [&](int64_t k, bool take) {
+                if (take) c += tri_ray(t.tris + 9 * k, p, R, unsure);
+            });
+        }
+        unsure = __ballot(unsure) != 0ull;
+        c = wave_sum(c);
+        if (lane == 0) {
+            decided[i] = unsure ? 0 : 1;
+            if (unsure) atomicAdd(undecided, 1u);
+            if (cross) cross[i] = c * 8 + R.w * 2 + (R.sg > 0 ? 1 : 0);
+            else if (!unsure && c >= 1) out[i] = -out[i];   // winding number > 1/2
+        }
     }
 }
 
@@ -2089,8 +2253,6 @@ void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* 
         }
         return (unsigned)std::min<int64_t>(most, (int64_t)per_cu * cus);
     };
-    constexpr auto dist1 = k_dist_packet<kPk, kFrontPacket>, dist2 = k_dist_packet<1, kFrontPoint>;
-    constexpr auto ray1 = k_ray_packet<kPk, kFrontPacket>, ray2 = k_ray_packet<1, kFrontPoint>;
     // every point's seed; with packets, also their order
     const bool packets = N >= kPacketPoints && N < (int64_t(1) << 32);
     DBuf<uint32_t> key(N), order(N), rest;
@@ -2106,12 +2268,12 @@ void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* 
         rest.alloc(N);
         all.list = order.p;
         left = Work{N, rest.p, counts};
-        hipLaunchKernelGGL(dist1, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, (const int32_t*)seed_at.p, d_out,
+        hipLaunchKernelGGL(k_dist_packet, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, (const int32_t*)seed_at.p, d_out,
                            d_tri, rest.p, counts);
         ITS_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(dist2, dim3(grid_of((const void*)dist2, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left,
-                       (const int32_t*)seed_at.p, d_out, d_tri, (uint32_t*)nullptr, (unsigned*)nullptr);
+    hipLaunchKernelGGL(k_dist_point, dim3(grid_of((const void*)k_dist_point, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left,
+                       (const int32_t*)seed_at.p, d_out, d_tri);
     ITS_LAUNCH_CHECK();
     // Signs by the ray, and the rim where there is a boundary, for the points
     // that they decide; the fans are built and walked only for the others.
@@ -2134,16 +2296,16 @@ void signed_distance(its_ctx ctx, const double* d_V, int64_t nV, const int32_t* 
         if (open) cross.alloc(N);
         if (packets) {
             left.list_n = counts + 1;
-            hipLaunchKernelGGL(ray1, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, d_out, decided.p,
+            hipLaunchKernelGGL(k_ray_packet, dim3(pgrid), dim3(64), 0, st, tr.view(), d_pts, all, d_out, decided.p,
                                cross.p, counts + 2, rest.p, counts + 1);
             ITS_LAUNCH_CHECK();
         }
-        hipLaunchKernelGGL(ray2, dim3(grid_of((const void*)ray2, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left, d_out,
-                           decided.p, cross.p, counts + 2, (uint32_t*)nullptr, (unsigned*)nullptr);
+        hipLaunchKernelGGL(k_ray_point, dim3(grid_of((const void*)k_ray_point, 64, N)), dim3(64), 0, st, tr.view(), d_pts, left,
+                           d_out, decided.p, cross.p, counts + 2);
         ITS_LAUNCH_CHECK();
         if (open) {
-            hipLaunchKernelGGL(k_rim, dim3(grid_of((const void*)k_rim, 64 * kRimWaves, (N + 63) / 64)),
-                               dim3(64 * kRimWaves), 0, st, (const RimEdge*)tr.rim.p,
+            hipLaunchKernelGGL(k_rim, dim3(strided_blocks(N, 64, 64 * kRimWaves)), dim3(64 * kRimWaves), 0, st,
+                               (const RimEdge*)tr.rim.p,
                                rim, d_pts, N, d_out, decided.p, (const int*)cross.p, counts + 2);
             ITS_LAUNCH_CHECK();
         }

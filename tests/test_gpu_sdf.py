@@ -186,10 +186,10 @@ def test_sdf_ray_signs(ctx, name):
         assert (d_ray < 0).sum() > 1000
 
 
-@pytest.mark.parametrize("N", [32767, 32768, 32769, 50021])
+@pytest.mark.parametrize("N", [32768, 49151, 49152, 49153, 65021])
 @pytest.mark.parametrize("name", ["icosphere", "open", "single", "nine", "collapsed"])
 def test_sdf_packets(ctx, name, N):
-    """Point sets walked in packets of 16 (from 32,768 points) against the
+    """Point sets walked in packets of 16 (from 49,152 points) against the
     same points in calls small enough to be walked one by one: identical bit
     for bit, since both take the exact minimum and exact crossings; and a
     sample of them against the brute-force oracle.  Dense points on the
@@ -231,6 +231,28 @@ def test_sdf_packets(ctx, name, N):
     assert np.abs(np.abs(d[k]) - np.abs(O.signed_distance(V, F, P[k]))).max() <= 1e-12
 
 
+@pytest.mark.parametrize("T", [1, 7, 8, 9, 63, 64, 65, 511, 513, 4097, 81920])
+def test_sdf_one_by_one(ctx, T):
+    """The walk of one point a wavefront against the brute-force oracle: meshes
+    that end inside a bucket or a leaf of 64, below and above 512 leaves.  At the
+    sphere's centre every leaf is needed, so that with 1,280 of them the frontier
+    stays above the leaves; far away rays and distances start outside."""
+    V, F = meshes.icosphere(6) if T > 20000 else meshes.noisy_icosphere(seed=3, level=4)
+    F = np.ascontiguousarray(F[:T], np.int32)
+    assert len(F) == T
+    rng = np.random.default_rng(T)
+    P = np.concatenate([np.zeros((1, 3)), 1e-3 * rng.standard_normal((20, 3)), 5 * rng.standard_normal((20, 3)),
+                        V[F[rng.integers(0, T, 60), 0]] + 0.02 * rng.standard_normal((60, 3)), [[40.0, 0, 0]]])
+    print(f"[sdf one by one] T={T}", flush=True)
+    d = ctx.signed_distance(V, F, P)
+    ref = O.signed_distance(V, F, P)
+    assert np.abs(np.abs(d) - np.abs(ref)).max() <= 1e-12
+    w = np.array([O.winding_number(V, F, p) for p in P])
+    clear = (np.abs(ref) > 1e-6) & (np.abs(w - 0.5) > 1e-3)
+    assert clear.sum() > 90
+    np.testing.assert_array_equal(np.signbit(d[clear]), np.signbit(ref[clear]))
+
+
 def _collapsed_mesh(order):
     """Closed sphere and one face on the chord between two far vertices i and
     j, of no area: a repeated corner (the distance to it is 0 / 0 for half of
@@ -242,7 +264,7 @@ def _collapsed_mesh(order):
     return np.ascontiguousarray(V), np.concatenate([F, [face]]).astype(np.int32), i, j
 
 
-@pytest.mark.parametrize("N", [2000, 40001])
+@pytest.mark.parametrize("N", [2000, 50021])
 @pytest.mark.parametrize("order", ["iij", "ijj", "iji", "line"])
 def test_sdf_collapsed_face(ctx, order, N):
     """Points around a face of no area far from all others, one by one and in
@@ -298,7 +320,7 @@ def _rim_mesh(kind):
     return V, np.ascontiguousarray(F, np.int32)
 
 
-@pytest.mark.parametrize("N", [1, 63, 2000, 40001])
+@pytest.mark.parametrize("N", [1, 63, 2000, 50021])
 @pytest.mark.parametrize("kind", ["patch", "holes", "flipped", "doubled", "limit", "over", "long", "too_long"])
 def test_sdf_rim_signs(ctx, kind, N):
     """Meshes with a boundary: distances are the brute-force oracle's (on a
