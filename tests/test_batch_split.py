@@ -44,8 +44,18 @@ def test_split_of_too_many_large_meshes(split):
 
 
 def test_split_moves_what_holds_the_launch_up(split):
-    """6 meshes of 7,165 to 55,852 unknowns: the largest would take 11 ms on its
-    workgroup, the many-mesh solver's launches 2.7; small meshes stay."""
-    assert split([(7165, 6), (14110, 7), (20000, 7), (31101, 7), (40000, 7), (55852, 7)]) <= 1
+    """6 meshes of 7,165 to 55,852 unknowns: the largest would take 6 ms on its
+    workgroup, the many-mesh solver's launches about 2; the small ones stay."""
+    assert split([(7165, 6), (14110, 7), (20000, 7), (31101, 7), (40000, 7), (55852, 7)]) == 2
     assert split([(160, 3), (3668, 5)]) == 2
-    assert split([(14110, 7)] * 256) == 256
+    assert split([(56062, 7)] * 2) == 0 and split([(14176, 6)] * 4) == 0
+    assert split([(56062, 7)] * 128) == 0   # beside each other both slow down
+
+
+@pytest.mark.parametrize("mesh", [(160, 3), (854, 4), (3694, 5), (14110, 7)])
+@pytest.mark.parametrize("count", [256, 600, 1000, 2000])
+def test_split_leaves_a_full_chip_alone(split, mesh, count):
+    """Where the one launch has a workgroup for every CU, nothing runs beside it:
+    many meshes of one small size stay together (moving 88 of 600 meshes of 854
+    unknowns doubled the fit's time)."""
+    assert split([mesh] * count) == count
