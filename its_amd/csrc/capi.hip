@@ -740,13 +740,32 @@ struct ShellInput {
     DBuf<double> V, tris;
     DBuf<uint64_t> edges;
     int64_t ne = 0;
+    // host sides of the copies, until the call ends
+    std::vector<uint64_t> h_edges;
+    std::vector<double> h_tris;
 };
+// Up to so many faces the edges are sorted on the host: the device's sort and
+// compaction are some 12 launches (iso values at 64^3, host and device: 80 faces
+// 0.24 and 0.29 ms, 1,280 0.26 and 0.30, 2,400 0.31 and 0.32, 5,120 0.67 and 0.33).
+constexpr int64_t kShellHostFaces = 2048;
+// Up to so many values the range is taken on the host, from one copy.
+constexpr int64_t kRangeHostValues = 4096;
 ShellInput shell_upload(const double* V, int64_t nV, const int32_t* F, int64_t nF, hipStream_t st) {
     ITS_REQUIRE(V && F && nV > 0 && nF > 0, ITS_E_INVALID, "empty mesh");
     for (int64_t i = 0; i < 3 * nF; ++i)
         ITS_REQUIRE(F[i] >= 0 && F[i] < nV, ITS_E_INVALID, "face index out of range");
     ShellInput in;
     in.V = upload(V, 3 * (size_t)nV, st);
+    if (nF <= kShellHostFaces) {
+        in.h_edges = mesh_edges_host(F, nF);
+        in.h_tris.resize(9 * (size_t)nF);
+        for (int64_t c = 0; c < 3 * nF; ++c)
+            for (int a = 0; a < 3; ++a) in.h_tris[3 * c + a] = V[3 * (int64_t)F[c] + a];
+        in.tris = upload(in.h_tris.data(), in.h_tris.size(), st);
+        in.edges = upload(in.h_edges.data(), in.h_edges.size(), st);
+        in.ne = (int64_t)in.h_edges.size();
+        return in;
+    }
     DBuf<int32_t> d_F = upload(F, 3 * (size_t)nF, st);
     in.tris.alloc(9 * (size_t)nF);
     face_corners(in.V.p, d_F.p, nF, in.tris.p, st);
@@ -797,7 +816,8 @@ int its_shell_iso(its_ctx ctx, its_svo s, const double* V, int64_t nV, const int
     eval_points_aos64(s, in.V.p, nV, dummy, ITS_EVAL_RAW, 0.f, f.p, st);
     if (np > 0) eval_points_aos64(s, P.p, np, dummy, ITS_EVAL_RAW, 0.f, f.p + nV, st);
     float range[2];
-    if (!value_range(f.p, nall, range, st)) {   // a NaN: whatever comparing in order leaves
+    // by comparing in order where there are few, or a NaN
+    if (nall <= kRangeHostValues || !value_range(f.p, nall, range, st)) {
         std::vector<float> h(nall);
         ITS_HIP(hipMemcpyAsync(h.data(), f.p, nall * sizeof(float), hipMemcpyDeviceToHost, st));
         ITS_HIP(hipStreamSynchronize(st));

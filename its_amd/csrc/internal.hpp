@@ -183,6 +183,7 @@ int64_t fine_edges(its_svo s, DBuf<double>& ends, DBuf<uint32_t>& owner, hipStre
 void shell_points(its_svo s, const double* d_V, const uint64_t* d_edges, int64_t ne, const double* d_tris, int64_t nT,
                   DBuf<double>& pts, int64_t* n_edge, int64_t* n_face, hipStream_t st);
 int64_t mesh_edges(const int32_t* d_F, int64_t nF, int64_t nV, DBuf<uint64_t>& edges, hipStream_t st);
+std::vector<uint64_t> mesh_edges_host(const int32_t* F, int64_t nF);
 void face_corners(const double* d_V, const int32_t* d_F, int64_t nF, double* d_tris, hipStream_t st);
 bool value_range(const float* d_f, int64_t n, float range[2], hipStream_t st);
 // batch.hip

@@ -507,7 +507,18 @@ __global__ __launch_bounds__(kT) void k_minmax(const float* f, int64_t n, float*
 }  // namespace
 
 // The ordered set of (smaller, larger) vertex pairs of the faces
-// (BaseModel.cpp:291-313): keys sorted by the radix sort, one of each kept.
+// (BaseModel.cpp:291-313), for few faces on the host
+std::vector<uint64_t> mesh_edges_host(const int32_t* F, int64_t nF) {
+    std::vector<uint64_t> e(3 * (size_t)nF);
+    for (int64_t k = 0; k < 3 * nF; ++k) {
+        const uint32_t a = (uint32_t)F[k], b = (uint32_t)F[k % 3 == 2 ? k - 2 : k + 1];
+        e[k] = ((uint64_t)std::min(a, b) << 32) | std::max(a, b);
+    }
+    std::sort(e.begin(), e.end());
+    e.erase(std::unique(e.begin(), e.end()), e.end());
+    return e;
+}
+// and on the device: keys sorted by the radix sort, one of each kept.
 // 600,000 pairs took 25 ms in a host sort.
 int64_t mesh_edges(const int32_t* d_F, int64_t nF, int64_t nV, DBuf<uint64_t>& edges, hipStream_t st) {
     const int64_t n = 3 * nF;

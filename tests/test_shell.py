@@ -77,6 +77,30 @@ def test_gpu_iso_values(ctx, name, R):
     g.close()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("faces", [1, 12, 2047, 2048, 2049])
+def test_gpu_points_few_faces(ctx, faces):
+    """Meshes whose edges are sorted on the host (up to 2,048 faces) and on the
+    device, with a face of two equal corners: the oracle's points."""
+    from its_amd import _capi, meshes
+    V, F = meshes.torus(40, 30)
+    F = np.ascontiguousarray(F[:faces], np.int32)
+    F[-1, 1] = F[-1, 0]
+    if faces == 1:
+        F = np.array([[0, 1, 31]], np.int32)
+    o, _, w = _capi.uniform_bbox(V)
+    tris = meshes.triangles(V, F)
+    print(f"[shell] {faces} faces", flush=True)
+    g = _capi.Octree(ctx, tris, o, w, 32)
+    P, ne = g.shell_points(V, F)
+    Q, qe = O.intersections(O.SVO(tris, o, w, 32), V, F)
+    assert np.array_equal(np.unique(P[:ne], axis=0), np.unique(Q[:qe], axis=0))
+    assert len(P) - ne == len(Q) - qe
+    d = np.abs(_sorted(P[ne:]) - _sorted(Q[qe:]))
+    assert d.max() <= 1e-12 if len(d) else True
+    g.close()
+
+
 def test_oracle_classify_rule():
     """The class rule on its boundaries: a value equal to the outer iso value
     is 1, equal to the inner one -1, NaN 0 (ThinShells.cpp:1412-1417)."""
